@@ -372,6 +372,15 @@ typedef struct nkv_decode_args {
 int nkv_decode(void* stream, const nkv_decode_args* args);
 
 /*
+ * n decodes of one operator (the segments of a cache, read one by one by
+ * decode_value, MG:516-539): every call has its own codec rows, centers, row
+ * list and output; all share HD, r, group, scale_dtype, w_dec and mean
+ * (NKV_ERR_INVALID otherwise).  Each result is that of nkv_decode on it; up to
+ * 16 batch items run in one launch.
+ */
+int nkv_decode_batch(void* stream, const nkv_decode_args* args, int n);
+
+/*
  * Decode-and-attend in one call: softmax(q k^T * softmax_scale) v over the
  * keys [decoded history (N tokens); current chunk (Nc tokens)], non-causal.
  * History K/V rows are decoded tile by tile with the nkv_decode arithmetic:

@@ -35,6 +35,7 @@ EXPORTED = (
     "nkv_fast_attend_workspace_size", "nkv_fast_attend", "nkv_rope_apply", "nkv_int8_pack",
     "nkv_int8_dequant", "nkv_c64_fit_workspace_size", "nkv_c64_fit", "nkv_camera_apply",
     "nkv_attend_static", "nkv_lift_lse_combine", "nkv_finish", "nkv_reader_rows",
+    "nkv_decode_batch",
 )
 NKV_STATIC_SCRATCH_BYTES = 64 << 20
 
@@ -210,6 +211,8 @@ def _declare(lib: ctypes.CDLL) -> None:
     lib.nkv_encode_batch.argtypes = [c_void_p, POINTER(NkvEncodeArgs), c_int]
     lib.nkv_decode.restype = c_int
     lib.nkv_decode.argtypes = [c_void_p, POINTER(NkvDecodeArgs)]
+    lib.nkv_decode_batch.restype = c_int
+    lib.nkv_decode_batch.argtypes = [c_void_p, POINTER(NkvDecodeArgs), c_int]
     lib.nkv_attend_workspace_size.restype = c_size_t
     lib.nkv_attend_workspace_size.argtypes = [POINTER(NkvAttendArgs)]
     lib.nkv_attend.restype = c_int

@@ -1191,6 +1191,254 @@ __global__ void __launch_bounds__(256) decode_gemm_kernel(DecodeA al, DecodeEpi 
     }
 }
 
+
+// ============================================================ staged decode
+// out[m, n] = bf16(bf16(latent[m] . w_dec[n] + bf16(mean[n])) + center[id[m], n])
+// (MG:438-454) for up to DEC_MAXB problems of one shape in one launch: the
+// segments of a cache, batch items.  A block owns 32 MI WR rows x 64 WC
+// columns (wave (wr, wc): 32 MI rows x 64 columns) and walks r in 64-wide
+// slices:
+//   - W_dec slice [columns][64] by 1 KB DMA pieces, double-buffered, issued
+//     one slice ahead;
+//   - the codes of the slice, held in registers one slice ahead (16 per
+//     thread), unpacked once per block into the latent image [rows][64].
+// Both images are [row][8 chunks of 16 bytes] with chunk c of row q at slot
+// c ^ ((q >> 1) & 7): the 16 rows that one LDS cycle serves fall in 16
+// distinct slots.  W is the MFMA's row operand, so a lane ends with four
+// consecutive columns of one row; bf16(acc + mean) goes through LDS and out
+// as whole 16-byte pieces of rows, the center row's piece added on the way.
+// The accumulator takes k in ascending steps of 16, as decode_gemm_kernel
+// does: the same bits.
+// Measured (12,480 x 3,072, r = 384, centers): 52.7 us = 559 TFLOP/s, 1.5 TB/s
+// written, against 214 us for decode_gemm_kernel (one 64 x 64 tile per block,
+// codes unpacked per 64 columns, 2-byte stores) and 43 us more to concatenate
+// the segments.  Not bound by one unit: with the W copies, the unpack or the
+// MFMAs left out it takes 47, 43 and 39 us; the rest (output, centers) 17.
+constexpr int DEC_MAXB = 16, DT_K = 64;
+struct DecProb {
+    const uint8_t* packed;
+    const uint16_t* scales;
+    const void* ids;
+    const uint16_t* centers;   // [C, HD], or NULL
+    const int32_t* row_index;  // [M], or NULL
+    uint16_t* out;             // [M, HD]
+    int64_t M;
+    int id_bytes, num_centers;
+};
+struct DecBatch {
+    DecProb p[DEC_MAXB];
+    const uint16_t* w;         // [HD, r]
+    const float* mean;         // [HD], or NULL
+    int n, HD, r, group, scale_dtype;
+    uint32_t row_blocks;       // of the largest problem
+};
+
+// bf16((code - 7) * scale) of eight codes, as unpack_kernel forms it (the
+// one-fma form of unpack8 gives NaN where an infinite scale gives +-inf here).
+__device__ __forceinline__ u32x4 latent8(uint32_t w, float s) {
+    uint32_t ev = w & 0x0f0f0f0fu, od = (w >> 4) & 0x0f0f0f0fu;
+    asm("" : "+v"(ev));  // one v_cvt_f32_ubyte per code (see unpack8)
+    asm("" : "+v"(od));
+    u32x4 o;
+#pragma unroll
+    for (int b = 0; b < 4; ++b)
+        o[b] = pack_bf16x2(((float)((ev >> (8 * b)) & 0xffu) - 7.0f) * s,
+                           ((float)((od >> (8 * b)) & 0xffu) - 7.0f) * s);
+    return o;
+}
+
+template <int MI, int WR, int WC>
+struct DecFmt {
+    static constexpr int ROWS = 32 * MI * WR, COLS = 64 * WC, WAVES = WR * WC, THREADS = 64 * WAVES;
+    static constexpr int WSTAGE = COLS * DT_K * 2, AIMG = ROWS * DT_K * 2;
+    static constexpr int WPIECES = WSTAGE / 1024 / WAVES;      // DMA pieces per wave
+    static constexpr int OSTRIDE = COLS * 2 + 16;              // staged output row, bytes
+    static constexpr int CROW = ROWS * OSTRIDE;                // center row pointers, after the GEMM
+    static constexpr int SMEM = 2 * WSTAGE + AIMG;
+    static_assert(CROW + 8 * ROWS <= SMEM, "the output tile fits the GEMM's buffers");
+    static constexpr bool BIG = MI == 2;
+    static constexpr int UNITS = ROWS * COLS / 8 / THREADS;    // 16-byte output pieces per thread
+    static_assert(ROWS * 4 == THREADS, "a thread unpacks 16 codes of one row");
+    static_assert(WSTAGE % (1024 * WAVES) == 0, "whole pieces per wave");
+};
+
+template <int MI, int WR, int WC>
+__global__ void __launch_bounds__(64 * WR * WC, 4) decode_tile_kernel(DecBatch B) {
+    using F = DecFmt<MI, WR, WC>;
+    extern __shared__ __align__(16) unsigned char smem_raw[];
+    // items: (problem, row block, column block), column block fastest, eight
+    // equal runs, one per XCD: the blocks of one XCD share code and center rows
+    const uint32_t ncb = (uint32_t)(B.HD + F::COLS - 1) / F::COLS;
+    const uint32_t items = (uint32_t)B.n * B.row_blocks * ncb;
+    const uint32_t item = (blockIdx.x & 7) * ((items + 7) >> 3) + (blockIdx.x >> 3);
+    if (item >= items) return;
+    const uint32_t rest = item / ncb, prob = rest / B.row_blocks;
+    const DecProb& P = B.p[prob];
+    const int64_t m0 = (int64_t)(rest - prob * B.row_blocks) * F::ROWS;
+    if (m0 >= P.M) return;
+    const int n0 = (int)(item - rest * ncb) * F::COLS;
+    const int r = B.r, S = (r + DT_K - 1) / DT_K;
+    const int t = threadIdx.x, lane = t & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
+    const int hf = lane >> 5, l32 = lane & 31;
+    const int wr = wave / WC, wc = wave % WC;
+    // this thread's codes: row t / 4, k 16 (t % 4) .. +16 of each slice
+    const int arow = t >> 2, aq = t & 3;
+    int64_t src = min(m0 + arow, P.M - 1);
+    if (P.row_index) src = P.row_index[src];
+    const uint8_t* cp = P.packed + src * (r / 2) + 8 * aq;
+    const uint16_t* sp = P.scales + src * (r / B.group);
+    const uint16_t* my_crow = nullptr;
+    if (P.centers && aq == 0) {
+        const int id = min(max(read_id(P.ids, P.id_bytes, src), 0), P.num_centers - 1);
+        my_crow = P.centers + (int64_t)id * B.HD;
+    }
+    const float inv_g = 1.0f / (float)B.group;
+    // floor(k / group) for k < 2^20: (k + 0.5) / group is at least 0.5 / group
+    // from an integer, the product's error is below k 2^-22 / group
+    auto grp = [&](int k) { return (int)(((float)k + 0.5f) * inv_g); };
+    // W pieces: piece e = wave + WAVES i holds columns 8e .. 8e + 8 (pieces
+    // past HD: the last eight); lane L brings slot L % 8 of column 8e + L / 8.
+    // WAVES is even, so the slot's chunk is the same in every piece.  A half
+    // slice (r % 64 == 32) repeats its first half in the second; unused.
+    static_assert(F::WAVES % 2 == 0, "one lane offset serves every piece");
+    const int wq = 8 * wave + (lane >> 3), wch = (lane & 7) ^ ((wq >> 1) & 7);
+    const uint32_t woff = (uint32_t)(lane >> 3) * (uint32_t)(2 * r);
+    const uint32_t woff_full = woff + 16 * wch, woff_half = woff + 16 * (wch & 3);
+    auto issue_w = [&](int s) {
+        unsigned char* dst = smem_raw + (s & 1) * F::WSTAGE;
+        const uint32_t off = r - s * DT_K >= DT_K ? woff_full : woff_half;
+#pragma unroll
+        for (int i = 0; i < F::WPIECES; ++i) {
+            const int e = wave + F::WAVES * i;
+            const unsigned char* g = reinterpret_cast<const unsigned char*>(B.w) +
+                                     2 * ((int64_t)min(n0 + 8 * e, B.HD - 8) * r + s * DT_K);
+            dma16(g + off, dst + 1024 * e);
+        }
+    };
+    u32x2 code;
+    float sc[2];
+    const bool g16 = B.group % 16 == 0;
+    auto load_codes = [&](int s) {
+        const int k = s * DT_K + 16 * aq;
+        if (k < r) {
+            code = *reinterpret_cast<const u32x2*>(cp + s * (DT_K / 2));
+            sc[0] = sc[1] = scale_bits_to_f32(sp[grp(k)], B.scale_dtype);
+            if (!g16) sc[1] = scale_bits_to_f32(sp[grp(k + 8)], B.scale_dtype);
+        }
+    };
+    unsigned char* aimg = smem_raw + 2 * F::WSTAGE;
+    const int asw = (arow >> 1) & 7;
+    f32x16 acc[MI][2] = {};
+    issue_w(0);
+    load_codes(0);
+    for (int s = 0; s < S; ++s) {
+        const int kn = min(r - s * DT_K, DT_K);
+        if (16 * aq < kn) {
+#pragma unroll
+            for (int c = 0; c < 2; ++c)
+                *reinterpret_cast<u32x4*>(aimg + arow * (DT_K * 2) + 16 * ((2 * aq + c) ^ asw)) =
+                    latent8(code[c], sc[c]);
+        }
+        // slice s landed and its latent image is written (nothing later is in flight)
+        wait_vmcnt<0>();
+        lds_barrier();
+        if (s + 1 < S) {
+            issue_w(s + 1);
+            load_codes(s + 1);
+        }
+        const unsigned char* wb = smem_raw + (s & 1) * F::WSTAGE;
+#pragma unroll
+        for (int k16 = 0; k16 < DT_K / 16; ++k16) {
+            if (16 * k16 >= kn) break;
+            const int sw = 16 * ((2 * k16 + hf) ^ ((l32 >> 1) & 7));
+            bf16x8 wf[2], af[MI];
+#pragma unroll
+            for (int j = 0; j < 2; ++j)
+                wf[j] = lds_b128(reinterpret_cast<const uint16_t*>(
+                    wb + (64 * wc + 32 * j + l32) * (DT_K * 2) + sw));
+#pragma unroll
+            for (int i = 0; i < MI; ++i)
+                af[i] = lds_b128(reinterpret_cast<const uint16_t*>(
+                    aimg + (32 * (MI * wr + i) + l32) * (DT_K * 2) + sw));
+#pragma unroll
+            for (int i = 0; i < MI; ++i)
+#pragma unroll
+                for (int j = 0; j < 2; ++j) acc[i][j] = mfma32(wf[j], af[i], acc[i][j]);
+        }
+        lds_barrier();
+    }
+    const uint16_t** crow = reinterpret_cast<const uint16_t**>(smem_raw + F::CROW);
+    if (aq == 0) crow[arow] = my_crow;
+    // bf16(acc + mean) to LDS: lane (hf, l32) holds row l32 of its tiles,
+    // columns 8 q + 4 hf + [0, 4) for q = 0 .. 3
+    const int nl = 64 * wc + 4 * hf;
+    f32x4 mean[8];
+#pragma unroll
+    for (int jq = 0; jq < 8; ++jq) {
+        mean[jq] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+        if (B.mean) {
+            __builtin_memcpy(&mean[jq], B.mean + min(n0 + nl + 8 * jq, B.HD - 4), 16);
+        }
+    }
+#pragma unroll
+    for (int jq = 0; jq < 8; ++jq) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) mean[jq][e] = bf16_round(mean[jq][e]);
+#pragma unroll
+        for (int i = 0; i < MI; ++i) {
+            const f32x16& v = acc[i][jq >> 2];
+            u32x2 o;
+#pragma unroll
+            for (int e = 0; e < 2; ++e)
+                o[e] = pack_bf16x2(v[4 * (jq & 3) + 2 * e] + mean[jq][2 * e],
+                                   v[4 * (jq & 3) + 2 * e + 1] + mean[jq][2 * e + 1]);
+            *reinterpret_cast<u32x2*>(smem_raw + (32 * (MI * wr + i) + l32) * F::OSTRIDE +
+                                      2 * (nl + 8 * jq)) = o;
+        }
+    }
+    __syncthreads();
+    // out: consecutive threads take consecutive 16-byte pieces of a row
+    constexpr int CH = F::COLS / 8, RSTEP = F::THREADS / CH;
+    const int frow = t / CH, fch = t % CH, n = n0 + 8 * fch;
+    if (n >= B.HD) return;
+    const int rows = (int)min(P.M - m0, (int64_t)F::ROWS);
+    uint16_t* out = P.out + (m0 + frow) * B.HD + n;
+    const unsigned char* st = smem_raw + frow * F::OSTRIDE + 16 * fch;
+    // a large output (16 MB and more) streams past the L2, which then keeps
+    // W_dec and the centers: 56.5 -> 52.7 us for 12,480 x 3,072 at r = 384
+    auto put = [&](int u, const u32x4& v) {
+        u32x4* o = reinterpret_cast<u32x4*>(out + (int64_t)RSTEP * u * B.HD);
+        if constexpr (F::BIG) __builtin_nontemporal_store(v, o);
+        else *o = v;
+    };
+    if (P.centers) {
+        u32x4 cv[F::UNITS];   // rows past the end have the last row's center
+#pragma unroll
+        for (int u = 0; u < F::UNITS; ++u)
+            cv[u] = ldg(reinterpret_cast<const u32x4*>(crow[frow + RSTEP * u] + n));
+#pragma unroll
+        for (int u = 0; u < F::UNITS; ++u) {
+            u32x4 v = *reinterpret_cast<const u32x4*>(st + RSTEP * u * F::OSTRIDE);
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+                v[e] = pack_bf16x2(__uint_as_float(v[e] << 16) + __uint_as_float(cv[u][e] << 16),
+                                   __uint_as_float(v[e] & 0xffff0000u) +
+                                       __uint_as_float(cv[u][e] & 0xffff0000u));
+            if (frow + RSTEP * u < rows) put(u, v);
+        }
+    } else {
+#pragma unroll
+        for (int u = 0; u < F::UNITS; ++u)
+            if (frow + RSTEP * u < rows)
+                put(u, *reinterpret_cast<const u32x4*>(st + RSTEP * u * F::OSTRIDE));
+    }
+}
+
+using DecBig = DecFmt<2, 2, 4>;
+using DecSmall = DecFmt<1, 2, 2>;
+static_assert(2 * DecBig::SMEM <= 160 * 1024, "two blocks per CU");
+
 }  // namespace nkv
 
 using namespace nkv;
@@ -1751,8 +1999,9 @@ extern "C" int nkv_encode_batch(void* stream, const nkv_encode_args* args, int n
     return encode_batch((hipStream_t)stream, args, n);
 }
 
-extern "C" int nkv_decode(void* stream, const nkv_decode_args* a) {
-    clear_error();
+namespace {
+
+int check_decode(const nkv_decode_args* a) {
     NKV_REQUIRE(a, NKV_ERR_INVALID, "null args");
     const nkv_codec& c = a->codec;
     NKV_REQUIRE(a->B >= 1 && a->N >= 0 && a->rows >= 0, NKV_ERR_INVALID, "bad B/N/rows");
@@ -1770,28 +2019,154 @@ extern "C" int nkv_decode(void* stream, const nkv_decode_args* a) {
     }
     if (a->rows == 0) return NKV_OK;
     NKV_REQUIRE(c.packed && c.scales && c.w_dec && a->out, NKV_ERR_INVALID, "null pointer");
-    hipStream_t s = (hipStream_t)stream;
+    return NKV_OK;
+}
+
+// Batch item b of a decode call as one problem.
+DecProb dec_problem(const nkv_decode_args* a, int b) {
+    const nkv_codec& c = a->codec;
+    DecProb p;
+    p.packed = c.packed + (int64_t)b * a->N * (c.r / 2);
+    p.scales = c.scales + (int64_t)b * a->N * (c.r / c.group);
+    p.ids = c.ids ? (const void*)((const uint8_t*)c.ids + (int64_t)b * a->N * c.id_bytes) : nullptr;
+    p.centers = c.centers ? c.centers + (int64_t)b * c.centers_batch_stride : nullptr;
+    p.row_index = a->row_index;
+    p.out = a->out + (int64_t)b * a->rows * a->HD;
+    p.M = a->rows;
+    p.id_bytes = c.id_bytes;
+    p.num_centers = c.num_centers;
+    return p;
+}
+
+// The staged kernel's 8- and 16-byte accesses (r % 32 == 0 and HD % 32 == 0
+// keep every row aligned when its base is).
+bool dec_aligned(const DecProb& p, const uint16_t* w) {
+    auto at = [](const void* q, uintptr_t n) { return reinterpret_cast<uintptr_t>(q) % n == 0; };
+    return at(p.packed, 8) && at(p.centers, 16) && at(p.out, 16) && at(w, 16);
+}
+
+template <int MI, int WR, int WC>
+int launch_decode_tiles(hipStream_t s, DecBatch& B, int64_t rows) {
+    using F = DecFmt<MI, WR, WC>;
+    static const hipError_t attr = hipFuncSetAttribute(
+        (const void*)decode_tile_kernel<MI, WR, WC>, hipFuncAttributeMaxDynamicSharedMemorySize, F::SMEM);
+    NKV_REQUIRE(attr == hipSuccess, NKV_ERR_HIP, "hipFuncSetAttribute failed for the decode kernels");
+    const int64_t items = B.n * cdiv(rows, F::ROWS) * cdiv(B.HD, F::COLS);
+    NKV_REQUIRE(items < INT32_MAX - 8, NKV_ERR_UNSUPPORTED, "decode grid too large");
+    B.row_blocks = (uint32_t)cdiv(rows, F::ROWS);
+    decode_tile_kernel<MI, WR, WC><<<xcd_grid(items), F::THREADS, F::SMEM, s>>>(B);
+    NKV_LAUNCH_CHECK();
+    return NKV_OK;
+}
+
+int launch_decode(hipStream_t s, const nkv_decode_args* first, const DecProb* p, int n) {
+    const nkv_codec& c = first->codec;
+    for (int i0 = 0; i0 < n; i0 += DEC_MAXB) {
+        DecBatch B{};
+        B.n = std::min(n - i0, DEC_MAXB);
+        B.w = c.w_dec;
+        B.mean = c.mean;
+        B.HD = first->HD;
+        B.r = c.r;
+        B.group = c.group;
+        B.scale_dtype = c.scale_dtype;
+        int64_t rows = 0, big = 0;
+        for (int i = 0; i < B.n; ++i) {
+            B.p[i] = p[i0 + i];
+            rows = std::max(rows, B.p[i].M);
+            big += cdiv(B.p[i].M, DecBig::ROWS) * cdiv(B.HD, DecBig::COLS);
+        }
+        // one round of 128 x 256 tiles over the 256 CUs, or more: those; below,
+        // 64 x 128 tiles (four times the blocks).  1,017 x 2,048 at r = 256:
+        // 9.4 us with the small tiles on 256 CUs, 64 blocks of the large ones
+        const int rc = big >= 256 ? launch_decode_tiles<2, 2, 4>(s, B, rows)
+                                  : launch_decode_tiles<1, 2, 2>(s, B, rows);
+        if (rc) return rc;
+    }
+    return NKV_OK;
+}
+
+int decode_one(hipStream_t s, const nkv_decode_args* a) {
+    const nkv_codec& c = a->codec;
+    if (a->rows == 0) return NKV_OK;
+    bool aligned = true;
+    for (int b = 0; b < a->B; ++b) aligned = aligned && dec_aligned(dec_problem(a, b), c.w_dec);
+    if (aligned) {
+        DecProb p[DEC_MAXB];
+        for (int b0 = 0; b0 < a->B; b0 += DEC_MAXB) {
+            const int nb = std::min(a->B - b0, DEC_MAXB);
+            for (int b = 0; b < nb; ++b) p[b] = dec_problem(a, b0 + b);
+            const int rc = launch_decode(s, a, p, nb);
+            if (rc) return rc;
+        }
+        return NKV_OK;
+    }
     dim3 grid((unsigned)cdiv(a->rows, GT_M), (unsigned)cdiv(a->HD, GT_N));
     for (int b = 0; b < a->B; ++b) {
+        const DecProb p = dec_problem(a, b);
         DecodeA al;
-        al.packed = c.packed + (int64_t)b * a->N * (c.r / 2);
-        al.scales = c.scales + (int64_t)b * a->N * (c.r / c.group);
-        al.row_index = a->row_index;
+        al.packed = p.packed;
+        al.scales = p.scales;
+        al.row_index = p.row_index;
         al.scale_dtype = c.scale_dtype;
         al.group = c.group;
-        al.M = a->rows;
+        al.M = p.M;
         al.K = c.r;
         DecodeEpi ep;
-        ep.centers = c.centers ? c.centers + (int64_t)b * c.centers_batch_stride : nullptr;
-        ep.ids = c.ids ? (const void*)((const uint8_t*)c.ids + (int64_t)b * a->N * c.id_bytes)
-                       : nullptr;
+        ep.centers = p.centers;
+        ep.ids = p.ids;
         ep.id_bytes = c.id_bytes;
         ep.num_centers = c.num_centers;
-        ep.row_index = a->row_index;
+        ep.row_index = p.row_index;
         ep.mean = c.mean;
-        decode_gemm_kernel<<<grid, 256, 0, s>>>(al, ep, c.w_dec, a->HD,
-                                                a->out + (int64_t)b * a->rows * a->HD);
+        decode_gemm_kernel<<<grid, 256, 0, s>>>(al, ep, c.w_dec, a->HD, p.out);
         NKV_LAUNCH_CHECK();
     }
     return NKV_OK;
+}
+
+}  // namespace
+
+extern "C" int nkv_decode(void* stream, const nkv_decode_args* a) {
+    clear_error();
+    const int rc = check_decode(a);
+    return rc ? rc : decode_one((hipStream_t)stream, a);
+}
+
+extern "C" int nkv_decode_batch(void* stream, const nkv_decode_args* a, int n) {
+    clear_error();
+    NKV_REQUIRE(n >= 0 && (n == 0 || a), NKV_ERR_INVALID, "null args");
+    bool one = true;
+    for (int i = 0; i < n; ++i) {
+        const int rc = check_decode(a + i);
+        if (rc) return rc;
+        const nkv_codec &c = a[i].codec, &f = a[0].codec;
+        NKV_REQUIRE(a[i].HD == a[0].HD && c.r == f.r && c.group == f.group &&
+                        c.scale_dtype == f.scale_dtype && c.w_dec == f.w_dec && c.mean == f.mean,
+                    NKV_ERR_INVALID,
+                    "the decodes of one batch must share HD, r, group, scale dtype, w_dec and mean");
+        for (int b = 0; b < a[i].B && a[i].rows > 0; ++b)
+            one = one && dec_aligned(dec_problem(a + i, b), c.w_dec);
+    }
+    hipStream_t s = (hipStream_t)stream;
+    if (!one) {
+        for (int i = 0; i < n; ++i) {
+            const int rc = decode_one(s, a + i);
+            if (rc) return rc;
+        }
+        return NKV_OK;
+    }
+    DecProb p[DEC_MAXB];
+    int np = 0;
+    for (int i = 0; i < n; ++i) {
+        for (int b = 0; b < a[i].B && a[i].rows > 0; ++b) {
+            p[np++] = dec_problem(a + i, b);
+            if (np == DEC_MAXB) {
+                const int rc = launch_decode(s, a, p, np);
+                if (rc) return rc;
+                np = 0;
+            }
+        }
+    }
+    return np ? launch_decode(s, a, p, np) : NKV_OK;
 }

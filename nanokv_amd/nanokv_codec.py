@@ -473,7 +473,16 @@ def decode_value(value: Any, *, dtype: torch.dtype, device: torch.device) -> tor
     if torch.is_tensor(value):
         return value.to(device=device, dtype=dtype)
     if value.get("codec") == SEGMENTS:
-        parts = [decode_value(item, dtype=dtype, device=device) for item in value["segments"]]
+        segments = value["segments"]
+        if len(segments) > 1 and all(is_payload(p) and p["codec"] == CODEC for p in segments):
+            views = [codec_view(p, torch.device(device)) for p in segments]
+            first = views[0]
+            if all(v.batch == 1 and v.w_dec is first.w_dec and v.mean is first.mean
+                   and (v.group, v.scales.dtype) == (first.group, first.scales.dtype)
+                   for v in views):
+                # one operator: every segment straight into its rows of the result
+                return ops.decode_batch(views, int(segments[0]["shape"][2])).to(dtype)
+        parts = [decode_value(item, dtype=dtype, device=device) for item in segments]
         return torch.cat(parts, dim=1) if parts else None
     return decode_tensor(value, dtype=dtype, device=device)
 

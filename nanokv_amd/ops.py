@@ -400,24 +400,48 @@ class Codec:
         return c
 
 
+def _decode_args(codec: Codec, hd: int) -> NkvDecodeArgs:
+    """nkv_decode_args of every row of a flat codec (out not set)."""
+    codec.validate(hd)
+    args = NkvDecodeArgs()
+    args.B, args.HD, args.N = codec.batch, hd, codec.tokens
+    args.rows = codec.tokens
+    args.codec = codec.struct()
+    return args
+
+
 def decode(codec: Codec, hd: int, row_index: Optional[torch.Tensor] = None) -> torch.Tensor:
     """Full-width bf16 decode [B, rows, HD] of all or selected rows (a flat
     codec; the segments of a segment list are decoded one by one)."""
     if codec.segments is not None:
         raise ValueError("decode takes a flat codec; decode segments one at a time")
     device = _require_gpu(codec.packed, row_index)
-    codec.validate(hd)
-    args = NkvDecodeArgs()
-    args.B, args.HD, args.N = codec.batch, hd, codec.tokens
+    args = _decode_args(codec, hd)
     if row_index is not None:
         _contig(row_index, torch.int32, "row_index")
         args.rows, args.row_index = row_index.numel(), row_index.data_ptr()
-    else:
-        args.rows = codec.tokens
-    args.codec = codec.struct()
     out = torch.empty((codec.batch, int(args.rows), hd), device=device, dtype=torch.bfloat16)
     args.out = out.data_ptr()
     check("nkv_decode", lib().nkv_decode(_stream(device), byref(args)))
+    return out
+
+
+def decode_batch(codecs: list, hd: int) -> torch.Tensor:
+    """Full-width bf16 decode [1, total rows, HD] of the flat codecs of one
+    operator (the segments of a one-item cache), written one after the other
+    into one tensor by one call (nkv_decode_batch)."""
+    device = _require_gpu(*[c.packed for c in codecs])
+    if any(c.segments is not None or c.batch != 1 for c in codecs):
+        raise ValueError("decode_batch takes flat codecs of batch 1")
+    built = [_decode_args(c, hd) for c in codecs]
+    out = torch.empty((1, sum(int(a.rows) for a in built), hd), device=device,
+                      dtype=torch.bfloat16)
+    base = out.data_ptr()
+    for a in built:
+        a.out = base
+        base += 2 * int(a.rows) * hd
+    arr = (NkvDecodeArgs * len(built))(*built)
+    check("nkv_decode_batch", lib().nkv_decode_batch(_stream(device), arr, len(built)))
     return out
 
 
