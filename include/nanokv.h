@@ -351,6 +351,34 @@ int nkv_c64_fit(void* stream, const float* x, int B, int64_t S, int HD, int C, i
                 size_t workspace_bytes);
 
 /*
+ * nkv_c64_fit with fp32 (x) or bf16 (x_bf16, read as value.float(), exact)
+ * rows, and the payload's forms of its results: centers_bf16 [B, C, HD] the
+ * centers rounded to bf16 (store_centers, MG:69-90), ids_u8 [B, S] the labels
+ * as uint8; each may be NULL.  bf16 rows need HD % 32 == 0, 16-byte alignment
+ * and at least one round, the two optional outputs at least one round
+ * (NKV_ERR_UNSUPPORTED otherwise).
+ */
+typedef struct nkv_c64_fit_args {
+    int B;
+    int HD;
+    int64_t S;
+    int C;
+    int iterations;
+    const float* x;
+    const uint16_t* x_bf16;
+    const int32_t* init_rows;     /* [C] in device memory, or NULL: init_rows_host */
+    const int32_t* init_rows_host;  /* [C] in host memory, read during the call */
+    float* centers;               /* [B, C, HD] */
+    uint16_t* centers_bf16;
+    int32_t* labels;              /* [B, S] */
+    uint8_t* ids_u8;
+    void* workspace;
+    size_t workspace_bytes;
+} nkv_c64_fit_args;
+
+int nkv_c64_fit_rows(void* stream, const nkv_c64_fit_args* args);
+
+/*
  * Full-width decode of all or selected rows to bf16 (the reference's decode
  * path, used for decode_value / decode_pair_selected):
  *   rows = bf16(latent @ w_dec^T + bf16(mean))                  MG:438-443

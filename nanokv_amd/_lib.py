@@ -35,7 +35,7 @@ EXPORTED = (
     "nkv_fast_attend_workspace_size", "nkv_fast_attend", "nkv_rope_apply", "nkv_int8_pack",
     "nkv_int8_dequant", "nkv_c64_fit_workspace_size", "nkv_c64_fit", "nkv_camera_apply",
     "nkv_attend_static", "nkv_lift_lse_combine", "nkv_finish", "nkv_reader_rows",
-    "nkv_decode_batch",
+    "nkv_decode_batch", "nkv_c64_fit_rows",
 )
 NKV_STATIC_SCRATCH_BYTES = 64 << 20
 
@@ -67,6 +67,15 @@ class NkvEncodeArgs(Structure):
         ("x", c_void_p), ("centers", c_void_p), ("mean", c_void_p), ("w_enc", c_void_p),
         ("ids", c_void_p), ("coeff", c_void_p), ("packed", c_void_p), ("scales", c_void_p),
         ("x_bf16", c_void_p), ("x_stride", c_int64),
+    ]
+
+
+class NkvC64FitArgs(Structure):
+    _fields_ = [
+        ("B", c_int), ("HD", c_int), ("S", c_int64), ("C", c_int), ("iterations", c_int),
+        ("x", c_void_p), ("x_bf16", c_void_p), ("init_rows", c_void_p), ("init_rows_host", c_void_p),
+        ("centers", c_void_p), ("centers_bf16", c_void_p), ("labels", c_void_p), ("ids_u8", c_void_p),
+        ("workspace", c_void_p), ("workspace_bytes", c_size_t),
     ]
 
 
@@ -230,6 +239,8 @@ def _declare(lib: ctypes.CDLL) -> None:
     lib.nkv_c64_fit.restype = c_int
     lib.nkv_c64_fit.argtypes = [c_void_p, c_void_p, c_int, c_int64, c_int, c_int, c_int, c_void_p,
                                 c_void_p, c_void_p, c_void_p, c_size_t]
+    lib.nkv_c64_fit_rows.restype = c_int
+    lib.nkv_c64_fit_rows.argtypes = [c_void_p, POINTER(NkvC64FitArgs)]
     lib.nkv_int8_pack.restype = c_int
     lib.nkv_int8_pack.argtypes = [c_void_p, c_void_p, c_int64, c_int, c_int, c_void_p, c_void_p]
     lib.nkv_int8_dequant.restype = c_int

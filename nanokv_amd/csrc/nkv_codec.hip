@@ -9,32 +9,52 @@
 namespace nkv {
 
 // ============================================================ quantiser
-// One thread per (row, group).  Each thread reads its group with 16-byte
-// loads, computes the exact amax (order-free), the IEEE-divided scale, and
-// writes group/2 packed bytes plus one scale.  Reference: MG:349-351 (fp32
-// arithmetic as in HY kv_codecs.py:244-255; bf16 arithmetic as MG deploys
-// it) and _pack_int4 MG:282-292.
+// quant_lanes(group) lanes of a wave share one (row, group): each takes runs
+// of 8 coefficients (two 16-byte loads, whole rows coalesced over the wave),
+// the exact amax (order-free) meets by lane exchanges, and every run becomes
+// one dword of codes; lane 0 of the group stores the IEEE-divided scale.  (One
+// thread per group read a row stride per load and had 1,560 threads for a
+// chunk with one scale per row: 51 us at r = 384, now 4.)  Reference:
+// MG:349-351 (fp32 arithmetic as in HY kv_codecs.py:244-255; bf16 arithmetic
+// as MG deploys it) and _pack_int4 MG:282-292.
+__host__ __device__ __forceinline__ int quant_lanes(int group) {
+    int n = 1;
+    while (n < 64 && 8 * n < group) n *= 2;
+    return n;
+}
+
+// Lane `sub` of the lpg lanes (aligned in the wave) of group gid; every lane
+// of the wave calls.
 template <int QUANT_MODE>
 __device__ __forceinline__ void quant_pack_group(const float* __restrict__ coeff, int64_t rows,
                                                  int r, int group, int scale_dtype,
                                                  uint8_t* __restrict__ packed,
-                                                 uint16_t* __restrict__ scales, int64_t gid) {
+                                                 uint16_t* __restrict__ scales, int64_t gid,
+                                                 int sub, int lpg) {
     const int ngroups = r / group;
-    if (gid >= rows * ngroups) return;
-    const int64_t row = gid / ngroups;
-    const int g = (int)(gid - row * ngroups);
+    const bool ok = gid < rows * ngroups;
+    const int64_t row = ok ? gid / ngroups : 0;
+    const int g = ok ? (int)(gid - row * ngroups) : 0;
     const float* x = coeff + row * r + (int64_t)g * group;
 
     float amax = 0.0f;
-    for (int j = 0; j < group; j += 4) {
-        f32x4 v = *reinterpret_cast<const f32x4*>(x + j);
+    f32x4 v0 = {}, v1 = {};
+    for (int j = 8 * sub; ok && j < group; j += 8 * lpg) {
+        v0 = *reinterpret_cast<const f32x4*>(x + j);
+        v1 = *reinterpret_cast<const f32x4*>(x + j + 4);
 #pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            float a = QUANT_MODE == NKV_QUANT_BF16 ? bf16_round(v[e]) : v[e];
+        for (int e = 0; e < 8; ++e) {
+            const float v = e < 4 ? v0[e] : v1[e - 4];
+            float a = QUANT_MODE == NKV_QUANT_BF16 ? bf16_round(v) : v;
             a = fabsf(a);
             amax = (a > amax || a != a) ? a : amax;  // NaN propagates like torch.amax
         }
     }
+    for (int off = 1; off < lpg; off <<= 1) {
+        const float o = __shfl_xor(amax, off);
+        amax = (o > amax || o != o) ? o : amax;
+    }
+    if (!ok) return;
     float s;
     const float eps = 1.1920928955078125e-07f;  // torch.finfo(torch.float32).eps
     float clamped = (amax > eps || amax != amax) ? amax : eps;
@@ -43,13 +63,16 @@ __device__ __forceinline__ void quant_pack_group(const float* __restrict__ coeff
     } else {
         s = __fdiv_rn(clamped, 7.0f);
     }
-    scales[row * ngroups + g] =
-        scale_dtype == NKV_DTYPE_FP16 ? f32_to_f16_bits(s) : f32_to_bf16_bits(s);
+    if (sub == 0)
+        scales[row * ngroups + g] =
+            scale_dtype == NKV_DTYPE_FP16 ? f32_to_f16_bits(s) : f32_to_bf16_bits(s);
 
     uint8_t* out = packed + row * (r / 2) + (int64_t)g * (group / 2);
-    for (int j = 0; j < group; j += 8) {
-        f32x4 v0 = *reinterpret_cast<const f32x4*>(x + j);
-        f32x4 v1 = *reinterpret_cast<const f32x4*>(x + j + 4);
+    for (int j = 8 * sub; j < group; j += 8 * lpg) {
+        if (group > 8 * lpg) {  // more than one run per lane: read again
+            v0 = *reinterpret_cast<const f32x4*>(x + j);
+            v1 = *reinterpret_cast<const f32x4*>(x + j + 4);
+        }
         uint32_t word = 0;
 #pragma unroll
         for (int e = 0; e < 8; ++e) {
@@ -71,8 +94,9 @@ __global__ void __launch_bounds__(256) quant_pack_kernel(const float* __restrict
                                                          int scale_dtype,
                                                          uint8_t* __restrict__ packed,
                                                          uint16_t* __restrict__ scales) {
+    const int lpg = quant_lanes(group), t = threadIdx.x;
     quant_pack_group<QUANT_MODE>(coeff, rows, r, group, scale_dtype, packed, scales,
-                                 (int64_t)blockIdx.x * blockDim.x + threadIdx.x);
+                                 (int64_t)blockIdx.x * (256 / lpg) + t / lpg, t % lpg, lpg);
 }
 
 // ============================================================ unpack
@@ -453,8 +477,9 @@ template <int QUANT_MODE>
 __global__ void __launch_bounds__(256) quant_pack_batch_kernel(EncBatch B, int group,
                                                                int scale_dtype) {
     const EncProb& P = B.p[blockIdx.y];
+    const int lpg = quant_lanes(group), t = threadIdx.x;
     quant_pack_group<QUANT_MODE>(P.coeff, P.M, B.r, group, scale_dtype, P.packed, P.scales,
-                                 (int64_t)blockIdx.x * blockDim.x + threadIdx.x);
+                                 (int64_t)blockIdx.x * (256 / lpg) + t / lpg, t % lpg, lpg);
 }
 
 // The search's small block state: ||x||^2 per row, the per-wave bounds U,
@@ -1125,12 +1150,18 @@ __global__ void __launch_bounds__(64 * EP_WAVES) encode_proj_kernel(EncBatch B) 
     // whole groups): the coefficients just stored, read back after the barrier
     __syncthreads();
     const int G = B.qgroup, ngroups = r / G, gpb = (min(r - n0, EP_COLS)) / G;
-    for (int it = t; it < EP_ROWS * gpb; it += 64 * EP_WAVES) {
-        const int64_t gid = (m0 + it / gpb) * ngroups + n0 / G + it % gpb;
+    const int lpg = quant_lanes(G);
+    for (int it0 = 0; it0 < EP_ROWS * gpb; it0 += 64 * EP_WAVES / lpg) {
+        const int it = it0 + t / lpg;
+        // (groups past the block's last: out of range, like rows past the end)
+        const int64_t gid = it < EP_ROWS * gpb ? (m0 + it / gpb) * ngroups + n0 / G + it % gpb
+                                               : P.M * ngroups;
         if (B.quant_mode == NKV_QUANT_BF16)
-            quant_pack_group<NKV_QUANT_BF16>(P.coeff, P.M, r, G, B.scale_dtype, P.packed, P.scales, gid);
+            quant_pack_group<NKV_QUANT_BF16>(P.coeff, P.M, r, G, B.scale_dtype, P.packed, P.scales, gid,
+                                             t % lpg, lpg);
         else
-            quant_pack_group<NKV_QUANT_FP32>(P.coeff, P.M, r, G, B.scale_dtype, P.packed, P.scales, gid);
+            quant_pack_group<NKV_QUANT_FP32>(P.coeff, P.M, r, G, B.scale_dtype, P.packed, P.scales, gid,
+                                             t % lpg, lpg);
     }
 }
 
@@ -1522,7 +1553,7 @@ extern "C" int nkv_quant_pack(void* stream, const float* coeff, int64_t rows, in
                 "bad quant_mode");
     if (rows == 0) return NKV_OK;
     NKV_REQUIRE(coeff && packed && scales, NKV_ERR_INVALID, "null pointer");
-    const int64_t threads = rows * (r / group);
+    const int64_t threads = rows * (r / group) * quant_lanes(group);
     dim3 grid((unsigned)cdiv(threads, 256));
     hipStream_t s = (hipStream_t)stream;
     if (quant_mode == NKV_QUANT_BF16)
@@ -1593,9 +1624,21 @@ namespace nkv {
 // row order (a stable counting sort), summed in fp64 in that order, rounded
 // to fp32 and divided by the count in fp32.
 
+constexpr int FIT_MAXC = 256;
+
+// The initial center rows: in device memory (dev), or a host list carried in
+// the kernel arguments (no copy to the device, which would wait for the stream).
+struct FitInit {
+    const int32_t* dev;
+    int32_t v[FIT_MAXC];
+    __device__ __forceinline__ int64_t row(int c, int64_t S) const {
+        return min(max((int64_t)(dev ? dev[c] : v[c]), (int64_t)0), S - 1);
+    }
+};
+
 __global__ void __launch_bounds__(256) c64_init_kernel(const float* __restrict__ x, int B, int64_t S,
                                                        int HD, int C,
-                                                       const int32_t* __restrict__ init_rows,
+                                                       FitInit init,
                                                        float* __restrict__ centers) {
     const int64_t total = (int64_t)B * C * HD;
     for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < total;
@@ -1603,75 +1646,245 @@ __global__ void __launch_bounds__(256) c64_init_kernel(const float* __restrict__
         const int d = (int)(i % HD);
         const int c = (int)((i / HD) % C);
         const int64_t b = i / ((int64_t)HD * C);
-        const int64_t row = min(max((int64_t)init_rows[c], (int64_t)0), S - 1);
+        const int64_t row = init.row(c, S);
         centers[i] = x[(b * S + row) * HD + d];
     }
 }
 
-constexpr int FIT_THREADS = 256, FIT_MAXC = 256;
+// Eight consecutive values of a row as exact doubles: fp32 or bf16 storage.
+template <bool XB>
+struct Row8 {
+    u32x4 w[XB ? 1 : 2];
+    __device__ __forceinline__ void load(const void* base, int64_t at) {
+        if constexpr (XB) {
+            w[0] = ldg(reinterpret_cast<const u32x4*>(reinterpret_cast<const uint16_t*>(base) + at));
+        } else {
+            const float* p = reinterpret_cast<const float*>(base) + at;
+            w[0] = ldg(reinterpret_cast<const u32x4*>(p));
+            w[1] = ldg(reinterpret_cast<const u32x4*>(p + 4));
+        }
+    }
+    __device__ __forceinline__ double get(int e) const {
+        if constexpr (XB)
+            return (double)__uint_as_float((e & 1) ? (w[0][e >> 1] & 0xffff0000u) : (w[0][e >> 1] << 16));
+        else
+            return (double)__uint_as_float(w[e >> 2][e & 3]);
+    }
+};
 
-// One block per batch item: cluster sizes, their exclusive offsets, and the
-// rows of each cluster in row order (order[offset[c] + k] = k-th row of c).
-__global__ void __launch_bounds__(FIT_THREADS) c64_sort_kernel(const int32_t* __restrict__ labels,
-                                                                int64_t S, int C,
-                                                                int32_t* __restrict__ counts,
-                                                                int32_t* __restrict__ offsets,
-                                                                int32_t* __restrict__ order) {
-    __shared__ int cnt[FIT_MAXC], cur[FIT_MAXC], lab[FIT_THREADS];
-    const int t = threadIdx.x;
-    const int64_t b = blockIdx.x;
-    const int32_t* lb = labels + b * S;
-    for (int c = t; c < C; c += FIT_THREADS) cnt[c] = 0;
-    __syncthreads();
-    for (int64_t i = t; i < S; i += FIT_THREADS) atomicAdd(&cnt[min(max(lb[i], 0), C - 1)], 1);
-    __syncthreads();
-    if (t == 0) {
-        int run = 0;
-        for (int c = 0; c < C; ++c) {
-            cur[c] = run;
-            run += cnt[c];
+// The fit's nearest-center search on fp64 MFMA: every product is exact, so
+// the decision is that of assign_kernel.  A block of eight waves owns 16 rows
+// x 32 centers (two 16 x 16 tiles per wave) and splits HD over its waves
+// (wave w: the 32-wide steps w, w + 8, ..); the partial sums meet in LDS and
+// are added in wave order.  At C = 64 a chunk of 1,560 rows is 196 blocks of
+// eight waves: one wave per 16 rows x 64 centers (the whole HD each, 98 waves
+// with work) took 132 us per round, this 11 us.  In a step lane l holds
+// row / center l % 16, k 8 (l / 16) .. +8: whole 128-byte lines per row, and
+// any order of k is valid for the products.  Bound by the fp64 matrix rate
+// (0.61 GFLOP per round of 64 centers, 32 flop per cycle and SIMD).
+// part_d / part_c [center blocks][B * S]: the best center of each block.
+// FIRST: the centers are the initial rows of x.  HD % 32 == 0, 16-byte rows.
+constexpr int FS_ROWS = 16, FS_CENT = 32, FS_WAVES = 8, FS_AHEAD = 2;
+
+template <bool XB, bool FIRST>
+__global__ void __launch_bounds__(64 * FS_WAVES) fit_search_kernel(
+    const void* __restrict__ x, const float* __restrict__ centers, FitInit init, int64_t S, int HD,
+    int C, double* __restrict__ part_d,
+    int32_t* __restrict__ part_c) {
+    constexpr bool CB = FIRST && XB;   // the centers' storage is bf16
+    // partial sums [wave][tile][element][lane], then ||c||^2 [wave][tile][lane]
+    __shared__ double red[FS_WAVES][2][5][64];
+    const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+    const int g = lane >> 4, col = lane & 15;
+    const int64_t row0 = (int64_t)blockIdx.x * FS_ROWS, b = blockIdx.z;
+    const int c0 = blockIdx.y * FS_CENT;
+    const int64_t xr = (b * S + min(row0 + col, S - 1)) * HD + 8 * g;
+    int64_t cr[2];
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+        const int c = min(c0 + 16 * j + col, C - 1);
+        int64_t r = b * C + c;
+        if constexpr (FIRST) r = b * S + init.row(c, S);
+        cr[j] = r * HD + 8 * g;
+    }
+    const void* cbase = FIRST ? x : (const void*)centers;
+    const int NS = HD / 32;
+    Row8<XB> xa[FS_AHEAD];
+    Row8<CB> ca[FS_AHEAD][2];
+    auto issue = [&](int st, int slot) {
+        xa[slot].load(x, xr + 32 * st);
+#pragma unroll
+        for (int j = 0; j < 2; ++j) ca[slot][j].load(cbase, cr[j] + 32 * st);
+    };
+    f64x4 acc[2] = {};
+    double cc[2] = {0.0, 0.0};
+#pragma unroll
+    for (int i = 0; i < FS_AHEAD; ++i)
+        if (wave + FS_WAVES * i < NS) issue(wave + FS_WAVES * i, i);
+    for (int st0 = wave; st0 < NS; st0 += FS_WAVES * FS_AHEAD) {
+#pragma unroll
+        for (int i = 0; i < FS_AHEAD; ++i) {
+            const int st = st0 + FS_WAVES * i;
+            if (st >= NS) break;
+            const Row8<XB> xv = xa[i];
+            Row8<CB> cv[2];
+#pragma unroll
+            for (int j = 0; j < 2; ++j) cv[j] = ca[i][j];
+            if (st + FS_WAVES * FS_AHEAD < NS) issue(st + FS_WAVES * FS_AHEAD, i);
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                const double a = xv.get(e);
+#pragma unroll
+                for (int j = 0; j < 2; ++j) {
+                    const double q = cv[j].get(e);
+                    acc[j] = __builtin_amdgcn_mfma_f64_16x16x4f64(a, q, acc[j], 0, 0, 0);
+                    cc[j] = fma(q, q, cc[j]);
+                }
+            }
         }
     }
-    __syncthreads();
-    for (int c = t; c < C; c += FIT_THREADS) {
-        counts[b * C + c] = cnt[c];
-        offsets[b * C + c] = cur[c];
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) red[wave][j][e][lane] = acc[j][e];
+        red[wave][j][4][lane] = cc[j];
     }
-    for (int64_t i0 = 0; i0 < S; i0 += FIT_THREADS) {
-        const int64_t i = i0 + t;
-        const int L = i < S ? min(max(lb[i], 0), C - 1) : -1;
-        lab[t] = L;
-        __syncthreads();
-        if (L >= 0) {
-            // rows of this cluster earlier in the chunk come first
-            int rank = 0;
-            for (int u = 0; u < t; ++u) rank += lab[u] == L;
-            order[b * S + cur[L] + rank] = (int32_t)i;
-        }
-        __syncthreads();
-        if (L >= 0) atomicAdd(&cur[L], 1);
-        __syncthreads();
+    __syncthreads();
+    // thread t: row t / 32, center t % 32 of the block.  Element e of lane
+    // 16 g + col is row 4 e + g, column col; ||c||^2 is over the four g.
+    const int row = t >> 5, cl = t & 31, j = cl >> 4, cc16 = cl & 15;
+    double dot = 0.0, cn = 0.0;
+    for (int w = 0; w < FS_WAVES; ++w) {
+        dot += red[w][j][row >> 2][16 * (row & 3) + cc16];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) cn += red[w][j][4][16 * q + cc16];
+    }
+    double bd = cn - 2.0 * dot;
+    int bc = c0 + cl < C ? c0 + cl : -1;
+#pragma unroll
+    for (int off = 1; off < 32; off <<= 1) {
+        const double od = __shfl_xor(bd, off);
+        const int oc = __shfl_xor(bc, off);
+        if (better(od, oc, bd, bc)) { bd = od; bc = oc; }
+    }
+    if (cl == 0 && row0 + row < S) {
+        const int64_t at = (int64_t)blockIdx.y * gridDim.z * S + b * S + row0 + row;
+        part_d[at] = bd;
+        part_c[at] = bc;
     }
 }
 
-// grid (cdiv(HD, 256), C, B): one thread per center element.
-__global__ void __launch_bounds__(256) c64_update_kernel(const float* __restrict__ x, int64_t S,
-                                                         int HD, int C,
-                                                         const int32_t* __restrict__ counts,
-                                                         const int32_t* __restrict__ offsets,
-                                                         const int32_t* __restrict__ order,
-                                                         float* __restrict__ centers) {
-    const int d = blockIdx.x * 256 + threadIdx.x;
-    const int c = blockIdx.y;
-    const int64_t b = blockIdx.z;
-    if (d >= HD) return;
-    const int n = counts[b * C + c];
-    if (n == 0) return;  // an empty cluster keeps its center
-    const int32_t* ord = order + b * S + offsets[b * C + c];
-    const float* xb = x + b * S * HD + d;
+// Label of row i (of all B S rows) from the best centers of nc center blocks,
+// or (part_d null) the labels as they are.
+__device__ __forceinline__ int fit_label(const double* part_d, const int32_t* part_c, int nc,
+                                         int64_t total, int64_t i) {
+    int c = part_c[i];
+    if (!part_d) return c;
+    double d = part_d[i];
+    for (int k = 1; k < nc; ++k) {
+        const double od = part_d[k * total + i];
+        const int oc = part_c[k * total + i];
+        if (better(od, oc, d, c)) { d = od; c = oc; }
+    }
+    return c;
+}
+
+// labels[i] from more than two center blocks (the update reads one or two itself).
+__global__ void __launch_bounds__(256) fit_label_kernel(const double* __restrict__ part_d,
+                                                        const int32_t* __restrict__ part_c, int nc,
+                                                        int64_t total, int32_t* __restrict__ labels) {
+    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (i < total) labels[i] = fit_label(part_d, part_c, nc, total, i);
+}
+
+// One block per (256 columns, cluster c, batch item b): the mean of c's rows.
+// The block finds the rows itself, in row order: FU_SCAN labels at a time, a
+// ballot per 64 and the counts of the (round, wave) pairs before it (a
+// separate stable counting sort by one block took 27 us per round).  Each
+// thread then sums its column in that order in fp64, FU_FLY loads in flight
+// (22-32 us one at a time, now 6 us with the scan: 1,560 rows, 64 clusters;
+// bound by the latency of the largest cluster's row list).
+// FIRST: an empty cluster's center is its initial row (else it stays).
+// The blocks of the first columns write their rows' labels (null: they are
+// the labels read).
+constexpr int FU_SCAN = 2048, FU_FLY = 16;
+
+template <bool XB>
+__global__ void __launch_bounds__(256) fit_update_kernel(
+    const void* __restrict__ x, int64_t S, int HD, int C, const double* __restrict__ part_d,
+    const int32_t* __restrict__ part_c, int nc, FitInit init, int first,
+    float* __restrict__ centers, uint16_t* __restrict__ centers_bf16,
+    int32_t* __restrict__ labels, uint8_t* __restrict__ ids) {
+    __shared__ int32_t list[FU_SCAN];
+    __shared__ int cnt[FU_SCAN / 256][4];
+    const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+    const int d = blockIdx.x * 256 + t, c = blockIdx.y;
+    const int64_t b = blockIdx.z, total = (int64_t)gridDim.z * S;
+    auto at = [&](int64_t row) -> double {
+        const int64_t i = (b * S + row) * HD + d;
+        if constexpr (XB) return (double)bf16_bits_to_f32(ldg(reinterpret_cast<const uint16_t*>(x) + i));
+        else return (double)ldg(reinterpret_cast<const float*>(x) + i);
+    };
     double sum = 0.0;
-    for (int k = 0; k < n; ++k) sum += (double)xb[(int64_t)ord[k] * HD];
-    centers[(b * C + c) * HD + d] = __fdiv_rn((float)sum, (float)n);
+    int64_t n = 0;
+    for (int64_t s0 = 0; s0 < S; s0 += FU_SCAN) {
+        bool mine[FU_SCAN / 256];
+        int before[FU_SCAN / 256];
+#pragma unroll
+        for (int k = 0; k < FU_SCAN / 256; ++k) {
+            const int64_t row = s0 + 256 * k + t;
+            // labels outside the table count as its nearest entry
+            mine[k] = row < S && min(max(fit_label(part_d, part_c, nc, total, b * S + row), 0), C - 1) == c;
+            const uint64_t m = __ballot(mine[k]);
+            before[k] = __popcll(m & ((1ull << lane) - 1));
+            if (lane == 0) cnt[k][wave] = __popcll(m);
+        }
+        __syncthreads();
+        int run = 0;
+#pragma unroll
+        for (int k = 0; k < FU_SCAN / 256; ++k) {
+#pragma unroll
+            for (int w = 0; w < 4; ++w) {
+                if (w == wave && mine[k]) list[run + before[k]] = (int32_t)(s0 + 256 * k + t);
+                run += cnt[k][w];
+            }
+        }
+        __syncthreads();
+        if (blockIdx.x == 0) {
+            for (int k = t; k < run; k += 256) {
+                if (labels) labels[b * S + list[k]] = c;
+                if (ids) ids[b * S + list[k]] = (uint8_t)c;
+            }
+        }
+        if (d < HD) {
+            int k = 0;
+            for (; k + FU_FLY <= run; k += FU_FLY) {
+                double v[FU_FLY];
+#pragma unroll
+                for (int u = 0; u < FU_FLY; ++u) v[u] = at(list[k + u]);
+#pragma unroll
+                for (int u = 0; u < FU_FLY; ++u) sum += v[u];
+            }
+            for (; k < run; k += 4) {
+                double v[4];
+#pragma unroll
+                for (int u = 0; u < 4; ++u) v[u] = at(list[min(k + u, run - 1)]);
+#pragma unroll
+                for (int u = 0; u < 4; ++u)
+                    if (k + u < run) sum += v[u];
+            }
+        }
+        n += run;
+        __syncthreads();
+    }
+    if (d >= HD) return;
+    const int64_t o = (b * C + c) * HD + d;
+    float v;
+    if (n > 0) v = __fdiv_rn((float)sum, (float)n);
+    else if (first) v = (float)at(init.row(c, S));
+    else v = centers[o];
+    centers[o] = v;
+    if (centers_bf16) centers_bf16[o] = f32_to_bf16_bits(v);
 }
 
 __global__ void zero_i32_kernel(int32_t* p, int64_t n) {
@@ -1784,53 +1997,122 @@ namespace {
 size_t fit_ws_align(size_t n) { return (n + 255) / 256 * 256; }
 }  // namespace
 
+// Workspace of a fit: the best distance and center of every row per block of
+// FS_CENT centers.
+static size_t fit_part_bytes(int B, int64_t S, int C, size_t elem) {
+    return fit_ws_align((size_t)cdiv(C, FS_CENT) * B * S * elem);
+}
+
 extern "C" size_t nkv_c64_fit_workspace_size(int B, int64_t S, int C) {
     if (B <= 0 || S <= 0 || C <= 0) return 0;
-    return 2 * fit_ws_align((size_t)B * C * sizeof(int32_t)) +
-           fit_ws_align((size_t)B * S * sizeof(int32_t));
+    return fit_part_bytes(B, S, C, sizeof(double)) + fit_part_bytes(B, S, C, sizeof(int32_t));
 }
 
 extern "C" int nkv_c64_fit(void* stream, const float* x, int B, int64_t S, int HD, int C,
                            int iterations, const int32_t* init_rows, float* centers,
                            int32_t* labels, void* workspace, size_t workspace_bytes) {
+    nkv_c64_fit_args a{};
+    a.x = x;
+    a.B = B;
+    a.S = S;
+    a.HD = HD;
+    a.C = C;
+    a.iterations = iterations;
+    a.init_rows = init_rows;
+    a.centers = centers;
+    a.labels = labels;
+    a.workspace = workspace;
+    a.workspace_bytes = workspace_bytes;
+    return nkv_c64_fit_rows(stream, &a);
+}
+
+extern "C" int nkv_c64_fit_rows(void* stream, const nkv_c64_fit_args* a) {
     clear_error();
+    NKV_REQUIRE(a, NKV_ERR_INVALID, "null args");
+    const int B = a->B, HD = a->HD, C = a->C;
+    const int64_t S = a->S;
     NKV_REQUIRE(B >= 0 && S >= 0 && HD > 0, NKV_ERR_INVALID, "bad shape");
-    NKV_REQUIRE(iterations >= 0, NKV_ERR_INVALID, "iterations must be >= 0");
+    NKV_REQUIRE(a->iterations >= 0, NKV_ERR_INVALID, "iterations must be >= 0");
     if (B == 0 || S == 0) return NKV_OK;
     NKV_REQUIRE(C >= 1 && C <= S && C <= FIT_MAXC, NKV_ERR_INVALID,
                 "C64 clusters must be in [1, min(S, 256)]");
     NKV_REQUIRE(S < INT32_MAX, NKV_ERR_INVALID, "rows must fit in 32 bits");
-    NKV_REQUIRE(x && init_rows && centers && labels, NKV_ERR_INVALID, "null pointer");
+    NKV_REQUIRE((a->x || a->x_bf16) && (a->init_rows || a->init_rows_host) && a->centers && a->labels,
+                NKV_ERR_INVALID, "null pointer");
+    NKV_REQUIRE(!(a->x && a->x_bf16), NKV_ERR_INVALID, "give x or x_bf16, not both");
     const size_t need = nkv_c64_fit_workspace_size(B, S, C);
-    NKV_REQUIRE(workspace && workspace_bytes >= need, NKV_ERR_WORKSPACE,
+    NKV_REQUIRE(a->workspace && a->workspace_bytes >= need, NKV_ERR_WORKSPACE,
                 "workspace missing or smaller than nkv_c64_fit_workspace_size()");
-    unsigned char* ws = reinterpret_cast<unsigned char*>(workspace);
-    int32_t* counts = reinterpret_cast<int32_t*>(ws);
-    int32_t* offsets = reinterpret_cast<int32_t*>(ws + fit_ws_align((size_t)B * C * 4));
-    int32_t* order = reinterpret_cast<int32_t*>(ws + 2 * fit_ws_align((size_t)B * C * 4));
+    const bool xb = a->x_bf16 != nullptr;
+    const void* x = xb ? (const void*)a->x_bf16 : (const void*)a->x;
+    // the fp64 MFMA search: whole 32-wide steps, 16-byte rows
+    const bool mfma = HD % 32 == 0 && reinterpret_cast<uintptr_t>(x) % 16 == 0 &&
+                      reinterpret_cast<uintptr_t>(a->centers) % 16 == 0 && B <= 65535 &&
+                      reinterpret_cast<uintptr_t>(a->workspace) % 8 == 0;
+    const bool rounds = a->iterations > 0;
+    NKV_REQUIRE(!xb || (mfma && rounds), NKV_ERR_UNSUPPORTED,
+                "a bf16 fit needs HD % 32 == 0, 16-byte aligned rows and at least one round");
+    NKV_REQUIRE(rounds || !(a->centers_bf16 || a->ids_u8), NKV_ERR_UNSUPPORTED,
+                "bf16 centers and uint8 ids need at least one round");
+    unsigned char* ws = reinterpret_cast<unsigned char*>(a->workspace);
+    double* part_d = reinterpret_cast<double*>(ws);
+    int32_t* part_c = reinterpret_cast<int32_t*>(ws + fit_part_bytes(B, S, C, sizeof(double)));
+    FitInit init{};
+    init.dev = a->init_rows;
+    if (!init.dev) std::copy(a->init_rows_host, a->init_rows_host + C, init.v);
     hipStream_t s = (hipStream_t)stream;
-    const int64_t elems = (int64_t)B * C * HD;
-    c64_init_kernel<<<dim3((unsigned)std::min<int64_t>(cdiv(elems, 256), 4096)), 256, 0, s>>>(
-        x, B, S, HD, C, init_rows, centers);
-    NKV_LAUNCH_CHECK();
-    if (iterations == 0) {
+    if (!mfma || !rounds) {
+        const int64_t elems = (int64_t)B * C * HD;
+        c64_init_kernel<<<dim3((unsigned)std::min<int64_t>(cdiv(elems, 256), 4096)), 256, 0, s>>>(
+            a->x, B, S, HD, C, init, a->centers);
+        NKV_LAUNCH_CHECK();
+    }
+    if (!rounds) {
         // no round: the labels stay zero, as the reference initialises them
         zero_i32_kernel<<<dim3((unsigned)std::min<int64_t>(cdiv((int64_t)B * S, 256), 4096)), 256,
-                          0, s>>>(labels, (int64_t)B * S);
+                          0, s>>>(a->labels, (int64_t)B * S);
         NKV_LAUNCH_CHECK();
         return NKV_OK;
     }
-    for (int it = 0; it < iterations; ++it) {
-        for (int b = 0; b < B; ++b) {
-            int rc = launch_assign_f32(s, x + (int64_t)b * S * HD, centers + (int64_t)b * C * HD,
-                                       S, C, HD, labels + (int64_t)b * S);
-            if (rc) return rc;
+    const int64_t total = (int64_t)B * S;
+    const int ncb = (int)cdiv(C, FS_CENT);
+    for (int it = 0; it < a->iterations; ++it) {
+        const bool first = mfma && it == 0, last = it + 1 == a->iterations;
+        const double* pd = part_d;
+        const int32_t* pc = part_c;
+        int nc = ncb;
+        if (mfma) {
+            const dim3 grid((unsigned)cdiv(S, FS_ROWS), (unsigned)ncb, (unsigned)B);
+            auto run = [&](auto kernel) {
+                kernel<<<grid, 64 * FS_WAVES, 0, s>>>(x, a->centers, init, S, HD, C, part_d, part_c);
+            };
+            if (xb) first ? run(fit_search_kernel<true, true>) : run(fit_search_kernel<true, false>);
+            else first ? run(fit_search_kernel<false, true>) : run(fit_search_kernel<false, false>);
+            NKV_LAUNCH_CHECK();
+            if (ncb > 2) {
+                fit_label_kernel<<<dim3((unsigned)cdiv(total, 256)), 256, 0, s>>>(part_d, part_c, ncb,
+                                                                                  total, a->labels);
+                NKV_LAUNCH_CHECK();
+                pd = nullptr;
+                pc = a->labels;
+            }
+        } else {
+            for (int b = 0; b < B; ++b) {
+                const int rc = launch_assign_f32(s, a->x + b * S * HD, a->centers + (int64_t)b * C * HD,
+                                                 S, C, HD, part_c + b * S);
+                if (rc) return rc;
+            }
+            pd = nullptr;
         }
-        c64_sort_kernel<<<dim3((unsigned)B), FIT_THREADS, 0, s>>>(labels, S, C, counts, offsets,
-                                                                  order);
-        NKV_LAUNCH_CHECK();
-        c64_update_kernel<<<dim3((unsigned)cdiv(HD, 256), (unsigned)C, (unsigned)B), 256, 0, s>>>(
-            x, S, HD, C, counts, offsets, order, centers);
+        const dim3 grid((unsigned)cdiv(HD, 256), (unsigned)C, (unsigned)B);
+        auto run = [&](auto kernel) {
+            kernel<<<grid, 256, 0, s>>>(x, S, HD, C, pd, pc, nc, init, first ? 1 : 0,
+                                        a->centers, last ? a->centers_bf16 : nullptr,
+                                        pc == a->labels ? nullptr : a->labels,
+                                        last ? a->ids_u8 : nullptr);
+        };
+        if (xb) run(fit_update_kernel<true>);
+        else run(fit_update_kernel<false>);
         NKV_LAUNCH_CHECK();
     }
     return NKV_OK;
@@ -1978,7 +2260,7 @@ int encode_batch(hipStream_t s, const nkv_encode_args* a, int n) {
             NKV_LAUNCH_CHECK();
         }
     }
-    const dim3 qgrid((unsigned)cdiv(rows * (r / a->group), 256), (unsigned)n);
+    const dim3 qgrid((unsigned)cdiv(rows * (r / a->group) * quant_lanes(a->group), 256), (unsigned)n);
     if (a->quant_mode == NKV_QUANT_BF16)
         quant_pack_batch_kernel<NKV_QUANT_BF16><<<qgrid, 256, 0, s>>>(B, a->group, a->scale_dtype);
     else

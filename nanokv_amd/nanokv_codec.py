@@ -263,16 +263,30 @@ def semantic_residual_centers(value: torch.Tensor, layer: int) -> tuple[torch.Te
     MG35_KVCODEC_C64_ITERS rounds of nearest-center labels and mean updates.
     Returns (bf16 centers [B, C, HD], labels [B, S] int32 of the last round),
     the stored centers of store_centers (MG:69-90)."""
-    batch, sequence, dim = value.shape
+    return _fit_centers(value.detach(), layer)[:2]
+
+
+def _fit_centers(value: torch.Tensor, layer: int):
+    """semantic_residual_centers of value [B, S, HD] (any float dtype; bf16
+    rows are read in place), and its labels as uint8 ids."""
+    sequence = int(value.shape[1])
     clusters = int(os.environ.get("MG35_KVCODEC_C64_CLUSTERS", "64"))
     iterations = int(os.environ.get("MG35_KVCODEC_C64_ITERS", "2"))
     if clusters <= 0 or clusters > sequence or clusters > 256:
         raise ValueError(f"C64 clusters must be in [1,min(S,256)], got {clusters}")
     draw = torch.Generator(device="cpu").manual_seed(20260804 + int(layer))
     init = torch.randperm(sequence, generator=draw)[:clusters].to(torch.int32)
-    centers, labels = ops.c64_fit(value.detach().float().contiguous(),
-                                  init.to(value.device), iterations)
-    return centers.to(torch.bfloat16), labels
+    if iterations < 1:
+        centers, labels = ops.c64_fit(value.float().contiguous(), init.to(value.device), iterations)
+        return centers.to(torch.bfloat16), labels, labels.to(torch.uint8)
+    return ops.c64_fit_payload(value if _bf16_rows(value, 32) else value.float().contiguous(),
+                               init, iterations)
+
+
+def _bf16_rows(value: torch.Tensor, multiple: int) -> bool:
+    """Whether the kernels read value's rows [.., HD] as bf16 in place."""
+    return value.dtype == torch.bfloat16 and value.is_contiguous() and \
+        value.shape[-1] % multiple == 0 and value.data_ptr() % 16 == 0
 
 
 # ---------------------------------------------------------------- encode
@@ -300,46 +314,34 @@ def encode_tensor(kind: str, layer: int, value: torch.Tensor) -> dict:
     group = _scale_group(r)
     sdt = _scale_dtype()
     qmode = _quant_mode()
-    rows = value.detach().float().contiguous()
-    shared = _CENTERS.get((kind, int(layer)))
-    packed, scales, ids_out, tables = [], [], [], []
-    centers = ids_t = None
+    value = value.detach()
+    shared = _CENTERS.get((kind, int(layer))) if semantic else None
     id_dtype = torch.uint8
-    center_batch_shared = False
-    if not semantic:
-        # the pca rung: the rows themselves are projected (MG:338-342)
-        for b in range(batch):
-            e = ops.encode(rows[b], op["encoder"], mean=op["mean"], group=group,
-                           scale_dtype=sdt, quant_mode=qmode)
-            packed.append(e["packed"])
-            scales.append(e["scales"])
-    elif shared is not None:
+    centers = ids = given = None
+    if shared is not None:
         shared = shared.to(value.device)
         id_dtype = ops.id_dtype_for(int(shared.shape[0]))
-        for b in range(batch):
-            e = ops.encode(rows[b], op["encoder"], centers=shared, mean=op["mean"], group=group,
-                           scale_dtype=sdt, quant_mode=qmode, id_dtype=id_dtype)
-            packed.append(e["packed"])
-            scales.append(e["scales"])
-            ids_out.append(e["ids"])
         centers = shared[None]
-        center_batch_shared = True
-    else:
-        fitted, labels = semantic_residual_centers(value, layer)
-        id_dtype = torch.uint8
-        for b in range(batch):
-            # the fit's labels are kept (MG:326-330): the encoder subtracts each
-            # row's stored center without searching again
-            ids = labels[b].to(torch.uint8)
-            e = ops.encode(rows[b], op["encoder"], centers=fitted[b], mean=op["mean"],
-                           group=group, scale_dtype=sdt, quant_mode=qmode, ids=ids)
-            packed.append(e["packed"])
-            scales.append(e["scales"])
-            ids_out.append(ids)
-        centers = fitted
-        center_batch_shared = False
-    if ids_out:
-        ids_t = torch.stack(ids_out)
+        ids = torch.empty((batch, seq), device=value.device, dtype=id_dtype)
+    elif semantic:
+        # the fit's labels are kept (MG:326-330): the encoder subtracts each
+        # row's stored center without searching again
+        centers, _, ids = _fit_centers(value, layer)
+        given = ids
+    # bf16 rows are read in place (exact) where the kernels take them
+    bf16 = _bf16_rows(value, 256) and (shared is None or shared.shape[0] <= 256)
+    rows = value if bf16 else value.float().contiguous()
+    packed = torch.empty((batch, seq, r // 2), device=value.device, dtype=torch.uint8)
+    scales = torch.empty((batch, seq, r // group), device=value.device, dtype=sdt)
+    # (the pca rung has no centers: the rows themselves are projected, MG:338-342)
+    problems = [{"x": rows[b], "w_enc": op["encoder"], "mean": op["mean"],
+                 "centers": None if centers is None else shared if shared is not None else centers[b],
+                 "ids": None if given is None else given[b], "id_dtype": id_dtype,
+                 "out": {"packed": packed[b], "scales": scales[b],
+                         "ids": None if ids is None else ids[b]}}
+                for b in range(batch)]
+    for b in range(0, batch, 8):
+        ops.encode_batch(problems[b:b + 8], group=group, scale_dtype=sdt, quant_mode=qmode)
     return {
         "codec": CODEC,
         "kind": kind,
@@ -347,16 +349,16 @@ def encode_tensor(kind: str, layer: int, value: torch.Tensor) -> dict:
         "shape": (batch, seq, dim),
         "latent_shape": (batch, seq, r),
         "latent_numel": batch * seq * r,
-        "packed_codes": torch.stack(packed).reshape(-1),
-        "scale": torch.stack(scales),
+        "packed_codes": packed.view(-1),
+        "scale": scales,
         "centers": centers,
-        "ids": ids_t,
+        "ids": ids,
         "semantic": semantic,
         "source_dtype": str(value.dtype).replace("torch.", ""),
         "scale_group": group,
         "scale_dtype": "fp16" if sdt == torch.float16 else "bf16",
         "id_dtype": str(id_dtype).replace("torch.", ""),
-        "shared_centers": center_batch_shared,
+        "shared_centers": shared is not None,
     }
 
 

@@ -19,7 +19,7 @@ from . import _lib
 from ._lib import (NKV_DTYPE_BF16, NKV_DTYPE_FP16, NKV_QUANT_BF16, NKV_QUANT_FP32,
                    NKV_SCHEDULE_AUTO, NKV_SCHEDULE_KEY_CHUNKS, NKV_SCHEDULE_QUERY_TILES,
                    NkvAttendArgs, NkvCodec, NkvDecodeArgs, NkvEncodeArgs, NkvFastArgs,
-                   NkvCamera, NkvFinishArgs, NkvLiftCombineArgs, NkvReaderGroup,
+                   NkvCamera, NkvFinishArgs, NkvLiftCombineArgs, NkvReaderGroup, NkvC64FitArgs,
                    NkvReaderRowsArgs, NkvRope,
                    NkvSegment, check, lib)
 
@@ -550,6 +550,43 @@ def c64_fit(x: torch.Tensor, init_rows: torch.Tensor, iterations: int = 2,
                                            centers.data_ptr(), labels.data_ptr(),
                                            workspace.data_ptr(), need))
     return centers, labels
+
+
+def c64_fit_payload(x: torch.Tensor, init_rows: torch.Tensor, iterations: int):
+    """c64_fit of fp32 or bf16 rows x [B, S, HD] with the results as a payload
+    holds them (nkv_c64_fit_rows): (centers [B, C, HD] bf16, labels [B, S]
+    int32, ids [B, S] uint8).  init_rows: int32 [C] on the CPU (passed with the
+    launch) or on x's device.  At least one round."""
+    device = _require_gpu(x)
+    _contig(init_rows, torch.int32, "init_rows")
+    if x.dim() != 3 or x.dtype not in (torch.float32, torch.bfloat16) or not x.is_contiguous():
+        raise ValueError("x must be contiguous fp32 or bf16 [B, S, HD]")
+    B, S, HD = x.shape
+    C = init_rows.numel()
+    a = NkvC64FitArgs()
+    a.B, a.S, a.HD, a.C, a.iterations = B, S, HD, C, int(iterations)
+    if x.dtype == torch.bfloat16:
+        a.x_bf16 = x.data_ptr()
+    else:
+        a.x = x.data_ptr()
+    if init_rows.is_cuda:
+        _require_gpu(x, init_rows)
+        a.init_rows = init_rows.data_ptr()
+    else:
+        a.init_rows_host = init_rows.data_ptr()
+    need = int(lib().nkv_c64_fit_workspace_size(B, S, C))
+    # one allocation for the scratch: the fp32 centers, then the fit's workspace
+    cbytes = (4 * B * C * HD + 255) // 256 * 256
+    scratch = torch.empty(max(cbytes + need, 1), device=device, dtype=torch.uint8)
+    centers = torch.empty((B, C, HD), device=device, dtype=torch.bfloat16)
+    labels = torch.empty((B, S), device=device, dtype=torch.int32)
+    ids = torch.empty((B, S), device=device, dtype=torch.uint8)
+    base = scratch.data_ptr()
+    a.centers, a.centers_bf16 = base, centers.data_ptr()
+    a.labels, a.ids_u8 = labels.data_ptr(), ids.data_ptr()
+    a.workspace, a.workspace_bytes = base + cbytes, need
+    check("nkv_c64_fit_rows", lib().nkv_c64_fit_rows(_stream(device), byref(a)))
+    return centers, labels, ids
 
 
 def int8_pack(weight: torch.Tensor, group_size: int = 0) -> dict:
