@@ -64,7 +64,7 @@
 extern "C" {
 #endif
 
-#define NKV_ABI_VERSION 7
+#define NKV_ABI_VERSION 8
 
 enum nkv_status {
     NKV_OK = 0,
@@ -318,7 +318,16 @@ typedef struct nkv_encode_args {
      * and to search, at most 256 centers and HD <= 16384. */
     const uint16_t* x_bf16;
     int64_t x_stride;             /* elements between rows of x / x_bf16; 0 = HD */
+    /* scratch of nkv_encode_workspace_size() bytes, 16-byte aligned, or NULL:
+     * with it the search and the projection run as plain GEMMs over the chip
+     * (same results; in a batch the first problem's is used) */
+    void* workspace;
+    size_t workspace_bytes;
 } nkv_encode_args;
+
+/* Scratch bytes an encode of these n problems can use (bounded: at most a few
+ * thousand rows at a time); 0 if it uses none. */
+size_t nkv_encode_workspace_size(const nkv_encode_args* args, int n);
 
 int nkv_encode(void* stream, const nkv_encode_args* args);
 

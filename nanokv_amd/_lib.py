@@ -13,7 +13,7 @@ from pathlib import Path
 
 LIB_PATH = Path(__file__).resolve().parent / "libnanokv_hip.so"
 
-NKV_ABI_VERSION = 7
+NKV_ABI_VERSION = 8
 NKV_OK = 0
 NKV_ERR_INVALID = -1
 NKV_ERR_UNSUPPORTED = -2
@@ -35,7 +35,7 @@ EXPORTED = (
     "nkv_fast_attend_workspace_size", "nkv_fast_attend", "nkv_rope_apply", "nkv_int8_pack",
     "nkv_int8_dequant", "nkv_c64_fit_workspace_size", "nkv_c64_fit", "nkv_camera_apply",
     "nkv_attend_static", "nkv_lift_lse_combine", "nkv_finish", "nkv_reader_rows",
-    "nkv_decode_batch", "nkv_c64_fit_rows",
+    "nkv_decode_batch", "nkv_c64_fit_rows", "nkv_encode_workspace_size",
 )
 NKV_STATIC_SCRATCH_BYTES = 64 << 20
 
@@ -66,7 +66,8 @@ class NkvEncodeArgs(Structure):
         ("id_bytes", c_int), ("ids_in", c_int),
         ("x", c_void_p), ("centers", c_void_p), ("mean", c_void_p), ("w_enc", c_void_p),
         ("ids", c_void_p), ("coeff", c_void_p), ("packed", c_void_p), ("scales", c_void_p),
-        ("x_bf16", c_void_p), ("x_stride", c_int64),
+        ("x_bf16", c_void_p), ("x_stride", c_int64), ("workspace", c_void_p),
+        ("workspace_bytes", c_size_t),
     ]
 
 
@@ -214,6 +215,8 @@ def _declare(lib: ctypes.CDLL) -> None:
     lib.nkv_assign.restype = c_int
     lib.nkv_assign.argtypes = [c_void_p, c_void_p, c_void_p, c_int64, c_int, c_int, c_void_p,
                                c_int]
+    lib.nkv_encode_workspace_size.restype = c_size_t
+    lib.nkv_encode_workspace_size.argtypes = [POINTER(NkvEncodeArgs), c_int]
     lib.nkv_encode.restype = c_int
     lib.nkv_encode.argtypes = [c_void_p, POINTER(NkvEncodeArgs)]
     lib.nkv_encode_batch.restype = c_int

@@ -21,10 +21,11 @@ LIB_NAME = "libnanokv_hip.so"
 ARCH = "gfx950"
 
 # Sources and their extra flags.  The codec TU holds bit-exact restatements
-# (quantiser, decode epilogue), so fp contraction is off there.
+# (quantiser, decode epilogue), so fp contraction is off there; its MFMA
+# accumulators stay in VGPRs, where the search folds them every 128 k.
 SOURCES = {
     "nkv_abi.hip": [],
-    "nkv_codec.hip": ["-ffp-contract=off"],
+    "nkv_codec.hip": ["-ffp-contract=off", "-mllvm", "-amdgpu-mfma-vgpr-form=1"],
     # MFMA accumulators in VGPRs: the fused kernel's softmax/rescale VALU work
     # runs on them every tile, and its read-only decoder fragments fill AGPRs
     "nkv_attend.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"],

@@ -6,6 +6,8 @@
 // not be fused away.
 #include "nkv_common.h"
 
+#include <type_traits>
+
 namespace nkv {
 
 // ============================================================ quantiser
@@ -496,6 +498,44 @@ __device__ __forceinline__ void assign_small_init(AssignSmall& sm, int t) {
     for (int e = t; e < AB_ROWS * AB_MAXC / 32; e += 64 * AB_WAVES) (&sm.cand[0][0])[e] = 0u;
 }
 
+// ||c||^2 - 2 x.c of row gr in fp64 (exact products), by the whole wave: 8
+// consecutive values per lane and step, four steps' loads issued together,
+// summed in ascending k per lane, then over the lanes.
+template <bool XB>
+__device__ __forceinline__ double exact_distance(const EncProb& P, const uint16_t* cr, int64_t gr,
+                                                 int HD, int lane) {
+    double cc = 0.0, xc = 0.0;
+    for (int k = 8 * lane; k < HD; k += 4 * 512) {
+        u32x4 cw[4];
+        X8<XB> x8[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            if (k + 512 * u < HD) {
+                cw[u] = *reinterpret_cast<const u32x4*>(cr + k + 512 * u);
+                x8[u].load(P, gr, k + 512 * u);
+            }
+        }
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            if (k + 512 * u >= HD) break;
+            const uint32_t w4[4] = {cw[u].x, cw[u].y, cw[u].z, cw[u].w};
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                const uint32_t hb = (e & 1) ? (w4[e >> 1] & 0xffff0000u) : (w4[e >> 1] << 16);
+                const double cv = (double)__uint_as_float(hb);
+                cc = fma(cv, cv, cc);
+                xc = fma((double)x8[u][e], cv, xc);
+            }
+        }
+    }
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) {
+        cc += __shfl_xor(cc, off);
+        xc += __shfl_xor(xc, off);
+    }
+    return cc - 2.0 * xc;
+}
+
 // The decision after the products: tot (this lane's 16 dot products x.c,
 // rows 8(i/4) + 4hf + i%4 of the block, center col), cnf = ||c||^2, and
 // sm.xn complete.  Rows with one candidate are decided; the others compare
@@ -554,39 +594,7 @@ __device__ __forceinline__ void assign_finish(const EncBatch& B, const EncProb& 
                 while (bits) {
                     const int c = 32 * w + __builtin_ctz(bits);
                     bits &= bits - 1;
-                    const uint16_t* cr = P.centers + (int64_t)c * HD;
-                    double cc = 0.0, xc = 0.0;
-                    // 8 consecutive values per lane and step (HD % 256 == 0), four
-                    // steps' loads issued together, summed in ascending k
-                    for (int k = 8 * lane; k < HD; k += 4 * 512) {
-                        u32x4 cw[4];
-                        X8<XB> x8[4];
-#pragma unroll
-                        for (int u = 0; u < 4; ++u) {
-                            if (k + 512 * u < HD) {
-                                cw[u] = *reinterpret_cast<const u32x4*>(cr + k + 512 * u);
-                                x8[u].load(P, gr, k + 512 * u);
-                            }
-                        }
-#pragma unroll
-                        for (int u = 0; u < 4; ++u) {
-                            if (k + 512 * u >= HD) break;
-                            const uint32_t w4[4] = {cw[u].x, cw[u].y, cw[u].z, cw[u].w};
-#pragma unroll
-                            for (int e = 0; e < 8; ++e) {
-                                const uint32_t hb = (e & 1) ? (w4[e >> 1] & 0xffff0000u) : (w4[e >> 1] << 16);
-                                const double cv = (double)__uint_as_float(hb);
-                                cc = fma(cv, cv, cc);
-                                xc = fma((double)x8[u][e], cv, xc);
-                            }
-                        }
-                    }
-#pragma unroll
-                    for (int off = 1; off < 64; off <<= 1) {
-                        cc += __shfl_xor(cc, off);
-                        xc += __shfl_xor(xc, off);
-                    }
-                    const double d = cc - 2.0 * xc;
+                    const double d = exact_distance<XB>(P, P.centers + (int64_t)c * HD, gr, HD, lane);
                     if (best < 0 || d < bd) { bd = d; best = c; }  // ascending c: first index on ties
                 }
             }
@@ -814,6 +822,457 @@ __global__ void __launch_bounds__(64 * AB_WAVES) assign_dma_kernel(EncBatch B) {
     cn += __shfl_xor(cn, 32);
     __syncthreads();
     assign_finish<ID_BYTES, true>(B, P, sm, tot, (float)cn, col, row0);
+}
+
+// ============================================================ encode with a workspace
+// With a caller's workspace an encode runs as (split_rows_kernel for fp32
+// rows,) search_dots_kernel, decide_kernel, project_kernel: two plain bf16
+// GEMMs whose tiles need not hold a row's whole search or residual, so that
+// they can be cut to fill the chip, and one pass over the rows between them.
+// A 1,560-row K + V chunk of bf16 rows (256 centers, r = 384): 18 + 15 + 24 us,
+// the call 53.7 us, against 36 for assign_dma_kernel and 43 for
+// encode_proj_kernel (98 and 196 blocks, which each stream the whole center
+// table or a W_enc slice beside their rows; the call 76 us).  780 fp32 rows
+// against 1,024 centers: 5 + 27 + 15 + 19 us (64 us a call) against 528 for
+// assign_mfma_kernel (fp64) and 43 (571 us).  Bound by latency, not by a unit:
+// project_kernel takes 8 us with one stage and 0.67 us per 128-wide stage (0.4
+// of it LDS reads and writes at 128 B a cycle), search_dots_kernel 9 us with
+// one stage.  Measured and not kept: four buffers of 64-wide stages (the same),
+// eight (37 us: one block per CU), operand rows padded so that one k goes
+// through all L2 channels (the same).
+
+// GEMM core: acc += A[rows, K] B[cols, K]^T over stages [s0, s1) of KS k, up
+// to two plane pairs one after the other.  Stages go global -> LDS by 1 KB DMA
+// pieces into NBUF buffers, NBUF - 1 ahead, one barrier per stage.  A row of a
+// stage is KS / 8 chunks of 16 bytes, chunk c of row q at slot c ^ swz(q): the
+// 16 rows that one LDS cycle serves fall in 16 distinct slots.
+template <int WM_, int WN_, int WR_, int WC_, int KS_, int NBUF_>
+struct GemmTile {
+    static constexpr int WM = WM_, WN = WN_, WR = WR_, WC = WC_, KS = KS_, NBUF = NBUF_;
+    static constexpr int TM = 32 * WM * WR, TN = 32 * WN * WC, WAVES = WR * WC, THREADS = 64 * WAVES;
+    static constexpr int ROWB = 2 * KS, CPR = KS / 8, RPP = 1024 / ROWB;   // bytes, chunks; rows per piece
+    static constexpr int STAGE = (TM + TN) * ROWB, SMEM = NBUF * STAGE;
+    // pieces e = wave + WAVES i: A's first, then B's; the first NHI waves take one more
+    static constexpr int PA = TM / RPP, PIECES = (TM + TN) / RPP;
+    static constexpr int QLO = PIECES / WAVES, NHI = PIECES % WAVES, QMAX = QLO + (NHI ? 1 : 0);
+    static_assert(KS == 64 || KS == 128, "the swizzles below");
+    static_assert(SMEM <= 160 * 1024, "LDS budget");
+    static __device__ __forceinline__ int swz(int q) { return KS == 64 ? (q >> 1) & 7 : q & 15; }
+    // row (of A's TM rows, then B's TN) that this lane brings in piece e
+    static __device__ __forceinline__ int piece_row(int e) { return RPP * e + (threadIdx.x & 63) / CPR; }
+    static __device__ __forceinline__ uint32_t piece_off(int q, int row, int64_t ld) {
+        return (uint32_t)row * (uint32_t)(2 * ld) + 16 * (((threadIdx.x & 63) % CPR) ^ swz(q));
+    }
+};
+
+// The second accumulators of a search: the first restart every SEG k, sums of
+// squares of B's columns (of the first plane) beside them.
+template <class T>
+struct GemmTotals {
+    f32x16 tot[T::WM][T::WN];
+    float csq[T::WN], ctot[T::WN];
+};
+
+// spp stages of the operands' first planes, then of their second ones (a_plane
+// and b_plane values on, 0: the same plane again); a at the tile's first row, b
+// at the table, off this lane's byte offsets of its pieces.  SEG: see
+// GemmTotals (0: none, t unused).
+template <class T, int SEG>
+__device__ __forceinline__ void gemm_stages(const uint16_t* a, int64_t a_plane, const uint16_t* b,
+                                            int64_t b_plane, const uint32_t (&off)[T::QMAX], int s0,
+                                            int s1, int spp, unsigned char* smem,
+                                            f32x16 (&acc)[T::WM][T::WN], GemmTotals<T>& t, bool norms) {
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int hf = lane >> 5, l32 = lane & 31;
+    const int wr = wave / T::WC, wc = wave % T::WC;
+    auto issue = [&](int s) {
+        const int p = s >= spp ? 1 : 0;
+        const int64_t k = T::KS * (int64_t)(s - p * spp);
+        const unsigned char* ab = reinterpret_cast<const unsigned char*>(a + p * a_plane + k);
+        const unsigned char* bb = reinterpret_cast<const unsigned char*>(b + p * b_plane + k);
+        unsigned char* dst = smem + ((s - s0) % T::NBUF) * T::STAGE;
+#pragma unroll
+        for (int i = 0; i < T::QMAX; ++i) {
+            const int e = wave + T::WAVES * i;
+            if (i < T::QLO || wave < T::NHI)
+                dma16((e < T::PA ? ab + 0 : bb + 0) + off[i], dst + 1024 * e);
+        }
+    };
+#pragma unroll
+    for (int i = 0; i < T::NBUF - 1; ++i)
+        if (s0 + i < s1) issue(s0 + i);
+    for (int s = s0; s < s1; ++s) {
+        // stage s landed; the NBUF - 2 after it may still be in flight
+        if (s + T::NBUF - 2 >= s1) wait_vmcnt<0>();
+        else if (T::NHI > 0 && wave < T::NHI) wait_vmcnt<(T::NBUF - 2) * T::QMAX>();
+        else wait_vmcnt<(T::NBUF - 2) * T::QLO>();
+        lds_barrier();
+        if (s + T::NBUF - 1 < s1) issue(s + T::NBUF - 1);
+        const unsigned char* sb = smem + ((s - s0) % T::NBUF) * T::STAGE;
+#pragma unroll
+        for (int k16 = 0; k16 < T::KS / 16; ++k16) {
+            const int sw = 16 * ((2 * k16 + hf) ^ T::swz(l32));
+            bf16x8 af[T::WM], bf[T::WN];
+#pragma unroll
+            for (int i = 0; i < T::WM; ++i)
+                af[i] = lds_b128(reinterpret_cast<const uint16_t*>(
+                    sb + (32 * (T::WM * wr + i) + l32) * T::ROWB + sw));
+#pragma unroll
+            for (int j = 0; j < T::WN; ++j)
+                bf[j] = lds_b128(reinterpret_cast<const uint16_t*>(
+                    sb + (T::TM + 32 * (T::WN * wc + j) + l32) * T::ROWB + sw));
+#pragma unroll
+            for (int i = 0; i < T::WM; ++i)
+#pragma unroll
+                for (int j = 0; j < T::WN; ++j) acc[i][j] = mfma32(af[i], bf[j], acc[i][j]);
+            if constexpr (SEG > 0) {
+                if (norms && s < spp) {
+#pragma unroll
+                    for (int j = 0; j < T::WN; ++j) {
+                        const u32x4 v = __builtin_bit_cast(u32x4, bf[j]);
+                        const uint32_t w4[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) {
+                            const bf16x2 wv = __builtin_bit_cast(bf16x2, w4[e]);
+                            t.csq[j] = __builtin_amdgcn_fdot2_f32_bf16(wv, wv, t.csq[j], false);
+                        }
+                    }
+                }
+            }
+        }
+        if constexpr (SEG > 0) {
+            if ((s - s0 + 1) % (SEG / T::KS) == 0 || s + 1 == s1) {
+#pragma unroll
+                for (int j = 0; j < T::WN; ++j) {
+                    t.ctot[j] += t.csq[j];
+                    t.csq[j] = 0.0f;
+#pragma unroll
+                    for (int i = 0; i < T::WM; ++i) {
+#pragma unroll
+                        for (int e = 0; e < 16; ++e) t.tot[i][j][e] += acc[i][j][e];
+                        acc[i][j] = f32x16{};
+                    }
+                }
+            }
+        }
+    }
+}
+
+// One problem's slices of the workspace.
+struct EncWs {
+    const uint16_t* xh;      // the rows' high plane [M][ld]: bf16 rows in place, or split
+    const uint16_t* xl;      // low plane (fp32 rows), or NULL
+    int64_t ld;
+    float* dots;             // [splits][M][C rounded up to 4]
+    float* cnorm;            // [splits][C]
+    uint16_t* resid;         // [M][K]
+};
+struct EncWsBatch {
+    EncBatch e;
+    EncWs w[ENC_MAXB];
+    int64_t m0;              // first row of this pass
+    int rows;                // rows of the largest problem in this pass
+    int splits;
+};
+
+// hi = bf16(x), lo = bf16(x - hi) of fp32 rows.
+__global__ void __launch_bounds__(256) split_rows_kernel(EncWsBatch W) {
+    const EncProb& P = W.e.p[blockIdx.y];
+    const EncWs& w = W.w[blockIdx.y];
+    const int per = W.e.K / 8;
+    const int64_t n = (int64_t)min((int64_t)W.rows, P.M - W.m0) * per;
+    for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (int64_t)gridDim.x * 256) {
+        const int64_t m = i / per;
+        const int k = (int)(i - m * per) * 8;
+        X8<false> x;
+        x.load(P, W.m0 + m, k);
+        u32x4 hi, lo;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            hi[e] = pack_bf16x2(x[2 * e], x[2 * e + 1]);
+            lo[e] = pack_bf16x2(x[2 * e] - __uint_as_float(hi[e] << 16),
+                                x[2 * e + 1] - __uint_as_float(hi[e] & 0xffff0000u));
+        }
+        *reinterpret_cast<u32x4*>(const_cast<uint16_t*>(w.xh) + m * w.ld + k) = hi;
+        *reinterpret_cast<u32x4*>(const_cast<uint16_t*>(w.xl) + m * w.ld + k) = lo;
+    }
+}
+
+// Approximate dot products of the search: split blockIdx.y of K's stages, rows
+// and centers a 128 x 128 tile (32 x 64 per wave).  As in assign_bf16_kernel
+// the MFMA accumulator restarts, here every SD_SEG k, and the segment sums are
+// added in a second fp32 accumulator; the splits are added in fp64.  The
+// blocks of the first row tile also sum ||c||^2 of their stages.
+using DotsTile = GemmTile<1, 2, 4, 2, 64, 4>;
+constexpr int SD_SEG = 128;
+
+__global__ void __launch_bounds__(DotsTile::THREADS) search_dots_kernel(EncWsBatch W) {
+    using T = DotsTile;
+    extern __shared__ __align__(16) unsigned char smem_raw[];
+    const EncProb& P = W.e.p[blockIdx.z];
+    const EncWs& w = W.w[blockIdx.z];
+    const int C = W.e.num_centers, K = W.e.K, spp = K / 64;
+    const int nct = (C + T::TN - 1) / T::TN;
+    const int tm0 = (int)(blockIdx.x / (uint32_t)nct) * T::TM;
+    const int tn0 = (int)(blockIdx.x % (uint32_t)nct) * T::TN;
+    const int left = (int)min(P.M - W.m0 - tm0, (int64_t)T::TM);
+    if (left <= 0) return;
+    const int total = w.xl ? 2 * spp : spp;
+    const int s0 = (int)((uint32_t)total * blockIdx.y / (uint32_t)W.splits);
+    const int s1 = (int)((uint32_t)total * (blockIdx.y + 1) / (uint32_t)W.splits);
+    const uint16_t* xh = w.xh + tm0 * w.ld;
+    uint32_t off[T::QMAX];
+#pragma unroll
+    for (int i = 0; i < T::QMAX; ++i) {
+        const int e = (threadIdx.x >> 6) + T::WAVES * i, q = T::piece_row(e);
+        off[i] = e < T::PA ? T::piece_off(q, min(q, left - 1), w.ld)
+                           : T::piece_off(q, min(tn0 + q - T::TM, C - 1), K);
+    }
+    f32x16 acc[T::WM][T::WN] = {};
+    GemmTotals<T> t = {};
+    const bool norms = tm0 == 0;
+    gemm_stages<T, SD_SEG>(xh, w.xl ? w.xl - w.xh : 0, P.centers, 0, off, s0, s1, spp, smem_raw, acc, t,
+                           norms);
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int hf = lane >> 5, l32 = lane & 31;
+    const int wr = wave / T::WC, wc = wave % T::WC;
+    const int Cs = (C + 3) & ~3;   // whole 16-byte pieces per row
+    float* out = w.dots + (int64_t)blockIdx.y * W.rows * Cs;
+#pragma unroll
+    for (int j = 0; j < T::WN; ++j) {
+        const int n = tn0 + 32 * (T::WN * wc + j) + l32;
+        const float cn = t.ctot[j] + __shfl_xor(t.ctot[j], 32);
+        if (n >= C) continue;
+        if (norms && wr == 0 && hf == 0) w.cnorm[blockIdx.y * C + n] = cn;
+#pragma unroll
+        for (int i = 0; i < T::WM; ++i)
+#pragma unroll
+            for (int e = 0; e < 16; ++e) {
+                const int m = 32 * (T::WM * wr + i) + 8 * (e / 4) + 4 * hf + (e % 4);
+                if (m < left) out[(int64_t)(tm0 + m) * Cs + n] = t.tot[i][j][e];
+            }
+    }
+}
+
+// One wave per row: the search's decision (as assign_finish: U = min dt + E,
+// candidates dt - E <= U, several compared exactly in fp64) and the bf16
+// residual x - center - mean the projection reads.
+// The bound: each segment's sum is within g_SEG of sum |x||c| of its k, the
+// segment sums within g_n of theirs (n <= 96 segments per split), g_n = n 2^-24
+// / (1 - n 2^-24); hi + lo misses 2^-16 |x|: (g_128 + g_96)(1 + 2^-7) + 2^-16
+// < 2.9e-5 of ||x|| ||c|| per dot product, twice the rounding part if the
+// matrix core truncated (4.3e-5).  ||c||^2 is summed the same way (< 1.4e-5
+// ||c||^2).  The distance ||c||^2 - 2 x.c is then within 8.6e-5 ||x|| ||c|| +
+// 2.8e-5 ||c||^2 of the exact one; E_c takes 1.2e-4 of both.
+constexpr float SD_KAPPA = 1.2e-4f;
+constexpr int SD_MAXC = 1024, SD_MAXK = 96 * SD_SEG / 2;
+
+constexpr int DK_FLY = 6;   // 512-wide steps of a row in flight: 3,072 values
+
+template <int ID_BYTES, bool XB, bool SEARCH>
+__global__ void __launch_bounds__(256) decide_kernel(EncWsBatch W) {
+    __shared__ float cns[SEARCH ? SD_MAXC : 1];
+    const EncProb& P = W.e.p[blockIdx.y];
+    const EncWs& w = W.w[blockIdx.y];
+    const int t = threadIdx.x, lane = t & 63;
+    const int C = W.e.num_centers, HD = W.e.K;
+    const int64_t m = (int64_t)blockIdx.x * 4 + (t >> 6), gr = W.m0 + m;
+    const bool row_ok = m < W.rows && gr < P.M;
+    const int64_t cr_row = row_ok ? gr : 0;
+    int id = 0;
+    if constexpr (SEARCH) {
+        for (int c = t; c < C; c += 256) {
+            double cn = 0.0;
+            for (int k = 0; k < W.splits; ++k) cn += (double)w.cnorm[k * C + c];
+            cns[c] = (float)cn;
+        }
+        __syncthreads();
+    }
+    if (!row_ok) return;
+    if constexpr (SEARCH) {
+        constexpr int NQ = SD_MAXC / 256;
+        // this lane's centers: 256 q + 4 lane + [0, 4); the splits' sums in fp64
+        const int Cs = (C + 3) & ~3;
+        const float* d = w.dots + m * Cs + 4 * lane;
+        double dot[NQ][4] = {};
+        for (int k = 0; k < W.splits; k += 2) {
+            f32x4 v[2][NQ];
+#pragma unroll
+            for (int u = 0; u < 2; ++u)
+#pragma unroll
+                for (int q = 0; q < NQ; ++q) {
+                    v[u][q] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+                    if (256 * q + 4 * lane < C && k + u < W.splits)
+                        v[u][q] = *reinterpret_cast<const f32x4*>(d + (int64_t)(k + u) * W.rows * Cs + 256 * q);
+                }
+#pragma unroll
+            for (int q = 0; q < NQ; ++q)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) dot[q][e] += (double)v[0][q][e] + (double)v[1][q][e];
+        }
+        float xsq = 0.0f;
+        for (int k0 = 8 * lane; k0 < HD; k0 += 512 * DK_FLY) {
+            X8<XB> x[DK_FLY];
+#pragma unroll
+            for (int u = 0; u < DK_FLY; ++u)
+                if (k0 + 512 * u < HD) x[u].load(P, cr_row, k0 + 512 * u);
+#pragma unroll
+            for (int u = 0; u < DK_FLY; ++u) {
+                if (k0 + 512 * u >= HD) break;
+#pragma unroll
+                for (int e = 0; e < 8; ++e) xsq = fmaf(x[u][e], x[u][e], xsq);
+            }
+        }
+#pragma unroll
+        for (int off = 1; off < 64; off <<= 1) xsq += __shfl_xor(xsq, off);
+        const float xn = sqrtf(xsq) * 1.001f;
+        float low[NQ][4];
+        float U = INFINITY;
+#pragma unroll
+        for (int q = 0; q < NQ; ++q)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                low[q][e] = INFINITY;
+                const int c = 256 * q + 4 * lane + e;
+                if (c < C) {
+                    const float cf = cns[c], dt = (float)((double)cf - 2.0 * dot[q][e]);
+                    const float E = SD_KAPPA * (xn * sqrtf(cf) * 1.001f + cf * 1.001f);
+                    low[q][e] = dt - E;
+                    U = fminf(U, dt + E);
+                }
+            }
+#pragma unroll
+        for (int off = 1; off < 64; off <<= 1) U = fminf(U, __shfl_xor(U, off));
+        int cnt = 0, first = 0;
+#pragma unroll
+        for (int q = 0; q < NQ; ++q)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const uint64_t bits = __ballot(256 * q + 4 * lane + e < C && low[q][e] <= U);
+                if (bits) first = 256 * q + 4 * (__ffsll((unsigned long long)bits) - 1) + e;
+                cnt += __popcll(bits);
+            }
+        // (no candidate only for non-finite rows: index 0 then)
+        id = cnt == 0 ? 0 : first;
+        if (cnt > 1) {
+            double bd = 0.0;
+            int best = -1;
+#pragma unroll
+            for (int q = 0; q < NQ; ++q)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    uint64_t bits = __ballot(256 * q + 4 * lane + e < C && low[q][e] <= U);
+                    while (bits) {
+                        const int c = 256 * q + 4 * (__ffsll((unsigned long long)bits) - 1) + e;
+                        bits &= bits - 1;
+                        const double dd = exact_distance<XB>(P, P.centers + (int64_t)c * HD, gr, HD, lane);
+                        if (better(dd, c, bd, best)) { bd = dd; best = c; }
+                    }
+                }
+            id = best;
+        }
+        if (lane == 0) store_id<ID_BYTES>(P.ids, gr, id);
+    } else if (P.centers) {
+        id = W.e.id_of(P, gr);
+    }
+    const uint16_t* cr = P.centers ? P.centers + (int64_t)id * HD : nullptr;
+    for (int k0 = 8 * lane; k0 < HD; k0 += 512 * DK_FLY) {
+        X8<XB> x[DK_FLY];
+        u32x4 c[DK_FLY];
+        f32x4 mn[DK_FLY][2];
+#pragma unroll
+        for (int u = 0; u < DK_FLY; ++u) {
+            const int k = k0 + 512 * u;
+            c[u] = u32x4{0, 0, 0, 0};
+            mn[u][0] = mn[u][1] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+            if (k >= HD) continue;
+            x[u].load(P, gr, k);
+            if (cr) c[u] = *reinterpret_cast<const u32x4*>(cr + k);
+            if (P.mean) {
+                __builtin_memcpy(&mn[u][0], P.mean + k, 16);
+                __builtin_memcpy(&mn[u][1], P.mean + k + 4, 16);
+            }
+        }
+#pragma unroll
+        for (int u = 0; u < DK_FLY; ++u) {
+            if (k0 + 512 * u >= HD) break;
+            float v[8];
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                const uint32_t cw = (e & 1) ? (c[u][e >> 1] & 0xffff0000u) : (c[u][e >> 1] << 16);
+                // (x - 0 = x: absent centers or mean change nothing)
+                v[e] = (x[u][e] - __uint_as_float(cw)) - mn[u][e >> 2][e & 3];
+            }
+            u32x4 o;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) o[e] = pack_bf16x2(v[2 * e], v[2 * e + 1]);
+            *reinterpret_cast<u32x4*>(w.resid + m * HD + k0 + 512 * u) = o;
+        }
+    }
+}
+
+// coeff = residual W_enc^T: one 32 x 32 accumulator per wave over the whole K
+// in ascending steps of 16 (the bits of encode_proj_kernel), 64 rows x 64, 96
+// or 128 columns per block.  Items (problem, row tile, column tile), column
+// fastest, in one run per XCD: the column tiles of a row tile share its
+// residual rows in one L2, W_enc (2.4 MB at r = 384) stays there.  Groups that
+// divide the tile's columns are quantised here.
+using Proj64 = GemmTile<1, 1, 2, 2, 128, 3>;
+using Proj96 = GemmTile<1, 1, 2, 3, 128, 3>;
+using Proj128 = GemmTile<1, 1, 2, 4, 64, 3>;
+
+template <class T>
+__global__ void __launch_bounds__(T::THREADS) project_kernel(EncWsBatch W) {
+    extern __shared__ __align__(16) unsigned char smem_raw[];
+    const int r = W.e.r, K = W.e.K;
+    const uint32_t nct = (uint32_t)(r + T::TN - 1) / T::TN, nrt = (uint32_t)(W.rows + T::TM - 1) / T::TM;
+    const uint32_t items = W.e.n * nrt * nct;
+    const uint32_t item = (blockIdx.x & 7) * ((items + 7) >> 3) + (blockIdx.x >> 3);
+    if (item >= items) return;
+    const uint32_t rest = item / nct, prob = rest / nrt;
+    const EncProb& P = W.e.p[prob];
+    const EncWs& w = W.w[prob];
+    const int tm0 = (int)(rest - prob * nrt) * T::TM, tn0 = (int)(item - rest * nct) * T::TN;
+    const int left = (int)min(P.M - W.m0 - tm0, (int64_t)T::TM);
+    if (left <= 0) return;
+    const uint16_t* rs = w.resid + (int64_t)tm0 * K;
+    uint32_t off[T::QMAX];
+#pragma unroll
+    for (int i = 0; i < T::QMAX; ++i) {
+        const int e = (threadIdx.x >> 6) + T::WAVES * i, q = T::piece_row(e);
+        off[i] = e < T::PA ? T::piece_off(q, min(q, left - 1), K)
+                           : T::piece_off(q, min(tn0 + q - T::TM, r - 1), K);
+    }
+    f32x16 acc[1][1] = {};
+    GemmTotals<T> none;
+    gemm_stages<T, 0>(rs, 0, P.w_enc, 0, off, 0, K / T::KS, K / T::KS, smem_raw, acc, none, false);
+    const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+    const int hf = lane >> 5, l32 = lane & 31;
+    const int n = tn0 + 32 * (wave % T::WC) + l32;
+    const int64_t m0 = W.m0 + tm0;
+    if (n < r) {
+#pragma unroll
+        for (int e = 0; e < 16; ++e) {
+            const int m = 32 * (wave / T::WC) + 8 * (e / 4) + 4 * hf + (e % 4);
+            if (m < left) P.coeff[(m0 + m) * r + n] = acc[0][0][e];
+        }
+    }
+    if (W.e.qgroup == 0) return;
+    // the coefficients just stored, read back after the barrier
+    __syncthreads();
+    const int G = W.e.qgroup, ngroups = r / G, gpb = min(r - tn0, T::TN) / G, lpg = quant_lanes(G);
+    for (int it0 = 0; it0 < T::TM * gpb; it0 += T::THREADS / lpg) {
+        const int it = it0 + t / lpg;
+        const bool in = it < T::TM * gpb && it / gpb < left;
+        const int64_t gid = in ? (m0 + it / gpb) * ngroups + tn0 / G + it % gpb : P.M * ngroups;
+        if (W.e.quant_mode == NKV_QUANT_BF16)
+            quant_pack_group<NKV_QUANT_BF16>(P.coeff, P.M, r, G, W.e.scale_dtype, P.packed, P.scales, gid,
+                                             t % lpg, lpg);
+        else
+            quant_pack_group<NKV_QUANT_FP32>(P.coeff, P.M, r, G, W.e.scale_dtype, P.packed, P.scales, gid,
+                                             t % lpg, lpg);
+    }
 }
 
 // ============================================================ MFMA GEMM core
@@ -1678,7 +2137,7 @@ struct Row8 {
 // (wave w: the 32-wide steps w, w + 8, ..); the partial sums meet in LDS and
 // are added in wave order.  At C = 64 a chunk of 1,560 rows is 196 blocks of
 // eight waves: one wave per 16 rows x 64 centers (the whole HD each, 98 waves
-// with work) took 132 us per round, this 11 us.  In a step lane l holds
+// with work) took 132 us per round, this 22 us.  In a step lane l holds
 // row / center l % 16, k 8 (l / 16) .. +8: whole 128-byte lines per row, and
 // any order of k is valid for the products.  Bound by the fp64 matrix rate
 // (0.61 GFLOP per round of 64 centers, 32 flop per cycle and SIMD).
@@ -1802,7 +2261,7 @@ __global__ void __launch_bounds__(256) fit_label_kernel(const double* __restrict
 // ballot per 64 and the counts of the (round, wave) pairs before it (a
 // separate stable counting sort by one block took 27 us per round).  Each
 // thread then sums its column in that order in fp64, FU_FLY loads in flight
-// (22-32 us one at a time, now 6 us with the scan: 1,560 rows, 64 clusters;
+// (22-32 us one at a time, now 11.4 us with the scan: 1,560 rows, 64 clusters;
 // bound by the latency of the largest cluster's row list).
 // FIRST: an empty cluster's center is its initial row (else it stays).
 // The blocks of the first columns write their rows' labels (null: they are
@@ -1820,10 +2279,12 @@ __global__ void __launch_bounds__(256) fit_update_kernel(
     const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
     const int d = blockIdx.x * 256 + t, c = blockIdx.y;
     const int64_t b = blockIdx.z, total = (int64_t)gridDim.z * S;
-    auto at = [&](int64_t row) -> double {
-        const int64_t i = (b * S + row) * HD + d;
-        if constexpr (XB) return (double)bf16_bits_to_f32(ldg(reinterpret_cast<const uint16_t*>(x) + i));
-        else return (double)ldg(reinterpret_cast<const float*>(x) + i);
+    using Raw = typename std::conditional<XB, uint16_t, float>::type;
+    const Raw* col = reinterpret_cast<const Raw*>(x) + b * S * HD + d;
+    auto at = [&](int64_t row) -> Raw { return ldg(col + row * HD); };
+    auto val = [](Raw v) -> float {
+        if constexpr (XB) return bf16_bits_to_f32(v);
+        else return v;
     };
     double sum = 0.0;
     int64_t n = 0;
@@ -1859,19 +2320,21 @@ __global__ void __launch_bounds__(256) fit_update_kernel(
         if (d < HD) {
             int k = 0;
             for (; k + FU_FLY <= run; k += FU_FLY) {
-                double v[FU_FLY];
+                Raw v[FU_FLY];
 #pragma unroll
                 for (int u = 0; u < FU_FLY; ++u) v[u] = at(list[k + u]);
 #pragma unroll
-                for (int u = 0; u < FU_FLY; ++u) sum += v[u];
+                for (int u = 0; u < FU_FLY; ++u) sum += (double)val(v[u]);
             }
-            for (; k < run; k += 4) {
-                double v[4];
+            // the rest (fewer than FU_FLY rows) in one flight too; repeats of
+            // the last row are not added
+            if (k < run) {
+                Raw v[FU_FLY];
 #pragma unroll
-                for (int u = 0; u < 4; ++u) v[u] = at(list[min(k + u, run - 1)]);
+                for (int u = 0; u < FU_FLY; ++u) v[u] = at(list[min(k + u, run - 1)]);
 #pragma unroll
-                for (int u = 0; u < 4; ++u)
-                    if (k + u < run) sum += v[u];
+                for (int u = 0; u < FU_FLY; ++u)
+                    if (k + u < run) sum += (double)val(v[u]);
             }
         }
         n += run;
@@ -1881,7 +2344,7 @@ __global__ void __launch_bounds__(256) fit_update_kernel(
     const int64_t o = (b * C + c) * HD + d;
     float v;
     if (n > 0) v = __fdiv_rn((float)sum, (float)n);
-    else if (first) v = (float)at(init.row(c, S));
+    else if (first) v = val(at(init.row(c, S)));
     else v = centers[o];
     centers[o] = v;
     if (centers_bf16) centers_bf16[o] = f32_to_bf16_bits(v);
@@ -2168,6 +2631,133 @@ int check_encode(const nkv_encode_args* a, const nkv_encode_args* first) {
     return NKV_OK;
 }
 
+// How an encode with a workspace runs: rows per pass (0: not at all) and
+// problem, splits of the search, workspace bytes.
+struct EncPlan {
+    int64_t pass;
+    int splits, cols;        // columns of a projection tile
+    size_t dots, cnorm, planes, resid, bytes;   // per problem, bytes in all
+};
+
+// At most ENC_PASS rows of all problems in one pass, so that the workspace
+// does not grow with the input; 4,096 rows are 32 row tiles of the search and
+// 64 x 6 tiles of the projection at r = 384: more fill the chip no better.
+constexpr int64_t ENC_PASS = 4096;
+
+EncPlan enc_plan(const nkv_encode_args* a, int n) {
+    EncPlan p{};
+    const bool search = a->centers && !a->ids_in;
+    int64_t rows = 0;
+    for (int i = 0; i < n; ++i) rows = std::max(rows, a[i].rows);
+    // whole stages; a decision keeps its row's centers in registers,
+    // its bound holds to SD_MAXK; byte offsets of rows in 32 bits
+    if (rows == 0 || a->HD % 128 || (search && (a->num_centers > SD_MAXC || a->HD > SD_MAXK))) return p;
+    if ((int64_t)std::max(a->r, search ? a->num_centers : 0) * a->HD * 2 > UINT32_MAX) return p;
+    for (int i = 0; i < n; ++i)
+        if (a[i].x_stride > (1 << 20)) return p;
+    p.pass = std::min(rows, std::max<int64_t>(ENC_PASS / n / DotsTile::TM, 1) * DotsTile::TM);
+    auto up = [](size_t b) { return (b + 255) / 256 * 256; };
+    p.resid = up((size_t)p.pass * a->HD * 2);
+    // the narrowest tile whose blocks run in one round of the 256 CUs (one
+    // block each: three stages of 128 k take 96 or 120 KB of LDS), else the
+    // widest (72 KB, two blocks per CU)
+    const int64_t row_tiles = n * cdiv(p.pass, Proj64::TM);
+    p.cols = row_tiles * cdiv(a->r, 64) <= 256 ? 64 : row_tiles * cdiv(a->r, 96) <= 256 ? 96 : 128;
+    if (search) {
+        const int64_t tiles = n * cdiv(p.pass, DotsTile::TM) * cdiv(a->num_centers, DotsTile::TN);
+        const int stages = (a->x_bf16 ? 1 : 2) * (a->HD / 64);
+        // one block per CU (128 KB of LDS): splits up to a full chip, of at
+        // least eight stages each
+        p.splits = (int)std::max<int64_t>(1, std::min<int64_t>({256 / tiles, stages / 8, 16}));
+        p.dots = up((size_t)p.splits * p.pass * ((a->num_centers + 3) & ~3) * 4);
+        p.cnorm = up((size_t)p.splits * a->num_centers * 4);
+        if (!a->x_bf16) p.planes = 2 * up((size_t)p.pass * a->HD * 2);
+    }
+    p.bytes = n * (p.resid + p.dots + p.cnorm + p.planes);
+    return p;
+}
+
+int encode_staged(hipStream_t s, const EncBatch& B, bool xb, bool search, const nkv_encode_args* a,
+                  const EncPlan& pl) {
+    static const hipError_t attr = [] {
+        const std::pair<const void*, int> k[] = {{(const void*)search_dots_kernel, DotsTile::SMEM},
+                                                 {(const void*)project_kernel<Proj64>, Proj64::SMEM},
+                                                 {(const void*)project_kernel<Proj96>, Proj96::SMEM},
+                                                 {(const void*)project_kernel<Proj128>, Proj128::SMEM}};
+        hipError_t e = hipSuccess;
+        for (const auto& f : k)
+            if (e == hipSuccess)
+                e = hipFuncSetAttribute(f.first, hipFuncAttributeMaxDynamicSharedMemorySize, f.second);
+        return e;
+    }();
+    NKV_REQUIRE(attr == hipSuccess, NKV_ERR_HIP, "hipFuncSetAttribute failed for the encode kernels");
+    EncWsBatch W{};
+    W.e = B;
+    W.splits = pl.splits;
+    const int n = B.n;
+    int64_t rows = 0;
+    unsigned char* ws = reinterpret_cast<unsigned char*>(a->workspace);
+    for (int i = 0; i < n; ++i) {
+        rows = std::max(rows, B.p[i].M);
+        EncWs& w = W.w[i];
+        auto take = [&](size_t b) { unsigned char* p = ws; ws += b; return p; };
+        w.resid = reinterpret_cast<uint16_t*>(take(pl.resid));
+        w.dots = reinterpret_cast<float*>(take(pl.dots));
+        w.cnorm = reinterpret_cast<float*>(take(pl.cnorm));
+        unsigned char* planes = take(pl.planes);
+        w.ld = xb ? B.p[i].ldx : B.K;
+        w.xh = reinterpret_cast<const uint16_t*>(planes);
+        w.xl = xb ? nullptr : reinterpret_cast<const uint16_t*>(planes + pl.planes / 2);
+    }
+    W.e.scale_dtype = a->scale_dtype;
+    W.e.quant_mode = a->quant_mode;
+    for (int64_t m0 = 0; m0 < rows; m0 += pl.pass) {
+        W.m0 = m0;
+        W.rows = (int)std::min(pl.pass, rows - m0);
+        if (xb)
+            for (int i = 0; i < n; ++i) W.w[i].xh = B.p[i].xb + m0 * B.p[i].ldx;
+        if (search) {
+            if (!xb) {
+                const int64_t units = (int64_t)W.rows * (B.K / 8);
+                split_rows_kernel<<<dim3((unsigned)std::min<int64_t>(cdiv(units, 256), 4096), n), 256, 0, s>>>(W);
+                NKV_LAUNCH_CHECK();
+            }
+            const unsigned tiles = (unsigned)(cdiv(W.rows, DotsTile::TM) * cdiv(B.num_centers, DotsTile::TN));
+            search_dots_kernel<<<dim3(tiles, pl.splits, n), DotsTile::THREADS, DotsTile::SMEM, s>>>(W);
+            NKV_LAUNCH_CHECK();
+        }
+        const dim3 dgrid((unsigned)cdiv(W.rows, 4), n);
+        auto decide = [&](auto k) { k<<<dgrid, 256, 0, s>>>(W); };
+        if (!search) {
+            xb ? decide(decide_kernel<1, true, false>) : decide(decide_kernel<1, false, false>);
+        } else if (B.id_bytes == 1) {
+            xb ? decide(decide_kernel<1, true, true>) : decide(decide_kernel<1, false, true>);
+        } else if (B.id_bytes == 2) {
+            xb ? decide(decide_kernel<2, true, true>) : decide(decide_kernel<2, false, true>);
+        } else {
+            xb ? decide(decide_kernel<4, true, true>) : decide(decide_kernel<4, false, true>);
+        }
+        NKV_LAUNCH_CHECK();
+        auto project = [&](auto tile, auto kernel) {
+            using T = decltype(tile);
+            W.e.qgroup = T::TN % a->group == 0 ? a->group : 0;
+            kernel<<<xcd_grid(n * cdiv(W.rows, T::TM) * cdiv(B.r, T::TN)), T::THREADS, T::SMEM, s>>>(W);
+        };
+        if (pl.cols == 64) project(Proj64{}, project_kernel<Proj64>);
+        else if (pl.cols == 96) project(Proj96{}, project_kernel<Proj96>);
+        else project(Proj128{}, project_kernel<Proj128>);
+        NKV_LAUNCH_CHECK();
+    }
+    if (W.e.qgroup) return NKV_OK;
+    const dim3 qgrid((unsigned)cdiv(rows * (B.r / a->group) * quant_lanes(a->group), 256), (unsigned)n);
+    if (a->quant_mode == NKV_QUANT_BF16)
+        quant_pack_batch_kernel<NKV_QUANT_BF16><<<qgrid, 256, 0, s>>>(B, a->group, a->scale_dtype);
+    else
+        quant_pack_batch_kernel<NKV_QUANT_FP32><<<qgrid, 256, 0, s>>>(B, a->group, a->scale_dtype);
+    NKV_LAUNCH_CHECK();
+    return NKV_OK;
+}
+
 int encode_batch(hipStream_t s, const nkv_encode_args* a, int n) {
     NKV_REQUIRE(a && n >= 1 && n <= ENC_MAXB, NKV_ERR_INVALID, "1..8 encode problems");
     for (int i = 0; i < n; ++i) {
@@ -2213,6 +2803,17 @@ int encode_batch(hipStream_t s, const nkv_encode_args* a, int n) {
     NKV_REQUIRE(!xb || (aligned && fast_proj && (!search || fast_search)), NKV_ERR_UNSUPPORTED,
                 "a bf16 input needs HD % 256 == 0, 16-byte aligned rows and, to search, at most 256 "
                 "centers and HD <= 16384");
+    // (a strided fp32 input needs the 16-byte kernels; see the launches below)
+    const bool strided_ok = aligned && fast_proj && (!search || fast_search);
+    bool packed_rows = true, w16 = reinterpret_cast<uintptr_t>(a->workspace) % 16 == 0;
+    for (int i = 0; i < n; ++i) {
+        packed_rows = packed_rows && B.p[i].ldx == HD;
+        w16 = w16 && reinterpret_cast<uintptr_t>(B.p[i].w_enc) % 16 == 0;
+    }
+    if (a->workspace && aligned && w16 && (packed_rows || strided_ok)) {
+        const EncPlan pl = enc_plan(a, n);
+        if (pl.pass > 0 && a->workspace_bytes >= pl.bytes) return encode_staged(s, B, xb, search, a, pl);
+    }
     int rc = NKV_OK;
     if (search) {
         if (fast_search && aligned) {
@@ -2270,6 +2871,14 @@ int encode_batch(hipStream_t s, const nkv_encode_args* a, int n) {
 }
 
 }  // namespace
+
+extern "C" size_t nkv_encode_workspace_size(const nkv_encode_args* a, int n) {
+    clear_error();
+    if (!a || n < 1 || n > ENC_MAXB) return 0;
+    for (int i = 0; i < n; ++i)
+        if (check_encode(a + i, a)) return 0;
+    return enc_plan(a, n).bytes;
+}
 
 extern "C" int nkv_encode(void* stream, const nkv_encode_args* a) {
     clear_error();

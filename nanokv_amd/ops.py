@@ -204,6 +204,18 @@ def _encode_args(x: torch.Tensor, w_enc: torch.Tensor, centers, mean, group, sca
     return args, {"packed": packed, "scales": scales, "ids": ids, "coeff": coeff}, device
 
 
+def _encode_scratch(first: NkvEncodeArgs, n: int, device: torch.device):
+    """Points the first problem of an encode at its scratch, which the caller
+    keeps over the launch (the caching allocator orders its reuse behind the
+    launch's stream)."""
+    need = lib().nkv_encode_workspace_size(byref(first), n)
+    if not need:
+        return None
+    scratch = torch.empty(need, device=device, dtype=torch.uint8)
+    first.workspace, first.workspace_bytes = scratch.data_ptr(), need
+    return scratch
+
+
 def encode(x: torch.Tensor, w_enc: torch.Tensor, *, centers: Optional[torch.Tensor] = None,
            mean: Optional[torch.Tensor] = None, group: int = 32,
            scale_dtype: torch.dtype = torch.bfloat16, quant_mode: str = "fp32",
@@ -220,7 +232,9 @@ def encode(x: torch.Tensor, w_enc: torch.Tensor, *, centers: Optional[torch.Tens
     labels of a C64 fit; returned as the payload's ids."""
     args, res, device = _encode_args(x, w_enc, centers, mean, group, scale_dtype, quant_mode,
                                      id_dtype, out, ids)
+    scratch = _encode_scratch(args, 1, device)
     check("nkv_encode", lib().nkv_encode(_stream(device), byref(args)))
+    del scratch
     return res
 
 
@@ -237,7 +251,9 @@ def encode_batch(problems: list, *, group: int = 32, scale_dtype: torch.dtype = 
              for p in problems]
     arr = (NkvEncodeArgs * len(built))(*(b[0] for b in built))
     device = built[0][2]
+    scratch = _encode_scratch(arr[0], len(built), device)
     check("nkv_encode_batch", lib().nkv_encode_batch(_stream(device), arr, len(built)))
+    del scratch
     return [b[1] for b in built]
 
 
