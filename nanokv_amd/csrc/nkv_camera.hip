@@ -1,8 +1,8 @@
 // nkv_camera.hip -- camera PRoPE transform of bf16 rows (nkv_camera_apply) and
 // the validation of nkv_camera shared with nkv_attend.
 //
-// One thread per (b, s, h, 4-vector): load its four dims, multiply by the
-// sub-frame matrix of the row's frame (nkv_camera.h), store.
+// Each 4-vector of a row is multiplied by the sub-frame matrix of the row's
+// frame (nkv_camera.h).
 #include "nkv_camera.h"
 
 #include "nkv_internal.h"
@@ -78,6 +78,106 @@ __global__ void __launch_bounds__(256) camera_apply_kernel(CameraApplyParams p) 
     }
 }
 
+// 16-byte pieces: one thread transforms piece `part` (8 dims, two 4-vectors)
+// of one (b, s) in CA_HEADS heads: the frame's matrices are fetched and rounded
+// once for them, their loads are in flight together.  The products are exact in
+// fp64, so the fused multiply-adds round as camera_vec4's sums do.
+// INTER: the vectors are the even and the odd dims, one sub-frame (FULL at
+// D = 128); else dims 0..3 and 4..7, each with its own sub-frame or (< 0) left
+// alone (FULL at D = 64, SF13).  1,560 x 24 x 128 (19 MB moved): 7.7 us; one
+// 4-vector per thread, four 2-byte accesses each way, 14 us.
+constexpr int CA_HEADS = 8;
+
+template <bool INTER>
+__global__ void __launch_bounds__(256) camera_pieces_kernel(CameraApplyParams p, uint32_t items) {
+    const uint32_t per_row = (uint32_t)p.D / 8, S = (uint32_t)p.S;
+    const uint32_t i = blockIdx.x * 256 + threadIdx.x;
+    if (i >= items) return;
+    const uint32_t bs = i / per_row, part = i - bs * per_row, b = bs / S, s = bs - b * S;
+    const int h0 = blockIdx.y * CA_HEADS;
+    const uint16_t* src = p.x + b * p.x_sb + s * p.x_st + h0 * p.x_sh + 8 * part;
+    uint16_t* dst = p.out + b * p.o_sb + s * p.o_st + h0 * p.o_sh + 8 * part;
+    u32x4 w[CA_HEADS];
+#pragma unroll
+    for (int h = 0; h < CA_HEADS; ++h)
+        if (h0 + h < p.H) w[h] = *reinterpret_cast<const u32x4*>(src + h * p.x_sh);
+    const float* mats = camera_mats(p.cam, (int)b, p.rows ? (int64_t)p.rows[s] : (int64_t)s);
+    double m[16];
+    auto matrix = [&](int sub) {
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const float4 f = reinterpret_cast<const float4*>(mats + 16 * sub)[q];
+            m[4 * q] = (double)bf16_round(f.x);
+            m[4 * q + 1] = (double)bf16_round(f.y);
+            m[4 * q + 2] = (double)bf16_round(f.z);
+            m[4 * q + 3] = (double)bf16_round(f.w);
+        }
+    };
+    // output r of m times the vector v
+    auto out = [&](int r, const double (&v)[4]) {
+        double acc = m[4 * r] * v[0];
+#pragma unroll
+        for (int j = 1; j < 4; ++j) acc = fma(m[4 * r + j], v[j], acc);
+        return f64_to_f32(acc);
+    };
+    auto lo = [](uint32_t x) { return (double)__uint_as_float(x << 16); };
+    auto hi = [](uint32_t x) { return (double)__uint_as_float(x & 0xffff0000u); };
+    if constexpr (INTER) {
+        matrix(part & 3);
+#pragma unroll
+        for (int h = 0; h < CA_HEADS; ++h) {
+            if (h0 + h >= p.H) break;
+            double a[4], c[4];
+#pragma unroll
+            for (int j = 0; j < 4; ++j) { a[j] = lo(w[h][j]); c[j] = hi(w[h][j]); }
+#pragma unroll
+            for (int r = 0; r < 4; ++r) w[h][r] = pack_bf16x2(out(r, a), out(r, c));
+        }
+    } else {
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+            int base, step, sub;
+            camera_vector_dims(p.cam.layout, p.D, 2 * (int)part + u, base, step, sub);
+            if (sub < 0) continue;
+            matrix(sub);
+#pragma unroll
+            for (int h = 0; h < CA_HEADS; ++h) {
+                if (h0 + h >= p.H) break;
+                const double a[4] = {lo(w[h][2 * u]), hi(w[h][2 * u]), lo(w[h][2 * u + 1]),
+                                     hi(w[h][2 * u + 1])};
+                w[h][2 * u] = pack_bf16x2(out(0, a), out(1, a));
+                w[h][2 * u + 1] = pack_bf16x2(out(2, a), out(3, a));
+            }
+        }
+    }
+#pragma unroll
+    for (int h = 0; h < CA_HEADS; ++h)
+        if (h0 + h < p.H) *reinterpret_cast<u32x4*>(dst + h * p.o_sh) = w[h];
+}
+
+// The 16-byte kernel where rows are whole aligned pieces and a piece's two
+// vectors lie in it; one 4-vector per thread for the rest (FULL at D >= 192,
+// odd strides).
+int camera_launch(hipStream_t s, const CameraApplyParams& p) {
+    const int D = p.D, layout = p.cam.layout;
+    const int64_t pieces = (int64_t)p.B * p.S * (D / 8);
+    const bool fits = layout == NKV_CAMERA_SF13 || D == 64 || D == 128;
+    if (D % 8 == 0 && fits && pieces <= INT32_MAX && cdiv(p.H, CA_HEADS) <= 65535 &&
+        rows16(p.x, p.x_sb, p.x_st, p.x_sh) && rows16(p.out, p.o_sb, p.o_st, p.o_sh)) {
+        const dim3 grid((unsigned)cdiv(pieces, 256), (unsigned)cdiv(p.H, CA_HEADS));
+        if (layout == NKV_CAMERA_FULL && D == 128)
+            camera_pieces_kernel<true><<<grid, 256, 0, s>>>(p, (uint32_t)pieces);
+        else
+            camera_pieces_kernel<false><<<grid, 256, 0, s>>>(p, (uint32_t)pieces);
+    } else {
+        const int64_t items = (int64_t)p.B * p.S * p.H * camera_vectors(layout, D);
+        const unsigned grid = (unsigned)std::min<int64_t>(cdiv(items, 256), 65536);
+        camera_apply_kernel<<<grid, 256, 0, s>>>(p);
+    }
+    NKV_LAUNCH_CHECK();
+    return NKV_OK;
+}
+
 }  // namespace
 }  // namespace nkv
 
@@ -103,11 +203,7 @@ int camera_apply_inplace(hipStream_t s, const CameraDev& cam, int B, int64_t S, 
     p.o_sb = sb;
     p.o_st = st;
     p.o_sh = sh;
-    const int64_t items = (int64_t)B * S * H * camera_vectors(cam.layout, D);
-    const unsigned grid = (unsigned)std::min<int64_t>(cdiv(items, 256), 65536);
-    camera_apply_kernel<<<grid, 256, 0, s>>>(p);
-    NKV_LAUNCH_CHECK();
-    return NKV_OK;
+    return camera_launch(s, p);
 }
 
 }  // namespace nkv
@@ -137,9 +233,5 @@ extern "C" int nkv_camera_apply(void* stream, const nkv_camera* camera, int B, i
     p.o_sb = o_sb;
     p.o_st = o_st;
     p.o_sh = o_sh;
-    const int64_t items = (int64_t)B * S * H * camera_vectors(camera->layout, D);
-    const unsigned grid = (unsigned)std::min<int64_t>(cdiv(items, 256), 65536);
-    camera_apply_kernel<<<grid, 256, 0, (hipStream_t)stream>>>(p);
-    NKV_LAUNCH_CHECK();
-    return NKV_OK;
+    return camera_launch((hipStream_t)stream, p);
 }
