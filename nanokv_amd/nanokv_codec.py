@@ -243,12 +243,21 @@ def preload_operator_weights(device: torch.device, path: Optional[str] = None) -
                           decoder=move(entry["decoder"]), mean=entry["mean"].float().to(device))
 
 
+def _indexed(device: torch.device) -> torch.device:
+    """device with its index: that of the current device for a bare "cuda"."""
+    if device.type == "cuda" and device.index is None:
+        return torch.device("cuda", torch.cuda.current_device())
+    return device
+
+
 def _operator(kind: str, layer: int, device: torch.device) -> dict:
     key = (kind, int(layer))
     if key not in _OPERATORS:
         raise RuntimeError(f"no codec operator registered for {kind}:{int(layer):02d}")
     op = _OPERATORS[key]
-    if op["encoder"].device != device:
+    have = op["encoder"].device
+    # ("cuda" is the current device: equal to its indexed form)
+    if have != device and have != _indexed(device):
         op = {k: (None if v is None else v.to(device)) for k, v in op.items()}
         _OPERATORS[key] = op
     return op
@@ -433,27 +442,36 @@ def codec_view(part: dict, device: torch.device) -> ops.Codec:
     """Device tensors of one encoded segment as an ops.Codec."""
     if part.get("codec") != CODEC:
         raise RuntimeError(f"unsupported WorldPlay payload {part.get('codec')}")
-    batch, seq, _ = (int(v) for v in part["shape"])
+    batch, seq, _ = part["shape"]
     r = int(part["latent_shape"][-1])
+    device = _indexed(device)
     op = _operator(str(part["kind"]), int(part["layer"]), device)
     group = int(part.get("scale_group", r))
-    scale = part["scale"].to(device)
+
+    def on(t: torch.Tensor) -> torch.Tensor:
+        return t if t.device == device else t.to(device)
+
+    def shaped(t: torch.Tensor, *shape: int) -> torch.Tensor:
+        return t if t.shape == shape else t.reshape(shape)
+
+    scale = on(part["scale"])
     if scale.dtype not in (torch.bfloat16, torch.float16):
         scale = scale.to(torch.bfloat16)
-    scale = scale.reshape(batch, seq, r // group).contiguous()
+    scale = shaped(scale, batch, seq, r // group).contiguous()
     centers = ids = None
     if part.get("semantic", True) and part.get("centers") is not None:
-        centers = part["centers"].to(device)
+        centers = on(part["centers"])
         if centers.dim() == 2:
             centers = centers[None]
-        centers = centers.to(torch.bfloat16).contiguous()
-        ids = part["ids"].to(device).reshape(batch, seq)
+        if centers.dtype != torch.bfloat16:
+            centers = centers.to(torch.bfloat16)
+        centers = centers.contiguous()
+        ids = shaped(on(part["ids"]), batch, seq)
         if ids.dtype not in (torch.uint8, torch.int16, torch.int32):
             ids = ids.to(ops.id_dtype_for(int(centers.shape[1])))
         ids = ids.contiguous()
-    return ops.Codec(packed=part["packed_codes"].to(device).reshape(batch, seq, r // 2),
-                     scales=scale, w_dec=op["decoder"], group=group, ids=ids,
-                     centers=centers, mean=op["mean"])
+    return ops.Codec(packed=on(part["packed_codes"]).reshape(batch, seq, r // 2), scales=scale,
+                     w_dec=op["decoder"], group=group, ids=ids, centers=centers, mean=op["mean"])
 
 
 # ---------------------------------------------------------------- decode
@@ -477,7 +495,8 @@ def decode_value(value: Any, *, dtype: torch.dtype, device: torch.device) -> tor
     if value.get("codec") == SEGMENTS:
         segments = value["segments"]
         if len(segments) > 1 and all(is_payload(p) and p["codec"] == CODEC for p in segments):
-            views = [codec_view(p, torch.device(device)) for p in segments]
+            dev = _indexed(torch.device(device))
+            views = [codec_view(p, dev) for p in segments]
             first = views[0]
             if all(v.batch == 1 and v.w_dec is first.w_dec and v.mean is first.mean
                    and (v.group, v.scales.dtype) == (first.group, first.scales.dtype)

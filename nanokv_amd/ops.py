@@ -33,7 +33,8 @@ if hasattr(torch, "uint16"):
 
 
 def _stream(device: torch.device) -> int:
-    return torch.cuda.current_stream(device).cuda_stream
+    # the raw handle: torch.cuda.current_stream builds a Stream object (3 us)
+    return torch._C._cuda_getCurrentRawStream(device.index)
 
 
 def _ptr(t: Optional[torch.Tensor]) -> Optional[int]:
@@ -41,19 +42,20 @@ def _ptr(t: Optional[torch.Tensor]) -> Optional[int]:
 
 
 def _require_gpu(*tensors: Optional[torch.Tensor]) -> torch.device:
-    device = None
+    first = index = None
     for t in tensors:
         if t is None:
             continue
-        if not t.is_cuda:
+        i = t.get_device()
+        if i < 0 or not t.is_cuda:
             raise ValueError("NanoKV HIP ops require GPU tensors (no CPU fallback)")
-        if device is None:
-            device = t.device
-        elif t.device != device:
-            raise ValueError(f"tensors on different devices: {device} vs {t.device}")
-    if device is None:
+        if first is None:
+            first, index = t, i
+        elif i != index:
+            raise ValueError(f"tensors on different devices: {first.device} vs {t.device}")
+    if first is None:
         raise ValueError("no tensor given")
-    return device
+    return first.device
 
 
 def _contig(t: torch.Tensor, dtype: torch.dtype, name: str) -> torch.Tensor:
@@ -355,9 +357,10 @@ class Codec:
         return src.dtype
 
     def validate(self, hd: int) -> None:
-        r = self.r
-        _contig(self.w_dec, torch.bfloat16, "w_dec")
-        if tuple(self.w_dec.shape) != (hd, r):
+        w = self.w_dec
+        _contig(w, torch.bfloat16, "w_dec")
+        r = w.shape[1]
+        if tuple(w.shape) != (hd, r):
             raise ValueError(f"w_dec must be [HD={hd}, r={r}]")
         if self.mean is not None:
             _contig(self.mean, torch.float32, "mean")
@@ -366,64 +369,62 @@ class Codec:
         if self.segments is not None:
             if self.group <= 0 or r % self.group:
                 raise ValueError("group must divide r")
+            batch, sdt = self.batch, self.scale_dtype
             for sg in self.segments.segments:
-                B, rows = int(sg.packed.shape[0]), int(sg.packed.shape[1])
-                if tuple(sg.packed.shape) != (B, rows, r // 2) or \
-                        tuple(sg.scales.shape) != (B, rows, r // self.group) or \
-                        B != self.batch or sg.scales.dtype != self.scale_dtype:
+                B, rows = sg.packed.shape[0], sg.packed.shape[1]
+                if sg.packed.shape != (B, rows, r // 2) or \
+                        sg.scales.shape != (B, rows, r // self.group) or \
+                        B != batch or sg.scales.dtype != sdt:
                     raise ValueError("every segment must be [B, rows, r/2] codes with "
                                      "[B, rows, r/group] scales of one dtype")
                 if sg.centers is not None and sg.centers.shape[2] != hd:
                     raise ValueError("segment centers must have HD columns")
             return
-        _contig(self.packed, torch.uint8, "packed")
-        _contig(self.w_dec, torch.bfloat16, "w_dec")
-        if self.scales.dtype not in _SCALE_CODES or not self.scales.is_contiguous():
+        packed, scales = self.packed, self.scales
+        _contig(packed, torch.uint8, "packed")
+        if scales.dtype not in _SCALE_CODES or not scales.is_contiguous():
             raise TypeError("scales must be a contiguous bf16 or fp16 tensor")
-        B, N = self.batch, self.tokens
-        if tuple(self.packed.shape) != (B, N, r // 2):
-            raise ValueError(f"packed must be [B, N, r/2], got {tuple(self.packed.shape)}")
-        if self.group <= 0 or r % self.group or tuple(self.scales.shape) != (B, N, r // self.group):
+        B, N = packed.shape[0], packed.shape[1]
+        if packed.shape != (B, N, r // 2):
+            raise ValueError(f"packed must be [B, N, r/2], got {tuple(packed.shape)}")
+        if self.group <= 0 or r % self.group or scales.shape != (B, N, r // self.group):
             raise ValueError("scales must be [B, N, r/group]")
         if self.centers is not None:
-            _contig(self.centers, torch.bfloat16, "centers")
-            if self.ids is None or self.ids.dtype not in _ID_BYTES or not self.ids.is_contiguous():
+            centers, ids = self.centers, self.ids
+            _contig(centers, torch.bfloat16, "centers")
+            if ids is None or ids.dtype not in _ID_BYTES or not ids.is_contiguous():
                 raise TypeError("ids must be a contiguous uint8/int16/int32 tensor with centers")
-            if tuple(self.ids.shape) != (B, N):
+            if ids.shape != (B, N):
                 raise ValueError("ids must be [B, N]")
-            if self.centers.dim() != 3 or self.centers.shape[0] not in (1, B) or \
-                    self.centers.shape[2] != hd:
+            if centers.dim() != 3 or centers.shape[0] not in (1, B) or centers.shape[2] != hd:
                 raise ValueError("centers must be [B or 1, C, HD]")
 
     def struct(self) -> NkvCodec:
-        c = NkvCodec()
-        c.w_dec = self.w_dec.data_ptr()
-        c.r, c.group, c.scale_dtype = self.r, self.group, _SCALE_CODES[self.scale_dtype]
-        if self.mean is not None:
-            c.mean = self.mean.data_ptr()
+        w, mean = self.w_dec, self.mean
+        mp = None if mean is None else mean.data_ptr()
         if self.segments is not None:
+            c = NkvCodec(None, None, None, None, w.data_ptr(), mp, w.shape[1], self.group,
+                         _SCALE_CODES[self.scale_dtype])
             c.n_segments = len(self.segments.segments)
             c.segments = ctypes.cast(self.segments.host, ctypes.POINTER(NkvSegment))
             c.segments_dev = self.segments.device.data_ptr()
             return c
-        c.packed, c.scales = self.packed.data_ptr(), self.scales.data_ptr()
-        if self.centers is not None:
-            c.centers, c.ids = self.centers.data_ptr(), self.ids.data_ptr()
-            c.id_bytes = _ID_BYTES[self.ids.dtype]
-            c.num_centers = int(self.centers.shape[1])
-            c.centers_batch_stride = (0 if self.centers.shape[0] == 1
-                                      else int(self.centers.stride(0)))
-        return c
+        centers = self.centers
+        if centers is None:
+            return NkvCodec(self.packed.data_ptr(), self.scales.data_ptr(), None, None,
+                            w.data_ptr(), mp, w.shape[1], self.group,
+                            _SCALE_CODES[self.scales.dtype])
+        return NkvCodec(self.packed.data_ptr(), self.scales.data_ptr(), self.ids.data_ptr(),
+                        centers.data_ptr(), w.data_ptr(), mp, w.shape[1], self.group,
+                        _SCALE_CODES[self.scales.dtype], _ID_BYTES[self.ids.dtype],
+                        centers.shape[1], 0, 0 if centers.shape[0] == 1 else centers.stride(0))
 
 
 def _decode_args(codec: Codec, hd: int) -> NkvDecodeArgs:
     """nkv_decode_args of every row of a flat codec (out not set)."""
     codec.validate(hd)
-    args = NkvDecodeArgs()
-    args.B, args.HD, args.N = codec.batch, hd, codec.tokens
-    args.rows = codec.tokens
-    args.codec = codec.struct()
-    return args
+    B, N = codec.packed.shape[0], codec.packed.shape[1]
+    return NkvDecodeArgs(B, hd, N, N, None, codec.struct())
 
 
 def decode(codec: Codec, hd: int, row_index: Optional[torch.Tensor] = None) -> torch.Tensor:
@@ -462,11 +463,12 @@ def decode_batch(codecs: list, hd: int) -> torch.Tensor:
 
 
 def _strides_bthd(t: torch.Tensor, name: str) -> tuple[int, int, int]:
-    if t.dim() != 4 or t.stride(3) != 1:
+    st = t.stride()
+    if len(st) != 4 or st[3] != 1:
         raise ValueError(f"{name} must be [B, T, H, D] with contiguous D")
-    if t.data_ptr() % 16 or any(s % 8 for s in t.stride()[:3]):
+    if t.data_ptr() % 16 or st[0] % 8 or st[1] % 8 or st[2] % 8:
         raise ValueError(f"{name} must be 16-byte aligned with strides divisible by 8")
-    return t.stride(0), t.stride(1), t.stride(2)
+    return st[0], st[1], st[2]
 
 
 def _attend_args(q: torch.Tensor, k_cur: Optional[torch.Tensor], v_cur: Optional[torch.Tensor],
@@ -706,24 +708,18 @@ class Rope:
         return int(self.frame_pos.numel()) * self.grid_h * self.grid_w
 
     def struct(self) -> NkvRope:
-        for name in ("cs_t", "cs_h", "cs_w"):
-            t = getattr(self, name)
-            _contig(t, torch.float64, name)
-            if t.dim() != 3 or t.shape[2] != 2:
+        t, h, w = self.cs_t, self.cs_h, self.cs_w
+        for name, x in (("cs_t", t), ("cs_h", h), ("cs_w", w)):
+            _contig(x, torch.float64, name)
+            if x.dim() != 3 or x.shape[2] != 2:
                 raise ValueError(f"{name} must be [n, pairs, 2] float64")
         _contig(self.frame_pos, torch.int32, "frame_pos")
-        _require_gpu(self.cs_t, self.cs_h, self.cs_w, self.frame_pos)
-        if self.cs_h.shape[0] < self.grid_h or self.cs_w.shape[0] < self.grid_w:
+        _require_gpu(t, h, w, self.frame_pos)
+        if h.shape[0] < self.grid_h or w.shape[0] < self.grid_w:
             raise ValueError("cs_h / cs_w have fewer rows than the token grid")
-        r = NkvRope()
-        r.cs_t, r.cs_h, r.cs_w = (self.cs_t.data_ptr(), self.cs_h.data_ptr(),
-                                  self.cs_w.data_ptr())
-        r.frame_pos, r.n_frames = self.frame_pos.data_ptr(), int(self.frame_pos.numel())
-        r.n_t = int(self.cs_t.shape[0])
-        r.pt, r.ph, r.pw = (int(self.cs_t.shape[1]), int(self.cs_h.shape[1]),
-                            int(self.cs_w.shape[1]))
-        r.grid_h, r.grid_w = self.grid_h, self.grid_w
-        return r
+        return NkvRope(t.data_ptr(), h.data_ptr(), w.data_ptr(), self.frame_pos.data_ptr(),
+                       self.frame_pos.numel(), t.shape[0], t.shape[1], h.shape[1], w.shape[1],
+                       self.grid_h, self.grid_w)
 
 
 @dataclass
@@ -816,7 +812,7 @@ def rope_apply(x: torch.Tensor, rope: Rope, rows: Optional[torch.Tensor] = None,
     device = _require_gpu(x, rows, out)
     if x.dtype != torch.bfloat16 or x.dim() != 4 or x.stride(3) != 1:
         raise ValueError("x must be bf16 [B, S, H, D] with contiguous D")
-    B, S, H, D = (int(v) for v in x.shape)
+    B, S, H, D = x.shape
     if rows is not None:
         _contig(rows, torch.int32, "rows")
         if rows.numel() != S:
@@ -826,9 +822,10 @@ def rope_apply(x: torch.Tensor, rope: Rope, rows: Optional[torch.Tensor] = None,
     elif out.shape != x.shape or out.dtype != torch.bfloat16 or out.stride(3) != 1:
         raise ValueError("out must match x")
     r = rope.struct()
+    xs, os_ = x.stride(), out.stride()
     check("nkv_rope_apply", lib().nkv_rope_apply(
-        _stream(device), byref(r), B, S, H, D, x.data_ptr(), x.stride(0), x.stride(1),
-        x.stride(2), _ptr(rows), out.data_ptr(), out.stride(0), out.stride(1), out.stride(2)))
+        _stream(device), byref(r), B, S, H, D, x.data_ptr(), xs[0], xs[1], xs[2], _ptr(rows),
+        out.data_ptr(), os_[0], os_[1], os_[2]))
     return out
 
 
@@ -856,14 +853,10 @@ class Camera:
             raise ValueError("mats must be [batches, n_mats, 4, 4, 4] float32")
         if self.layout not in CAMERA_LAYOUTS:
             raise ValueError(f"camera layout must be one of {sorted(CAMERA_LAYOUTS)}")
-        c = NkvCamera()
-        c.mats = self.mats.data_ptr()
-        c.mats_bs = self.mats.stride(0) if self.mats.shape[0] > 1 else 0
-        c.n_mats, c.layout = int(self.mats.shape[1]), CAMERA_LAYOUTS[self.layout]
-        c.frame_mat, c.n_frames = self.frame_mat.data_ptr(), int(self.frame_mat.numel())
-        c.tokens_per_frame = int(self.tokens_per_frame)
-        c.n_batches = int(self.mats.shape[0])
-        return c
+        m = self.mats
+        return NkvCamera(m.data_ptr(), m.stride(0) if m.shape[0] > 1 else 0, m.shape[1],
+                         CAMERA_LAYOUTS[self.layout], self.frame_mat.data_ptr(),
+                         self.frame_mat.numel(), int(self.tokens_per_frame), m.shape[0])
 
 
 def camera_apply(x: torch.Tensor, camera: Camera, rows: Optional[torch.Tensor] = None,
@@ -875,7 +868,7 @@ def camera_apply(x: torch.Tensor, camera: Camera, rows: Optional[torch.Tensor] =
     device = _require_gpu(x, rows, out)
     if x.dtype != torch.bfloat16 or x.dim() != 4 or x.stride(3) != 1:
         raise ValueError("x must be bf16 [B, S, H, D] with contiguous D")
-    B, S, H, D = (int(v) for v in x.shape)
+    B, S, H, D = x.shape
     if camera.mats.shape[0] not in (1, B):
         raise ValueError("camera batch must match x or broadcast")
     if rows is not None:
@@ -887,9 +880,10 @@ def camera_apply(x: torch.Tensor, camera: Camera, rows: Optional[torch.Tensor] =
     elif out.shape != x.shape or out.dtype != torch.bfloat16 or out.stride(3) != 1:
         raise ValueError("out must match x")
     c = camera.struct()
+    xs, os_ = x.stride(), out.stride()
     check("nkv_camera_apply", lib().nkv_camera_apply(
-        _stream(device), byref(c), B, S, H, D, x.data_ptr(), x.stride(0), x.stride(1),
-        x.stride(2), _ptr(rows), out.data_ptr(), out.stride(0), out.stride(1), out.stride(2)))
+        _stream(device), byref(c), B, S, H, D, x.data_ptr(), xs[0], xs[1], xs[2], _ptr(rows),
+        out.data_ptr(), os_[0], os_[1], os_[2]))
     return out
 
 
