@@ -834,34 +834,79 @@ int resolve_schedule(const nkv_attend_args* a, int* schedule) {
 }  // namespace
 
 // ------------------------------------------------- heads narrower than 128
-// A head width D < 128 (D % 8 == 0; BASELINE config 0 has D = 64) runs
+// A head width D < 128 (D % 8 == 0, for example 64) runs
 // through the D = 128 kernels on operands padded with zero columns to 128 per
 // head.  The zero dimensions add nothing to q.k, and the padded decoder rows,
 // centers and mean make every padded history row exactly the decoded row
 // followed by zeros (bf16(bf16(0 + 0) + 0) = 0), so the first D columns of
 // the output are the attention at width D (the caller's softmax_scale is
-// used as given).  The padded q, current K/V, output, decoder weights,
-// centers and means sit at the front of the caller's workspace; the rest is
-// the D = 128 call's workspace.  RoPE, the camera and segmented codecs keep
+// used as given).  The padded q, current K/V, decoder weights, centers and
+// means sit at the front of the caller's workspace; the rest is the D = 128
+// call's workspace.  The key-chunk schedule's merge writes the first D
+// columns straight to the caller's output; the query tiles write a padded
+// output, which one more launch cuts.  RoPE, the camera and segmented codecs keep
 // their D = 128 requirement.
 namespace {
 
-// [rows = B*T, H, D] strided bf16 -> [rows, H, 128] contiguous, one 16-byte
-// unit per thread, zero units past D
-__global__ void __launch_bounds__(256) pad_heads_kernel(const uint16_t* __restrict__ src,
-                                                        int64_t sb, int64_t st, int64_t sh,
-                                                        int64_t T, int H, int D, int64_t rows,
-                                                        uint16_t* __restrict__ dst) {
-    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if (i >= rows * H * (AT_D / 8)) return;
-    const int c = (int)(i % (AT_D / 8));
-    const int64_t rh = i / (AT_D / 8);
-    const int h = (int)(rh % H);
-    const int64_t row = rh / H;
+// One padded operand: destination blocks of `full` 16-byte units, block
+// (row, h) = rows [B*T] x [H], whose first `part` units are copied from src +
+// (row / T)*sb + (row % T)*st + h*sh and whose others are zero.  Rows of
+// q / K / V and of the center tables are blocks of one head (16 units, D / 8
+// of them copied); a decoder is one row of H blocks of 128 rows of r, a mean
+// one row of H blocks of 128 fp32.
+struct PadJob {
+    const uint16_t* src;
+    uint16_t* dst;
+    int64_t sb, st, sh, T;
+    int64_t units;  // B * T * H * full
+    int64_t first;  // first block of the launch that works on it
+    int H, full, part;
+    int vec;        // the source units are 16-byte aligned
+};
+constexpr int kPadJobs = 9;  // q, K, V of the current keys; decoder, centers, mean of K and V
+struct PadJobs {
+    PadJob job[kPadJobs];
+    int n;
+};
+
+// Every padded operand of a call in one launch, one unit per thread: at the
+// sizes these calls have, a launch costs more than the copy.  At 8 heads of
+// 64, 256 queries and current keys over 2,048 rows of rank 64, one launch per
+// operand took 7 x 2.4 - 2.7 us and the cut of a padded output 4.1 us; this
+// one takes 4.2 us (the call 52.4 -> 39.6 us).
+__global__ void __launch_bounds__(256) pad_operands_kernel(PadJobs P) {
+    int k = 0;
+#pragma unroll
+    for (int i = 1; i < kPadJobs; ++i)
+        if (i < P.n && blockIdx.x >= P.job[i].first) k = i;
+    const PadJob& J = P.job[k];
+    const int64_t i = (blockIdx.x - J.first) * 256 + threadIdx.x;
+    if (i >= J.units) return;
+    // unit, head, row and batch item of i (a 64-bit quotient costs several
+    // 32-bit ones)
+    int c, h;
+    int64_t t, b;
+    auto locate = [&](auto u, auto T) {
+        const auto rh = u / (decltype(u))J.full, row = rh / (decltype(u))J.H;
+        c = (int)(u - rh * J.full);
+        h = (int)(rh - row * J.H);
+        b = row / T;
+        t = row - b * T;
+    };
+    if (J.units <= UINT32_MAX) locate((uint32_t)i, (uint32_t)J.T);
+    else locate((uint64_t)i, (uint64_t)J.T);
     u32x4 v = {0u, 0u, 0u, 0u};
-    if (c < D / 8)
-        v = *reinterpret_cast<const u32x4*>(src + (row / T) * sb + (row % T) * st + h * sh + 8 * c);
-    *reinterpret_cast<u32x4*>(dst + 8 * i) = v;
+    if (c < J.part) {
+        const uint16_t* src = J.src + b * J.sb + t * J.st + h * J.sh + 8 * c;
+        if (J.vec) {
+            v = *reinterpret_cast<const u32x4*>(src);
+        } else {
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+                v[e] = (uint32_t)src[2 * e] | ((uint32_t)src[2 * e + 1] << 16);
+        }
+    }
+    *reinterpret_cast<u32x4*>(J.dst + 8 * i) = v;
 }
 
 // the reverse: the first D columns of [rows, H, 128] into the strided output
@@ -878,18 +923,6 @@ __global__ void __launch_bounds__(256) unpad_heads_kernel(const uint16_t* __rest
     const int64_t row = rh / H;
     *reinterpret_cast<u32x4*>(dst + (row / T) * sb + (row % T) * st + h * sh + 8 * c) =
         *reinterpret_cast<const u32x4*>(src + (rh * AT_D + 8 * c));
-}
-
-// [A, D, W] -> [A, 128, W] of 16-bit elements, zero rows past D (decoder
-// rows [H, D, r], center tables [C*H, D, 1], fp32 means as [H, D, 2])
-__global__ void __launch_bounds__(256) pad_rows_kernel(const uint16_t* __restrict__ src, int64_t A,
-                                                       int D, int64_t W, uint16_t* __restrict__ dst) {
-    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if (i >= A * AT_D * W) return;
-    const int64_t w = i % W, rest = i / W;
-    const int d = (int)(rest % AT_D);
-    const int64_t a = rest / AT_D;
-    dst[i] = d < D ? src[(a * D + d) * W + w] : (uint16_t)0;
 }
 
 constexpr size_t kNarrowAlign = 256;
@@ -912,6 +945,12 @@ int narrow_check(const nkv_attend_args* a) {
     return NKV_OK;
 }
 
+// Whether the D = 128 call over the padded operands takes the key chunks
+// (a bad schedule is refused by that call's own check).
+bool narrow_key_chunks(const nkv_attend_args* a) {
+    return a->schedule == NKV_SCHEDULE_AUTO || a->schedule == NKV_SCHEDULE_KEY_CHUNKS;
+}
+
 int center_tables(const nkv_attend_args* a, const nkv_codec& c) {
     return c.centers_batch_stride ? a->B : 1;
 }
@@ -926,7 +965,7 @@ NarrowLayout narrow_layout(const nkv_attend_args* a) {
     };
     const size_t row = (size_t)a->H * AT_D * sizeof(uint16_t);
     L.q = take((size_t)a->B * a->Q * row);
-    L.o = take((size_t)a->B * a->Q * row);
+    if (!narrow_key_chunks(a)) L.o = take((size_t)a->B * a->Q * row);
     L.kc = take((size_t)a->B * a->Nc * row);
     L.vc = take((size_t)a->B * a->Nc * row);
     for (int i = 0; i < 2; ++i) {
@@ -948,8 +987,10 @@ nkv_attend_args narrow_args(const nkv_attend_args* a, const NarrowLayout& L, uns
     const int64_t hd = (int64_t)a->H * AT_D;
     n.q = reinterpret_cast<const uint16_t*>(base + L.q);
     n.q_sb = a->Q * hd, n.q_st = hd, n.q_sh = AT_D;
-    n.out = reinterpret_cast<uint16_t*>(base + L.o);
-    n.o_sb = a->Q * hd, n.o_st = hd, n.o_sh = AT_D;
+    if (!narrow_key_chunks(a)) {
+        n.out = reinterpret_cast<uint16_t*>(base + L.o);
+        n.o_sb = a->Q * hd, n.o_st = hd, n.o_sh = AT_D;
+    }
     if (a->Nc > 0) {
         n.k_cur = reinterpret_cast<const uint16_t*>(base + L.kc);
         n.v_cur = reinterpret_cast<const uint16_t*>(base + L.vc);
@@ -1009,7 +1050,8 @@ int inner_workspace(const nkv_attend_args* a, size_t* need) {
     return NKV_OK;
 }
 
-int attend_d128(hipStream_t s, const nkv_attend_args* a, void* workspace, size_t workspace_bytes);
+int attend_d128(hipStream_t s, const nkv_attend_args* a, void* workspace, size_t workspace_bytes,
+                int out_cols);
 
 int attend_narrow(hipStream_t s, const nkv_attend_args* a, void* workspace, size_t workspace_bytes) {
     int rc = narrow_check(a);
@@ -1045,48 +1087,44 @@ int attend_narrow(hipStream_t s, const nkv_attend_args* a, void* workspace, size
     const NarrowLayout L = narrow_layout(a);
     const nkv_attend_args n = narrow_args(a, L, base);
     const int D = a->D;
-    auto blocks = [](int64_t work) { return dim3((unsigned)cdiv(work, 256)); };
-    const int64_t qrows = (int64_t)a->B * a->Q;
-    pad_heads_kernel<<<blocks(qrows * a->H * (AT_D / 8)), 256, 0, s>>>(
-        a->q, a->q_sb, a->q_st, a->q_sh, a->Q, a->H, D, qrows, const_cast<uint16_t*>(n.q));
-    NKV_LAUNCH_CHECK();
+    PadJobs jobs{};
+    int64_t blocks = 0;
+    auto pad = [&](const uint16_t* src, const uint16_t* dst, int64_t B, int64_t T, int64_t width,
+                   int64_t sb, int64_t st, int64_t sh) {
+        PadJob& J = jobs.job[jobs.n++];
+        J.src = src, J.dst = const_cast<uint16_t*>(dst);
+        J.sb = sb, J.st = st, J.sh = sh, J.T = T, J.H = a->H;
+        J.full = (int)(width * AT_D / 8), J.part = (int)(width * D / 8);
+        J.units = B * T * a->H * J.full;
+        J.vec = rows16(src, sb, st, sh);
+        J.first = blocks;
+        blocks += cdiv(J.units, 256);
+    };
+    const int64_t hd = (int64_t)a->H * D;
+    pad(a->q, n.q, a->B, a->Q, 1, a->q_sb, a->q_st, a->q_sh);
     if (a->Nc > 0) {
-        const int64_t crows = (int64_t)a->B * a->Nc;
-        pad_heads_kernel<<<blocks(crows * a->H * (AT_D / 8)), 256, 0, s>>>(
-            a->k_cur, a->k_sb, a->k_st, a->k_sh, a->Nc, a->H, D, crows, const_cast<uint16_t*>(n.k_cur));
-        NKV_LAUNCH_CHECK();
-        pad_heads_kernel<<<blocks(crows * a->H * (AT_D / 8)), 256, 0, s>>>(
-            a->v_cur, a->v_sb, a->v_st, a->v_sh, a->Nc, a->H, D, crows, const_cast<uint16_t*>(n.v_cur));
-        NKV_LAUNCH_CHECK();
+        pad(a->k_cur, n.k_cur, a->B, a->Nc, 1, a->k_sb, a->k_st, a->k_sh);
+        pad(a->v_cur, n.v_cur, a->B, a->Nc, 1, a->v_sb, a->v_st, a->v_sh);
     }
     if (a->N > 0) {
         for (int i = 0; i < 2; ++i) {
             const nkv_codec& c = i ? a->value : a->key;
             const nkv_codec& cn = i ? n.value : n.key;
-            pad_rows_kernel<<<blocks((int64_t)a->H * AT_D * c.r), 256, 0, s>>>(
-                c.w_dec, a->H, D, c.r, const_cast<uint16_t*>(cn.w_dec));
-            NKV_LAUNCH_CHECK();
-            if (c.centers) {
-                const int tables = center_tables(a, c);
-                const int64_t A = (int64_t)c.num_centers * a->H;
-                for (int t = 0; t < tables; ++t) {
-                    pad_rows_kernel<<<blocks(A * AT_D), 256, 0, s>>>(
-                        c.centers + t * c.centers_batch_stride, A, D, 1,
-                        const_cast<uint16_t*>(cn.centers) + (int64_t)t * A * AT_D);
-                    NKV_LAUNCH_CHECK();
-                }
-            }
-            if (c.mean) {
-                pad_rows_kernel<<<blocks((int64_t)a->H * AT_D * 2), 256, 0, s>>>(
-                    reinterpret_cast<const uint16_t*>(c.mean), a->H, D, 2,
-                    reinterpret_cast<uint16_t*>(const_cast<float*>(cn.mean)));
-                NKV_LAUNCH_CHECK();
-            }
+            pad(c.w_dec, cn.w_dec, 1, 1, c.r, 0, 0, (int64_t)D * c.r);
+            if (c.centers)
+                pad(c.centers, cn.centers, center_tables(a, c), c.num_centers, 1,
+                    c.centers_batch_stride, hd, D);
+            if (c.mean)  // an fp32 is two 16-bit elements
+                pad(reinterpret_cast<const uint16_t*>(c.mean),
+                    reinterpret_cast<const uint16_t*>(cn.mean), 1, 1, 2, 0, 0, 2 * D);
         }
     }
-    rc = attend_d128(s, &n, base + L.inner, workspace_bytes - L.inner);
-    if (rc) return rc;
-    unpad_heads_kernel<<<blocks(qrows * a->H * (D / 8)), 256, 0, s>>>(
+    pad_operands_kernel<<<dim3((unsigned)blocks), 256, 0, s>>>(jobs);
+    NKV_LAUNCH_CHECK();
+    rc = attend_d128(s, &n, base + L.inner, workspace_bytes - L.inner, D);
+    if (rc || narrow_key_chunks(a)) return rc;
+    const int64_t qrows = (int64_t)a->B * a->Q;
+    unpad_heads_kernel<<<dim3((unsigned)cdiv(qrows * a->H * (D / 8), 256)), 256, 0, s>>>(
         n.out, a->Q, a->H, D, qrows, a->out, a->o_sb, a->o_st, a->o_sh);
     NKV_LAUNCH_CHECK();
     return NKV_OK;
@@ -1105,12 +1143,15 @@ extern "C" int nkv_attend(void* stream, const nkv_attend_args* a, void* workspac
     clear_error();
     hipStream_t s = (hipStream_t)stream;
     if (a && a->D != AT_D) return attend_narrow(s, a, workspace, workspace_bytes);
-    return attend_d128(s, a, workspace, workspace_bytes);
+    return attend_d128(s, a, workspace, workspace_bytes, AT_D);
 }
 
 namespace {
 
-int attend_d128(hipStream_t s, const nkv_attend_args* a, void* workspace, size_t workspace_bytes) {
+// out_cols: the columns of each output row that the key chunks' merge writes
+// (the query tiles always write all 128).
+int attend_d128(hipStream_t s, const nkv_attend_args* a, void* workspace, size_t workspace_bytes,
+                int out_cols) {
     AttendPlan pl;
     int rc = plan_attend(a, &pl);
     if (rc) return rc;
@@ -1118,7 +1159,8 @@ int attend_d128(hipStream_t s, const nkv_attend_args* a, void* workspace, size_t
     rc = resolve_schedule(a, &sch);
     if (rc) return rc;
     if (a->Q == 0) return NKV_OK;
-    if (sch == NKV_SCHEDULE_KEY_CHUNKS) return chunk_attend_launch(s, a, workspace, workspace_bytes);
+    if (sch == NKV_SCHEDULE_KEY_CHUNKS)
+        return chunk_attend_launch(s, a, workspace, workspace_bytes, out_cols);
     const size_t need = workspace_bytes_for(a, pl);
     NKV_REQUIRE(need == 0 || (workspace && workspace_bytes >= need), NKV_ERR_WORKSPACE,
                 "workspace missing or smaller than nkv_attend_workspace_size()");

@@ -105,6 +105,7 @@ struct ChunkParams {
     float* part_ml;     // [B*H, nch_total, qblocks * 32, 2]: running max (log2 units), row sum
     uint16_t* out;
     int64_t o_sb, o_st, o_sh;
+    int o_cols;         // columns of each output row to write (a multiple of 8, at most 128)
     float* lse;
     RopeDev rope;       // RoPE of the history keys (cs_t null: none)
     CameraDev cam;      // camera P^-1 of the history keys and values (mats null: none)
@@ -1906,8 +1907,8 @@ __device__ __forceinline__ void combine_partials(CombineAcc& A, const uint16_t* 
 // query (lane and lane ^ 32, which hold the two halves of every 8-dim
 // block) must reach this call.
 __device__ __forceinline__ void combine_store(const CombineAcc& A, uint16_t* out, int64_t o_sb,
-                                              int64_t o_st, int64_t o_sh, float* lse, int64_t Q,
-                                              int H, int b, int h, int64_t qi, int half, int lane,
+                                              int64_t o_st, int64_t o_sh, int o_cols, float* lse,
+                                              int64_t Q, int H, int b, int h, int64_t qi, int half, int lane,
                                               const float* shift, const CameraDev* ocam = nullptr) {
     const int hf = lane >> 5;
     const float inv = A.L > 0.0f ? 1.0f / A.L : 0.0f;
@@ -1934,6 +1935,7 @@ __device__ __forceinline__ void combine_store(const CombineAcc& A, uint16_t* out
         const int st = CB_ROWS * half + (n >> 1);
         const int db = st >> 1, i = 8 * (st & 1) + 4 * (n & 1);
         const int d = 32 * db + 8 * (i >> 2);
+        if (d >= o_cols) continue;  // o_cols is a multiple of 8: whole 8-column units
         float v[4];
 #pragma unroll
         for (int e = 0; e < 4; ++e) v[e] = A.acc[4 * n + e];
@@ -1989,7 +1991,7 @@ __global__ void __launch_bounds__(64 * CB_WAVES) chunk_combine_kernel(ChunkParam
     const int64_t gw = (int64_t)blockIdx.x * CB_WAVES + wave;
     const int64_t gq = gw >> 1;
     const int half = (int)(gw & 1);
-    if (gq >= (int64_t)p.B * p.H * p.qblocks) return;
+    if (gq >= (int64_t)p.B * p.H * p.qblocks || half * (CK_D / 2) >= p.o_cols) return;
     const int64_t bh = gq / p.qblocks;
     const int qblk = (int)(gq % p.qblocks);
     CombineAcc A;
@@ -1997,8 +1999,8 @@ __global__ void __launch_bounds__(64 * CB_WAVES) chunk_combine_kernel(ChunkParam
     combine_partials(A, p.part_o, p.part_ml, bh, p.nch_total, p.qblocks, qblk, half, lane, false);
     const int64_t qi = (int64_t)qblk * 32 + (lane & 31);
     if (qi >= p.Q) return;
-    combine_store(A, p.out, p.o_sb, p.o_st, p.o_sh, p.lse, p.Q, p.H, (int)(bh / p.H),
-                  (int)(bh % p.H), qi, half, lane, nullptr);
+    combine_store(A, p.out, p.o_sb, p.o_st, p.o_sh, p.o_cols, p.lse, p.Q, p.H,
+                  (int)(bh / p.H), (int)(bh % p.H), qi, half, lane, nullptr);
 }
 
 // The staged schedule's merge over every partition (CN/core.py:33-42 for
@@ -2017,7 +2019,7 @@ __global__ void __launch_bounds__(64 * CB_WAVES) staged_combine_kernel(MultiPara
     const int64_t gw = (int64_t)blockIdx.x * CB_WAVES + wave;
     const int64_t gq = gw >> 1;
     const int half = (int)(gw & 1);
-    if (gq >= (int64_t)n.B * n.H * n.qblocks) return;
+    if (gq >= (int64_t)n.B * n.H * n.qblocks || half * (CK_D / 2) >= n.o_cols) return;
     const int64_t bh = gq / n.qblocks;
     const int qblk = (int)(gq % n.qblocks);
     const int b = (int)(bh / n.H), h = (int)(bh % n.H);
@@ -2039,7 +2041,7 @@ __global__ void __launch_bounds__(64 * CB_WAVES) staged_combine_kernel(MultiPara
     }
     const int64_t qi = (int64_t)qblk * 32 + (lane & 31);
     if (qi >= n.Q) return;
-    combine_store(A, n.out, n.o_sb, n.o_st, n.o_sh, n.lse, n.Q, n.H, b, h, qi, half, lane,
+    combine_store(A, n.out, n.o_sb, n.o_st, n.o_sh, n.o_cols, n.lse, n.Q, n.H, b, h, qi, half, lane,
                   lp && shift ? shift + (int64_t)b * sh_sb + (int64_t)h * sh_sh : nullptr,
                   ocam.mats ? &ocam : nullptr);
 }
@@ -2735,6 +2737,7 @@ ChunkParams chunk_params(const ChunkLaunchDesc& d) {
     p.o_sb = d.o_sb;
     p.o_st = d.o_st;
     p.o_sh = d.o_sh;
+    p.o_cols = d.o_cols ? d.o_cols : CK_D;
     p.lse = d.lse;
     p.rope = d.rope;
     p.cam = d.cam;
@@ -2940,12 +2943,13 @@ int chunk_check(const nkv_attend_args* a) {
 }
 
 int chunk_attend_launch(hipStream_t s, const nkv_attend_args* a, void* workspace,
-                        size_t workspace_bytes) {
+                        size_t workspace_bytes, int out_cols) {
     int rc = chunk_check(a);
     if (rc) return rc;
     ChunkLaunchDesc d;
     rc = full_desc(a, &d);
     if (rc) return rc;
+    d.o_cols = out_cols;
     return chunk_launch(s, d, workspace, workspace_bytes);
 }
 

@@ -122,6 +122,7 @@ struct ChunkLaunchDesc {
     ChunkCodec key, value;
     uint16_t* out;
     int64_t o_sb, o_st, o_sh;
+    int o_cols;  // columns of each output row to write: a multiple of 8 (0: all 128)
     float* lse;
     void* ev_begin;  // optional hipEvent_t recorded around the attention kernel
     void* ev_end;
@@ -151,8 +152,9 @@ int check_segments(const nkv_codec& c, int64_t N);
 // Key-chunk schedule (nkv_chunk.hip).
 int chunk_check(const nkv_attend_args* a);
 size_t chunk_workspace_bytes(const nkv_attend_args* a);
+// out_cols: columns of each output row to write (0: all 128).
 int chunk_attend_launch(hipStream_t s, const nkv_attend_args* a, void* workspace,
-                        size_t workspace_bytes);
+                        size_t workspace_bytes, int out_cols);
 size_t chunk_launch_workspace(const ChunkLaunchDesc& d);
 int chunk_launch(hipStream_t s, const ChunkLaunchDesc& d, void* workspace, size_t workspace_bytes);
 

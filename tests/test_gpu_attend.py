@@ -60,6 +60,39 @@ def test_attend_narrow_heads(dev, D, B, with_mean, schedule):
 
 
 @pytest.mark.parametrize("schedule", SCHEDULES)
+@pytest.mark.parametrize("D,Q,Nc", [(8, 1, 0), (56, 33, 1), (64, 65, 40), (72, 32, 31),
+                                    (120, 257, 33)])
+def test_attend_narrow_operands(dev, D, Q, Nc, schedule):
+    """Narrow heads at the edges of the output's column halves, with decoder
+    rows, centers (a table per batch item) and means that start off a 16-byte
+    boundary: the oracle's bar, and the bits of aligned tables; nothing past
+    the output's columns is written."""
+    sc = Scenario(B=2, H=16 if D == 8 else 3, D=D, N=257, Q=Q, Nc=Nc, rK=64, rV=128, G=32, C=5,
+                  with_mean=True, seed=D)
+
+    def shifted(t, by):
+        room = torch.zeros(t.numel() + by, dtype=t.dtype, device=dev)
+        room[by:] = t.reshape(-1)
+        return room[by:].view(t.shape)
+
+    key, value = sc.codecs(dev)
+    out, lse = _check(sc, dev, schedule=schedule)
+    off = []
+    for c in (key, value):
+        off.append(ops.Codec(packed=c.packed, scales=c.scales, w_dec=shifted(c.w_dec, 1),
+                             group=c.group, ids=c.ids,
+                             centers=shifted(c.centers.expand(2, -1, -1).contiguous(), 3),
+                             mean=shifted(c.mean, 1)))
+    kc = sc.k_cur.to(dev) if Nc else None
+    vc = sc.v_cur.to(dev) if Nc else None
+    room = torch.full((2, Q, sc.H, D + 8), 7.0, dtype=torch.bfloat16, device=dev)
+    _, lse2 = ops.attend(sc.q.to(dev), kc, vc, *off, out=room[..., :D], schedule=schedule)
+    assert np.array_equal(room[..., :D].float().cpu().numpy(), out)
+    assert np.array_equal(lse2.cpu().numpy(), lse)
+    assert bool((room[..., D:] == 7.0).all())
+
+
+@pytest.mark.parametrize("schedule", SCHEDULES)
 @pytest.mark.parametrize("N,Nc,Q", [(200, 64, 100), (257, 37, 300), (64, 0, 1), (0, 100, 33),
                                     (1000, 130, 513)])
 def test_attend_shapes(dev, N, Nc, Q, schedule):
