@@ -114,6 +114,16 @@ def test_attend_current_chunk_query_shares(dev, N, Nc, Q):
     _check(Scenario(H=2, N=N, Q=Q, Nc=Nc, rK=128, rV=128, G=32, C=8), dev, schedule="key_chunks")
 
 
+# key splits down to a single tile, and both sides of the line (128 query
+# blocks of 32 over all heads) where a merge wave's share of a block changes:
+# 16 and 9 splits of one query block each, 128 and 129 blocks, more splits
+# than a wave's loads in flight, a ragged last tile
+@pytest.mark.parametrize("H,N,Nc,Q", [(2, 2100, 0, 33), (1, 1, 1153, 1), (16, 300, 0, 256),
+                                      (43, 130, 0, 65), (22, 2300, 5, 161)])
+def test_attend_few_tiles_per_split(dev, H, N, Nc, Q):
+    _check(Scenario(H=H, N=N, Q=Q, Nc=Nc, rK=64, rV=64, G=32, C=4), dev, heads=[0, H - 1])
+
+
 @pytest.mark.parametrize("splits", [1, 2, 5, 0])
 def test_attend_splits(dev, splits):
     _check(Scenario(H=2, N=700, Q=260, Nc=100, rK=128, rV=64, G=32, C=8), dev, splits=splits)
