@@ -510,8 +510,9 @@ int nkv_attend(void* stream, const nkv_attend_args* args, void* workspace,
  * HIP graph capture, tight serving loops, harnesses that forbid hipMalloc).
  * Same arguments, arithmetic and results as nkv_attend, but the scratch is a
  * static array of NKV_STATIC_SCRATCH_BYTES per GPU inside the library (held
- * until the process ends); a call that needs more (nkv_attend_workspace_size)
- * fails with NKV_ERR_WORKSPACE and launches nothing.  No part of the scratch
+ * until the process ends).  Where nkv_attend_workspace_size exceeds that, the
+ * call takes fewer key splits (the same attention within rounding); if none
+ * fits, it fails with NKV_ERR_WORKSPACE and launches nothing.  No part of the scratch
  * needs to start at zero: every byte a call reads it wrote first (the
  * flash kernel copies no tile the decode left unwritten).  Every call
  * on one GPU shares that GPU's array, so calls that overlap on one GPU (two

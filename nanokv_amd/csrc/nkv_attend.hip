@@ -1015,25 +1015,32 @@ nkv_attend_args narrow_args(const nkv_attend_args* a, const NarrowLayout& L, uns
 // a non-null, aligned stand-in base for the size query
 unsigned char* narrow_placeholder() { return reinterpret_cast<unsigned char*>((uintptr_t)1 << 12); }
 
-int inner_workspace(const nkv_attend_args* a, size_t* need);
+int inner_workspace(const nkv_attend_args* a, size_t limit, size_t* need);
 
-// workspace bytes of a call at any supported D
-int attend_need(const nkv_attend_args* a, size_t* need) {
+// What a limit on a narrow call's workspace leaves its D = 128 call (0: no
+// limit; a limit that the padded operands alone exceed leaves one byte).
+size_t narrow_limit(size_t limit, const NarrowLayout& L) {
+    return limit ? std::max<size_t>(1, limit - std::min(limit, L.inner)) : 0;
+}
+
+// Workspace bytes of a call at any supported D.  limit: the scratch the call
+// will run in, which its key splits are then chosen to fit (0: no limit).
+int attend_need(const nkv_attend_args* a, size_t limit, size_t* need) {
     if (a && a->D != AT_D) {
         int rc = narrow_check(a);
         if (rc) return rc;
         const NarrowLayout L = narrow_layout(a);
         const nkv_attend_args n = narrow_args(a, L, narrow_placeholder());
         size_t inner = 0;
-        rc = inner_workspace(&n, &inner);
+        rc = inner_workspace(&n, narrow_limit(limit, L), &inner);
         if (rc) return rc;
         *need = L.inner + inner;
         return NKV_OK;
     }
-    return inner_workspace(a, need);
+    return inner_workspace(a, limit, need);
 }
 
-int inner_workspace(const nkv_attend_args* a, size_t* need) {
+int inner_workspace(const nkv_attend_args* a, size_t limit, size_t* need) {
     AttendPlan pl;
     int rc = plan_attend(a, &pl);
     if (rc) return rc;
@@ -1043,7 +1050,7 @@ int inner_workspace(const nkv_attend_args* a, size_t* need) {
     if (sch == NKV_SCHEDULE_KEY_CHUNKS) {
         rc = chunk_check(a);
         if (rc) return rc;
-        *need = chunk_workspace_bytes(a);
+        *need = chunk_workspace_bytes(a, limit);
     } else {
         *need = workspace_bytes_for(a, pl);
     }
@@ -1051,9 +1058,10 @@ int inner_workspace(const nkv_attend_args* a, size_t* need) {
 }
 
 int attend_d128(hipStream_t s, const nkv_attend_args* a, void* workspace, size_t workspace_bytes,
-                int out_cols);
+                int out_cols, size_t limit);
 
-int attend_narrow(hipStream_t s, const nkv_attend_args* a, void* workspace, size_t workspace_bytes) {
+int attend_narrow(hipStream_t s, const nkv_attend_args* a, void* workspace, size_t workspace_bytes,
+                  size_t limit) {
     int rc = narrow_check(a);
     if (rc) return rc;
     NKV_REQUIRE(a->B >= 1 && a->H >= 1, NKV_ERR_INVALID, "B and H must be >= 1");
@@ -1078,7 +1086,7 @@ int attend_narrow(hipStream_t s, const nkv_attend_args* a, void* workspace, size
         }
     }
     size_t need = 0;
-    rc = attend_need(a, &need);
+    rc = attend_need(a, limit, &need);
     if (rc) return rc;
     if (a->Q == 0) return NKV_OK;
     NKV_REQUIRE(workspace && workspace_bytes >= need, NKV_ERR_WORKSPACE,
@@ -1121,7 +1129,7 @@ int attend_narrow(hipStream_t s, const nkv_attend_args* a, void* workspace, size
     }
     pad_operands_kernel<<<dim3((unsigned)blocks), 256, 0, s>>>(jobs);
     NKV_LAUNCH_CHECK();
-    rc = attend_d128(s, &n, base + L.inner, workspace_bytes - L.inner, D);
+    rc = attend_d128(s, &n, base + L.inner, workspace_bytes - L.inner, D, narrow_limit(limit, L));
     if (rc || narrow_key_chunks(a)) return rc;
     const int64_t qrows = (int64_t)a->B * a->Q;
     unpad_heads_kernel<<<dim3((unsigned)cdiv(qrows * a->H * (D / 8), 256)), 256, 0, s>>>(
@@ -1135,23 +1143,29 @@ int attend_narrow(hipStream_t s, const nkv_attend_args* a, void* workspace, size
 extern "C" size_t nkv_attend_workspace_size(const nkv_attend_args* a) {
     clear_error();
     size_t need = 0;
-    return attend_need(a, &need) ? 0 : need;
+    return attend_need(a, 0, &need) ? 0 : need;
 }
+
+namespace {
+int attend_any(hipStream_t s, const nkv_attend_args* a, void* workspace, size_t workspace_bytes,
+               size_t limit) {
+    if (a && a->D != AT_D) return attend_narrow(s, a, workspace, workspace_bytes, limit);
+    return attend_d128(s, a, workspace, workspace_bytes, AT_D, limit);
+}
+}  // namespace
 
 extern "C" int nkv_attend(void* stream, const nkv_attend_args* a, void* workspace,
                           size_t workspace_bytes) {
     clear_error();
-    hipStream_t s = (hipStream_t)stream;
-    if (a && a->D != AT_D) return attend_narrow(s, a, workspace, workspace_bytes);
-    return attend_d128(s, a, workspace, workspace_bytes, AT_D);
+    return attend_any((hipStream_t)stream, a, workspace, workspace_bytes, 0);
 }
 
 namespace {
 
 // out_cols: the columns of each output row that the key chunks' merge writes
-// (the query tiles always write all 128).
+// (the query tiles always write all 128); limit: attend_need's.
 int attend_d128(hipStream_t s, const nkv_attend_args* a, void* workspace, size_t workspace_bytes,
-                int out_cols) {
+                int out_cols, size_t limit) {
     AttendPlan pl;
     int rc = plan_attend(a, &pl);
     if (rc) return rc;
@@ -1160,7 +1174,7 @@ int attend_d128(hipStream_t s, const nkv_attend_args* a, void* workspace, size_t
     if (rc) return rc;
     if (a->Q == 0) return NKV_OK;
     if (sch == NKV_SCHEDULE_KEY_CHUNKS)
-        return chunk_attend_launch(s, a, workspace, workspace_bytes, out_cols);
+        return chunk_attend_launch(s, a, workspace, workspace_bytes, out_cols, limit);
     const size_t need = workspace_bytes_for(a, pl);
     NKV_REQUIRE(need == 0 || (workspace && workspace_bytes >= need), NKV_ERR_WORKSPACE,
                 "workspace missing or smaller than nkv_attend_workspace_size()");
@@ -1270,7 +1284,9 @@ int scratch_address(int dev, void** ptr) {
 extern "C" int nkv_attend_static(void* stream, const nkv_attend_args* a) {
     clear_error();
     size_t need = 0;
-    int rc = attend_need(a, &need);
+    // a call keeps within the scratch where fewer key splits allow it
+    const size_t limit = NKV_STATIC_SCRATCH_BYTES;
+    int rc = attend_need(a, limit, &need);
     if (rc) return rc;
     NKV_REQUIRE(need <= (size_t)NKV_STATIC_SCRATCH_BYTES, NKV_ERR_WORKSPACE,
                 "the call needs " + std::to_string(need) + " bytes of scratch; "
@@ -1287,7 +1303,7 @@ extern "C" int nkv_attend_static(void* stream, const nkv_attend_args* a) {
     void* ptr = nullptr;
     rc = scratch_address(dev, &ptr);
     if (rc) return rc;
-    return nkv_attend(stream, a, need ? ptr : nullptr, need);
+    return attend_any((hipStream_t)stream, a, need ? ptr : nullptr, need, limit);
 }
 
 extern "C" int nkv_lse_merge(void* stream, int64_t rows, int D, const uint16_t* a,

@@ -2293,6 +2293,24 @@ int64_t cam_table_bytes(const ChunkLaunchDesc& d) {
     return (int64_t)camera_batches(d.cam, d.B) * d.cam.n_mats * 64 * (int64_t)sizeof(double);
 }
 
+// The workspace areas of a plan whose tiles and key splits are set.
+void plan_layout(const ChunkLaunchDesc* d, int n, MultiPlan& P) {
+    size_t off = 0;
+    for (int i = 0; i < n; ++i) {
+        const FlashPlan& f = P.f[i];
+        P.tiles_off[i] = off;
+        off += align256((size_t)d[i].B * d[i].H * f.ntiles * tile_elems(d[i].dk) * sizeof(uint16_t));
+        P.part_off[i] = off;
+        off += align256((size_t)d[i].B * d[i].H * f.splits * cdiv(d[i].Q, 32) * 32 * PARTIAL_ROW_BYTES);
+    }
+    P.areas_end = off;
+    for (int i = 0; i < n; ++i) {
+        P.cam_off[i] = off;
+        off += align256((size_t)cam_table_bytes(d[i]));
+    }
+    P.total = off;
+}
+
 // Key splits: every split count of every partition gives a candidate block
 // cost; each candidate gives each partition the fewest splits whose blocks
 // stay within it, and the plan with the least modelled time (the makespan,
@@ -2303,7 +2321,8 @@ int64_t cam_table_bytes(const ChunkLaunchDesc& d) {
 // 4 splits on 32 CUs took 22.4 us, 9 on 72 take 13.8; 16 heads, 417 queries,
 // 26 tiles 25.2 and 23.3).  Over 34 calls of at most 24 heads x 2,000 x 500
 // keys and queries, 1.08x as a geometric mean, none more than 2% slower;
-// without the combine's chain in the model 1.07x, one 5% slower.
+// without the combine's chain in the model 1.07x, one 5% slower.  With a
+// workspace limit, split counts whose plan exceeds it are left out.
 void plan_flash(const ChunkLaunchDesc* d, int n, MultiPlan& P) {
     std::vector<double> cand;
     double work[NKV_MAX_PARTS];
@@ -2318,6 +2337,11 @@ void plan_flash(const ChunkLaunchDesc* d, int n, MultiPlan& P) {
     double best = 1e300;
     int64_t best_blocks = 0;
     int best_sp[NKV_MAX_PARTS] = {};
+    auto fits = [&](const int (&sp)[NKV_MAX_PARTS]) {
+        for (int i = 0; i < n; ++i) P.f[i].splits = sp[i];
+        plan_layout(d, n, P);
+        return P.total <= d[0].ws_limit;
+    };
     for (const double c : cand) {
         std::vector<std::pair<double, int64_t>> groups;
         int sp[NKV_MAX_PARTS] = {};
@@ -2335,6 +2359,9 @@ void plan_flash(const ChunkLaunchDesc* d, int n, MultiPlan& P) {
             blocks += nb;
             bytes += 2.0 * (double)d[i].B * d[i].H * sp[i] * cdiv(d[i].Q, 32) * 32 * PARTIAL_ROW_BYTES;
         }
+        // (none within the limit: the first candidate, one split each, stays,
+        // and the caller finds the plan too large)
+        if (d[0].ws_limit && best < 1e300 && !fits(sp)) continue;
         // a head's merge folds in partition 0's splits and one other's
         int folds = sp[0], others = 0;
         for (int i = 1; i < n; ++i) others = std::max(others, sp[i]);
@@ -2508,7 +2535,7 @@ MultiPlan multi_plan(const ChunkLaunchDesc* d, int n) {
     for (int i = 0; i < n; ++i)
         for (int64_t v : {(int64_t)d[i].B, (int64_t)d[i].H, (int64_t)d[i].dk, d[i].Q, d[i].n_rows,
                           d[i].Nc, (int64_t)staged_gemm(d[i]), cam_table_bytes(d[i]),
-                          (int64_t)d[i].key.r, (int64_t)d[i].value.r})
+                          (int64_t)d[i].key.r, (int64_t)d[i].value.r, (int64_t)d[i].ws_limit})
             key.push_back(v);
     thread_local std::vector<int64_t> last_key;
     thread_local MultiPlan last;
@@ -2517,20 +2544,7 @@ MultiPlan multi_plan(const ChunkLaunchDesc* d, int n) {
     P.n = n;
     plan_flash(d, n, P);
     plan_decode(d, n, P);
-    size_t off = 0;
-    for (int i = 0; i < n; ++i) {
-        const FlashPlan& f = P.f[i];
-        P.tiles_off[i] = off;
-        off += align256((size_t)d[i].B * d[i].H * f.ntiles * tile_elems(d[i].dk) * sizeof(uint16_t));
-        P.part_off[i] = off;
-        off += align256((size_t)d[i].B * d[i].H * f.splits * cdiv(d[i].Q, 32) * 32 * PARTIAL_ROW_BYTES);
-    }
-    P.areas_end = off;
-    for (int i = 0; i < n; ++i) {
-        P.cam_off[i] = off;
-        off += align256((size_t)cam_table_bytes(d[i]));
-    }
-    P.total = off;
+    plan_layout(d, n, P);
     last_key = key;
     last = P;
     return P;
@@ -2956,9 +2970,10 @@ int full_desc(const nkv_attend_args* a, ChunkLaunchDesc* d) {
     return NKV_OK;
 }
 
-size_t chunk_workspace_bytes(const nkv_attend_args* a) {
+size_t chunk_workspace_bytes(const nkv_attend_args* a, size_t ws_limit) {
     ChunkLaunchDesc d;
     if (full_desc(a, &d)) return 0;
+    d.ws_limit = ws_limit;
     return chunk_launch_workspace(d);
 }
 
@@ -2982,13 +2997,14 @@ int chunk_check(const nkv_attend_args* a) {
 }
 
 int chunk_attend_launch(hipStream_t s, const nkv_attend_args* a, void* workspace,
-                        size_t workspace_bytes, int out_cols) {
+                        size_t workspace_bytes, int out_cols, size_t ws_limit) {
     int rc = chunk_check(a);
     if (rc) return rc;
     ChunkLaunchDesc d;
     rc = full_desc(a, &d);
     if (rc) return rc;
     d.o_cols = out_cols;
+    d.ws_limit = ws_limit;
     return chunk_launch(s, d, workspace, workspace_bytes);
 }
 

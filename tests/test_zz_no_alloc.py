@@ -50,6 +50,21 @@ def test_static_scratch_matches_nkv_attend_twice(dev):
     assert torch.equal(out.view(torch.int16), r_out.view(torch.int16))
 
 
+def test_static_scratch_takes_fewer_splits(dev):
+    """A call whose plan for a caller's workspace exceeds the scratch by its
+    key splits alone still runs in it, with fewer splits (as do 64-wide heads,
+    whose padded operands take part of it)."""
+    for D, N in ((128, 4352), (64, 4352)):
+        sc = Scenario(H=24, D=D, N=N, Q=256, Nc=0, rK=64, rV=64, G=32, C=4, seed=3)
+        key, value = sc.codecs(dev)
+        need = ops.attend_workspace_size(sc.q, sc.N, sc.Nc, key, value)
+        assert need > _lib.NKV_STATIC_SCRATCH_BYTES, need
+        out, _ = ops.attend_static(sc.q.to(dev), None, None, key, value)
+        ref, _ = sc.reference(0, heads=[0, 23])
+        diff, cos = max_abs_cos(out[0][:, [0, 23]].float().cpu().numpy(), ref)
+        assert diff <= 2e-2 and cos >= 0.9995, (diff, cos)
+
+
 def test_static_scratch_refuses_oversize_calls(dev):
     """A config-1-sized key-chunk call (206 MB of tiles and partials) is refused with
     NKV_ERR_WORKSPACE before anything is launched.  The size query (host
