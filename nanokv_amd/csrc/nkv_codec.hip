@@ -1149,25 +1149,29 @@ __global__ void __launch_bounds__(256) decide_kernel(EncWsBatch W) {
         for (int q = 0; q < NQ; ++q)
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
-                const uint64_t bits = __ballot(256 * q + 4 * lane + e < C && low[q][e] <= U);
+                const uint64_t bits = __ballot(256 * q + 4 * lane + e < C && !(low[q][e] > U));
                 if (bits) first = 256 * q + 4 * (__ffsll((unsigned long long)bits) - 1) + e;
                 cnt += __popcll(bits);
             }
-        // (no candidate only for non-finite rows: index 0 then)
-        id = cnt == 0 ? 0 : first;
-        if (cnt > 1) {
+        // Where a sum overflowed (an infinity, or norms past fp32) the bound is
+        // NaN and the center stays a candidate, so fp64 decides as the search
+        // without a workspace does; a row with a NaN is NaN from every center: 0.
+        const bool nan_row = xsq != xsq;
+        id = nan_row ? 0 : first;
+        if (cnt > 1 && !nan_row) {
             double bd = 0.0;
             int best = -1;
 #pragma unroll
             for (int q = 0; q < NQ; ++q)
 #pragma unroll
                 for (int e = 0; e < 4; ++e) {
-                    uint64_t bits = __ballot(256 * q + 4 * lane + e < C && low[q][e] <= U);
+                    uint64_t bits = __ballot(256 * q + 4 * lane + e < C && !(low[q][e] > U));
                     while (bits) {
                         const int c = 256 * q + 4 * (__ffsll((unsigned long long)bits) - 1) + e;
                         bits &= bits - 1;
                         const double dd = exact_distance<XB>(P, P.centers + (int64_t)c * HD, gr, HD, lane);
-                        if (better(dd, c, bd, best)) { bd = dd; best = c; }
+                        // (a center with a NaN loses to any other)
+                        if (better(dd, c, bd, best) || (bd != bd && dd == dd)) { bd = dd; best = c; }
                     }
                 }
             id = best;

@@ -3,6 +3,7 @@ GEMM) against the same encode without one: ids, coefficients, codes and scales
 bit for bit."""
 import ctypes
 
+import numpy as np
 import pytest
 import torch
 
@@ -87,3 +88,33 @@ def test_workspace_size_and_short_workspace(dev):
                                             ctypes.byref(args)))
     assert not scratch.any()
     assert torch.equal(out["ids"], ops.encode(x, w, centers=c)["ids"])
+
+
+@pytest.mark.parametrize("C", [9, 300, 1024])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_search_of_infinities_and_overflowing_sums(dev, C, dtype):
+    """Rows and centers whose fp32 sums overflow take the center that 64 bits
+    give; a row with a NaN takes center 0."""
+    if dtype == torch.bfloat16 and C > 256:
+        pytest.skip("bf16 rows are searched against at most 256 centers")
+    g = torch.Generator().manual_seed(C)
+    x = torch.randn(70, 256, generator=g)
+    c = torch.randn(C, 256, generator=g).to(torch.bfloat16)
+    c[c == 0] = 1.0                       # no infinity times zero
+    c[2] *= 1e20                          # ||c||^2 overflows fp32
+    x[3, 7] = float("inf")
+    x[4, 9] = float("-inf")
+    x[5, 11] = 3.3e38
+    x[6] *= 1e30
+    x[7, 13] = float("nan")
+    if dtype == torch.float32:
+        x[8, 1] = 3.4e38                  # finite, past the largest bf16
+    x = x.to(dtype)
+    with np.errstate(invalid="ignore"):
+        xd, cd = x.double().numpy(), c.double().numpy()
+        dist = (cd * cd).sum(1)[None] - 2.0 * (xd[:, None, :] * cd[None]).sum(2)
+    want = np.argmin(dist, axis=1)        # the first of equal ones; NaN: 0
+    w = torch.randn(64, 256, generator=g).to(torch.bfloat16).to(dev)
+    got = ops.encode_batch([{"x": x.to(dev), "w_enc": w, "centers": c.to(dev),
+                             "id_dtype": torch.int32}], group=32)[0]["ids"]
+    assert np.array_equal(got.cpu().numpy(), want)
