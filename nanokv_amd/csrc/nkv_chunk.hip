@@ -96,6 +96,7 @@ struct ChunkParams {
     int64_t q_sb, q_st, q_sh;
     const int32_t* q_heads;  // query head of launch head i (null: i), clamped to [0, q_heads_n)
     int q_heads_n;
+    int o_cols;         // columns of each row of out to write (a multiple of 8, at most 128)
     const uint16_t* k_cur;
     int64_t k_sb, k_st, k_sh;
     const uint16_t* v_cur;
@@ -105,7 +106,6 @@ struct ChunkParams {
     float* part_ml;     // [B*H, nch_total, qblocks * 32, 2]: running max (log2 units), row sum
     uint16_t* out;
     int64_t o_sb, o_st, o_sh;
-    int o_cols;         // columns of each output row to write (a multiple of 8, at most 128)
     float* lse;
     RopeDev rope;       // RoPE of the history keys (cs_t null: none)
     CameraDev cam;      // camera P^-1 of the history keys and values (mats null: none)
