@@ -1154,8 +1154,9 @@ __global__ void __launch_bounds__(256) decide_kernel(EncWsBatch W) {
                 cnt += __popcll(bits);
             }
         // Where a sum overflowed (an infinity, or norms past fp32) the bound is
-        // NaN and the center stays a candidate, so fp64 decides as the search
-        // without a workspace does; a row with a NaN is NaN from every center: 0.
+        // NaN and the center stays a candidate, so fp64 decides, as it does in
+        // the search without a workspace above 256 centers (assign_finish, below
+        // that, takes 0); a row with a NaN is NaN from every center: 0.
         const bool nan_row = xsq != xsq;
         id = nan_row ? 0 : first;
         if (cnt > 1 && !nan_row) {
