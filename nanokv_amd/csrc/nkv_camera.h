@@ -49,39 +49,33 @@ __device__ __forceinline__ const float* camera_mats(const CameraDev& c, int b, i
     return c.mats + (int64_t)b * c.mats_bs + (int64_t)m * 64;
 }
 
-// y = bf16(M . x) for one 4-vector, M row-major 4x4 (fp32, used as bf16).
-__device__ __forceinline__ void camera_vec4(const float* M, const float (&x)[4], float (&y)[4]) {
-#pragma clang fp contract(off)
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        double acc = 0.0;
-#pragma unroll
-        for (int j = 0; j < 4; ++j) acc += (double)(bf16_round(M[4 * i + j]) * x[j]);
-        y[i] = bf16_round(f64_to_f32(acc));
-    }
-}
-
-// Output r of camera_vec4: bf16(M[r] . x), M row-major 4x4 (fp32, used as
-// bf16).
-__device__ __forceinline__ float camera_vec4_row(const float* M, int r, const float (&x)[4]) {
-#pragma clang fp contract(off)
+// m . x of a matrix row (entries rounded to bf16, as float or double) and a
+// 4-vector of bf16 values, summed in order from +0 in fp64: the one sum of every
+// camera kernel.  A product of two bf16 values is exact in fp64, so the fused
+// multiply-add rounds as the sum of the products does; in fp32 a product could
+// overflow where the sum does not.
+template <typename T>
+__device__ __forceinline__ float camera_dot(const T* m, const float (&x)[4]) {
     double acc = 0.0;
 #pragma unroll
-    for (int j = 0; j < 4; ++j) acc += (double)(bf16_round(M[4 * r + j]) * x[j]);
-    return bf16_round(f64_to_f32(acc));
+    for (int j = 0; j < 4; ++j) acc = __builtin_fma((double)m[j], (double)x[j], acc);
+    return f64_to_f32(acc);
 }
 
 // y = bf16(m . x) for one 4-vector, m row-major 4x4 already rounded to bf16.
-__device__ __forceinline__ void camera_vec4_rounded(const float (&m)[16], const float (&x)[4],
+template <typename T>
+__device__ __forceinline__ void camera_vec4_rounded(const T (&m)[16], const float (&x)[4],
                                                     float (&y)[4]) {
-#pragma clang fp contract(off)
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        double acc = 0.0;
+    for (int i = 0; i < 4; ++i) y[i] = bf16_round(camera_dot(m + 4 * i, x));
+}
+
+// The same, M row-major 4x4 in memory (fp32, used as bf16).
+__device__ __forceinline__ void camera_vec4(const float* M, const float (&x)[4], float (&y)[4]) {
+    float m[16];
 #pragma unroll
-        for (int j = 0; j < 4; ++j) acc += (double)(m[4 * i + j] * x[j]);
-        y[i] = bf16_round(f64_to_f32(acc));
-    }
+    for (int i = 0; i < 16; ++i) m[i] = bf16_round(M[i]);
+    camera_vec4_rounded(m, x, y);
 }
 
 // The camera transform of one head row of D dims (D == 128 or the SF13

@@ -80,8 +80,7 @@ __global__ void __launch_bounds__(256) camera_apply_kernel(CameraApplyParams p) 
 
 // 16-byte pieces: one thread transforms piece `part` (8 dims, two 4-vectors)
 // of one (b, s) in CA_HEADS heads: the frame's matrices are fetched and rounded
-// once for them, their loads are in flight together.  The products are exact in
-// fp64, so the fused multiply-adds round as camera_vec4's sums do.
+// once for them, their loads are in flight together.
 // INTER: the vectors are the even and the odd dims, one sub-frame (FULL at
 // D = 128); else dims 0..3 and 4..7, each with its own sub-frame or (< 0) left
 // alone (FULL at D = 64, SF13).  1,560 x 24 x 128 (19 MB moved): 7.7 us; one
@@ -113,25 +112,19 @@ __global__ void __launch_bounds__(256) camera_pieces_kernel(CameraApplyParams p,
             m[4 * q + 3] = (double)bf16_round(f.w);
         }
     };
-    // output r of m times the vector v
-    auto out = [&](int r, const double (&v)[4]) {
-        double acc = m[4 * r] * v[0];
-#pragma unroll
-        for (int j = 1; j < 4; ++j) acc = fma(m[4 * r + j], v[j], acc);
-        return f64_to_f32(acc);
-    };
-    auto lo = [](uint32_t x) { return (double)__uint_as_float(x << 16); };
-    auto hi = [](uint32_t x) { return (double)__uint_as_float(x & 0xffff0000u); };
+    auto lo = [](uint32_t x) { return __uint_as_float(x << 16); };
+    auto hi = [](uint32_t x) { return __uint_as_float(x & 0xffff0000u); };
     if constexpr (INTER) {
         matrix(part & 3);
 #pragma unroll
         for (int h = 0; h < CA_HEADS; ++h) {
             if (h0 + h >= p.H) break;
-            double a[4], c[4];
+            float a[4], c[4];
 #pragma unroll
             for (int j = 0; j < 4; ++j) { a[j] = lo(w[h][j]); c[j] = hi(w[h][j]); }
 #pragma unroll
-            for (int r = 0; r < 4; ++r) w[h][r] = pack_bf16x2(out(r, a), out(r, c));
+            for (int r = 0; r < 4; ++r)
+                w[h][r] = pack_bf16x2(camera_dot(m + 4 * r, a), camera_dot(m + 4 * r, c));
         }
     } else {
 #pragma unroll
@@ -143,10 +136,10 @@ __global__ void __launch_bounds__(256) camera_pieces_kernel(CameraApplyParams p,
 #pragma unroll
             for (int h = 0; h < CA_HEADS; ++h) {
                 if (h0 + h >= p.H) break;
-                const double a[4] = {lo(w[h][2 * u]), hi(w[h][2 * u]), lo(w[h][2 * u + 1]),
-                                     hi(w[h][2 * u + 1])};
-                w[h][2 * u] = pack_bf16x2(out(0, a), out(1, a));
-                w[h][2 * u + 1] = pack_bf16x2(out(2, a), out(3, a));
+                const float a[4] = {lo(w[h][2 * u]), hi(w[h][2 * u]), lo(w[h][2 * u + 1]),
+                                    hi(w[h][2 * u + 1])};
+                w[h][2 * u] = pack_bf16x2(camera_dot(m, a), camera_dot(m + 4, a));
+                w[h][2 * u + 1] = pack_bf16x2(camera_dot(m + 8, a), camera_dot(m + 12, a));
             }
         }
     }

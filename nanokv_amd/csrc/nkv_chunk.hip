@@ -1365,18 +1365,13 @@ struct TXformSmem {
     const double* mats[FT_T];     // camera: each key's sub-frame matrices in the fp64 table
 };
 
-// m_row . x for one row of a matrix of the fp64 table (entries rounded to
-// bf16) and a 4-vector x of bf16 values: camera_vec4's sum, in order, in
-// fp64.  Every product of two bf16 values is exact in fp64, so a fused
-// multiply-add rounds exactly as the sum of the product does.
+// bf16(m_row . x) for one row of a matrix of the fp64 table (entries rounded
+// to bf16) and a 4-vector x of bf16 values.
 __device__ __forceinline__ float camera_dot64(const double* m_row, const float (&x)[4]) {
     const f64x2 a = ldg(reinterpret_cast<const f64x2*>(m_row));
     const f64x2 c = ldg(reinterpret_cast<const f64x2*>(m_row) + 1);
-    double acc = a.x * (double)x[0];
-    acc = __builtin_fma(a.y, (double)x[1], acc);
-    acc = __builtin_fma(c.x, (double)x[2], acc);
-    acc = __builtin_fma(c.y, (double)x[3], acc);
-    return bf16_round(f64_to_f32(acc));
+    const double m[4] = {a.x, a.y, c.x, c.y};
+    return bf16_round(camera_dot(m, x));
 }
 
 // Lane q of every quad (lanes 4 a .. 4 a + 4) receives v of lane 4 a + Q.
@@ -1972,14 +1967,7 @@ __device__ __forceinline__ void combine_store(const CombineAcc<ROWS>& A, uint16_
 #pragma unroll
             for (int r = 0; r < 2; ++r)
 #pragma unroll
-                for (int v = 0; v < 2; ++v) {
-                    // camera_vec4's sum for one output, the products exact
-#pragma clang fp contract(off)
-                    double acc = 0.0;
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) acc += (double)(pm[c][r][e] * (v ? x1[e] : x0[e]));
-                    y[r][v] = bf16_round(f64_to_f32(acc));
-                }
+                for (int v = 0; v < 2; ++v) y[r][v] = camera_dot(pm[c][r], v ? x1 : x0);
             pk = {pack_bf16x2(y[0][0], y[0][1]), pack_bf16x2(y[1][0], y[1][1])};
         }
         *reinterpret_cast<u32x2*>(orow + d) = pk;

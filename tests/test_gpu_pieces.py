@@ -2,10 +2,12 @@
 nkv_lift_lse_combine against the element-wise ones, which misaligned operands
 still take: RoPE and the camera bit for bit, the lift (fp32 sums in another
 order) to one bf16 rounding."""
+import numpy as np
 import pytest
 import torch
 
 from nanokv_amd import ops, synth
+from oracle import oracle as orc
 from tests._helpers import u16
 
 pytestmark = pytest.mark.gpu
@@ -51,6 +53,36 @@ def test_camera_pieces(dev, layout, D, B, S, H):
     _same(ops.camera_apply(x, cam), ops.camera_apply(_shift(x), cam, out=_shift(x)))
     y = x.clone()
     _same(ops.camera_apply(y, cam, out=y), ops.camera_apply(x, cam))
+
+
+@pytest.mark.parametrize("layout,D", [("full", 128), ("full", 64), ("sf13", 128)])
+def test_camera_pieces_at_the_limits(dev, layout, D):
+    """Products past fp32's range and below it, sums that cancel, zeros of both
+    signs against negative entries: the element-wise kernel's bits, and the
+    oracle's sum in 64 bits."""
+    g = torch.Generator().manual_seed(D)
+    x = torch.randn(1, 12, 9, D, generator=g)
+    x[0, 0] = 0.0
+    x[0, 1] = -0.0
+    x[0, 2] = 3e38 * x[0, 2].sign()
+    x[0, 3] = 3e38
+    x[0, 4] *= 1e-30
+    x[0, 5, :, ::3] = 3e38
+    P = torch.randn(1, 3, 4, 4, 4, generator=g) * 2
+    P[0, 0] = -P[0, 0].abs()
+    P[0, 1, :, :, ::2] = 4.0                 # 4 x - 4 x of equal values past fp32
+    P[0, 1, :, :, 1::2] = -4.0
+    P[0, 2] *= 1e-12
+    cam = ops.Camera(P.to(dev), torch.tensor([0, 1, 2], dtype=torch.int32, device=dev), 1, layout)
+    x = x.to(torch.bfloat16).to(dev)
+    rows = torch.arange(12, dtype=torch.int32, device=dev)
+    for shift in range(3):                   # every row meets every matrix
+        r = (rows + shift) % 3
+        got = ops.camera_apply(x, cam, rows=r)
+        _same(got, ops.camera_apply(_shift(x), cam, rows=r, out=_shift(x)))
+        with np.errstate(over="ignore"):      # past the largest fp32: an infinity, as on the GPU
+            ref = orc.camera_apply(u16(x[0]), P[0, r.cpu().long()].numpy(), layout)
+        assert np.array_equal(orc.bf16_to_f32(ref), got[0].float().cpu().numpy(), equal_nan=True)
 
 
 @pytest.mark.parametrize("low", [32, 64, 96])
