@@ -320,8 +320,7 @@ typedef struct nkv_encode_args {
     int64_t x_stride;             /* elements between rows of x / x_bf16; 0 = HD */
     /* scratch of nkv_encode_workspace_size() bytes, 16-byte aligned, or NULL:
      * with it the search and the projection run as plain GEMMs over the chip
-     * (same results for finite rows whose squares sum within fp32; past that
-     * fp64 decides; in a batch the first problem's is used) */
+     * (same results; in a batch the first problem's is used) */
     void* workspace;
     size_t workspace_bytes;
 } nkv_encode_args;

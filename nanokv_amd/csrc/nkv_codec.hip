@@ -567,14 +567,14 @@ __device__ __forceinline__ void assign_finish(const EncBatch& B, const EncProb& 
         if (l32 == 0) sm.red[wave][8 * (i / 4) + 4 * hf + (i % 4)] = u;
     }
     __syncthreads();
-    // candidates: dt - E <= U
+    // candidates: those not above U
 #pragma unroll
     for (int i = 0; i < 16; ++i) {
         const int r = 8 * (i / 4) + 4 * hf + (i % 4);
         float U = sm.red[0][r];
 #pragma unroll
         for (int w = 1; w < AB_WAVES; ++w) U = fminf(U, sm.red[w][r]);
-        if (col < C && dt[i] - ee[i] <= U) {
+        if (col < C && !(dt[i] - ee[i] > U)) {
             atomicAdd(&sm.cnt[r], 1);
             atomicMin(&sm.first[r], col);
             atomicOr(&sm.cand[r][col >> 5], 1u << (col & 31));
@@ -584,9 +584,12 @@ __device__ __forceinline__ void assign_finish(const EncBatch& B, const EncProb& 
     for (int r = wave; r < AB_ROWS; r += AB_WAVES) {
         const int64_t gr = row0 + r;
         if (gr >= rows) continue;
-        // (no candidate only for non-finite rows: index 0 then)
-        int best = sm.cnt[r] == 0 ? 0 : sm.first[r];
-        if (sm.cnt[r] > 1) {
+        // Where a sum overflowed (an infinity, or norms past fp32) the bound is
+        // NaN and the center stays a candidate, so fp64 decides; a row with a
+        // NaN is NaN from every center: 0.
+        const bool nan_row = sm.xn[r] != sm.xn[r];
+        int best = nan_row ? 0 : sm.first[r];
+        if (sm.cnt[r] > 1 && !nan_row) {
             double bd = 0.0;
             best = -1;
             for (int w = 0; w < AB_MAXC / 32; ++w) {
@@ -595,7 +598,8 @@ __device__ __forceinline__ void assign_finish(const EncBatch& B, const EncProb& 
                     const int c = 32 * w + __builtin_ctz(bits);
                     bits &= bits - 1;
                     const double d = exact_distance<XB>(P, P.centers + (int64_t)c * HD, gr, HD, lane);
-                    if (best < 0 || d < bd) { bd = d; best = c; }  // ascending c: first index on ties
+                    // (a center with a NaN loses to any other)
+                    if (better(d, c, bd, best) || (bd != bd && d == d)) { bd = d; best = c; }
                 }
             }
         }
@@ -1153,10 +1157,7 @@ __global__ void __launch_bounds__(256) decide_kernel(EncWsBatch W) {
                 if (bits) first = 256 * q + 4 * (__ffsll((unsigned long long)bits) - 1) + e;
                 cnt += __popcll(bits);
             }
-        // Where a sum overflowed (an infinity, or norms past fp32) the bound is
-        // NaN and the center stays a candidate, so fp64 decides, as it does in
-        // the search without a workspace above 256 centers (assign_finish, below
-        // that, takes 0); a row with a NaN is NaN from every center: 0.
+        // (overflowed sums and NaN: see assign_finish)
         const bool nan_row = xsq != xsq;
         id = nan_row ? 0 : first;
         if (cnt > 1 && !nan_row) {
@@ -1171,7 +1172,6 @@ __global__ void __launch_bounds__(256) decide_kernel(EncWsBatch W) {
                         const int c = 256 * q + 4 * (__ffsll((unsigned long long)bits) - 1) + e;
                         bits &= bits - 1;
                         const double dd = exact_distance<XB>(P, P.centers + (int64_t)c * HD, gr, HD, lane);
-                        // (a center with a NaN loses to any other)
                         if (better(dd, c, bd, best) || (bd != bd && dd == dd)) { bd = dd; best = c; }
                     }
                 }

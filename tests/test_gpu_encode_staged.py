@@ -94,7 +94,8 @@ def test_workspace_size_and_short_workspace(dev):
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 def test_search_of_infinities_and_overflowing_sums(dev, C, dtype):
     """Rows and centers whose fp32 sums overflow take the center that 64 bits
-    give; a row with a NaN takes center 0."""
+    give; a row with a NaN takes center 0: with a workspace, without one and
+    in nkv_assign."""
     if dtype == torch.bfloat16 and C > 256:
         pytest.skip("bf16 rows are searched against at most 256 centers")
     g = torch.Generator().manual_seed(C)
@@ -115,6 +116,10 @@ def test_search_of_infinities_and_overflowing_sums(dev, C, dtype):
         dist = (cd * cd).sum(1)[None] - 2.0 * (xd[:, None, :] * cd[None]).sum(2)
     want = np.argmin(dist, axis=1)        # the first of equal ones; NaN: 0
     w = torch.randn(64, 256, generator=g).to(torch.bfloat16).to(dev)
-    got = ops.encode_batch([{"x": x.to(dev), "w_enc": w, "centers": c.to(dev),
-                             "id_dtype": torch.int32}], group=32)[0]["ids"]
+    problem = {"x": x.to(dev), "w_enc": w, "centers": c.to(dev), "id_dtype": torch.int32}
+    got = ops.encode_batch([problem], group=32)[0]["ids"]
     assert np.array_equal(got.cpu().numpy(), want)
+    plain = _plain([problem], group=32, scale_dtype=torch.float16, quant_mode="fp32")[0]["ids"]
+    assert np.array_equal(plain.cpu().numpy(), want)
+    if dtype == torch.float32:
+        assert np.array_equal(ops.assign(problem["x"], problem["centers"], torch.int32).cpu().numpy(), want)
