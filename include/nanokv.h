@@ -498,7 +498,10 @@ typedef struct nkv_attend_args {
     int cur_mask_words;           /* >= ceil(Nc / 32) */
 } nkv_attend_args;
 
-/* Bytes of workspace nkv_attend needs for these arguments (0 if none). */
+/* Bytes of workspace nkv_attend wants for these arguments (0 if none).  In a
+ * smaller one the staged schedule takes fewer key splits (the same attention
+ * within rounding); if none fits, the call fails with NKV_ERR_WORKSPACE and
+ * launches nothing. */
 size_t nkv_attend_workspace_size(const nkv_attend_args* args);
 
 int nkv_attend(void* stream, const nkv_attend_args* args, void* workspace,
@@ -622,7 +625,8 @@ typedef struct nkv_fast_args {
     const nkv_camera* o_camera;
 } nkv_fast_args;
 
-/* Bytes of workspace nkv_fast_attend needs for these arguments. */
+/* Bytes of workspace nkv_fast_attend wants for these arguments (in a smaller
+ * one: as nkv_attend_workspace_size). */
 size_t nkv_fast_attend_workspace_size(const nkv_fast_args* args);
 
 int nkv_fast_attend(void* stream, const nkv_fast_args* args, void* workspace,

@@ -1058,10 +1058,9 @@ int inner_workspace(const nkv_attend_args* a, size_t limit, size_t* need) {
 }
 
 int attend_d128(hipStream_t s, const nkv_attend_args* a, void* workspace, size_t workspace_bytes,
-                int out_cols, size_t limit);
+                int out_cols);
 
-int attend_narrow(hipStream_t s, const nkv_attend_args* a, void* workspace, size_t workspace_bytes,
-                  size_t limit) {
+int attend_narrow(hipStream_t s, const nkv_attend_args* a, void* workspace, size_t workspace_bytes) {
     int rc = narrow_check(a);
     if (rc) return rc;
     NKV_REQUIRE(a->B >= 1 && a->H >= 1, NKV_ERR_INVALID, "B and H must be >= 1");
@@ -1086,7 +1085,7 @@ int attend_narrow(hipStream_t s, const nkv_attend_args* a, void* workspace, size
         }
     }
     size_t need = 0;
-    rc = attend_need(a, limit, &need);
+    rc = attend_need(a, workspace_bytes, &need);
     if (rc) return rc;
     if (a->Q == 0) return NKV_OK;
     NKV_REQUIRE(workspace && workspace_bytes >= need, NKV_ERR_WORKSPACE,
@@ -1129,7 +1128,7 @@ int attend_narrow(hipStream_t s, const nkv_attend_args* a, void* workspace, size
     }
     pad_operands_kernel<<<dim3((unsigned)blocks), 256, 0, s>>>(jobs);
     NKV_LAUNCH_CHECK();
-    rc = attend_d128(s, &n, base + L.inner, workspace_bytes - L.inner, D, narrow_limit(limit, L));
+    rc = attend_d128(s, &n, base + L.inner, workspace_bytes - L.inner, D);
     if (rc || narrow_key_chunks(a)) return rc;
     const int64_t qrows = (int64_t)a->B * a->Q;
     unpad_heads_kernel<<<dim3((unsigned)cdiv(qrows * a->H * (D / 8), 256)), 256, 0, s>>>(
@@ -1146,26 +1145,20 @@ extern "C" size_t nkv_attend_workspace_size(const nkv_attend_args* a) {
     return attend_need(a, 0, &need) ? 0 : need;
 }
 
-namespace {
-int attend_any(hipStream_t s, const nkv_attend_args* a, void* workspace, size_t workspace_bytes,
-               size_t limit) {
-    if (a && a->D != AT_D) return attend_narrow(s, a, workspace, workspace_bytes, limit);
-    return attend_d128(s, a, workspace, workspace_bytes, AT_D, limit);
-}
-}  // namespace
-
 extern "C" int nkv_attend(void* stream, const nkv_attend_args* a, void* workspace,
                           size_t workspace_bytes) {
     clear_error();
-    return attend_any((hipStream_t)stream, a, workspace, workspace_bytes, 0);
+    hipStream_t s = (hipStream_t)stream;
+    if (a && a->D != AT_D) return attend_narrow(s, a, workspace, workspace_bytes);
+    return attend_d128(s, a, workspace, workspace_bytes, AT_D);
 }
 
 namespace {
 
 // out_cols: the columns of each output row that the key chunks' merge writes
-// (the query tiles always write all 128); limit: attend_need's.
+// (the query tiles always write all 128).
 int attend_d128(hipStream_t s, const nkv_attend_args* a, void* workspace, size_t workspace_bytes,
-                int out_cols, size_t limit) {
+                int out_cols) {
     AttendPlan pl;
     int rc = plan_attend(a, &pl);
     if (rc) return rc;
@@ -1174,7 +1167,7 @@ int attend_d128(hipStream_t s, const nkv_attend_args* a, void* workspace, size_t
     if (rc) return rc;
     if (a->Q == 0) return NKV_OK;
     if (sch == NKV_SCHEDULE_KEY_CHUNKS)
-        return chunk_attend_launch(s, a, workspace, workspace_bytes, out_cols, limit);
+        return chunk_attend_launch(s, a, workspace, workspace_bytes, out_cols);
     const size_t need = workspace_bytes_for(a, pl);
     NKV_REQUIRE(need == 0 || (workspace && workspace_bytes >= need), NKV_ERR_WORKSPACE,
                 "workspace missing or smaller than nkv_attend_workspace_size()");
@@ -1285,8 +1278,7 @@ extern "C" int nkv_attend_static(void* stream, const nkv_attend_args* a) {
     clear_error();
     size_t need = 0;
     // a call keeps within the scratch where fewer key splits allow it
-    const size_t limit = NKV_STATIC_SCRATCH_BYTES;
-    int rc = attend_need(a, limit, &need);
+    int rc = attend_need(a, NKV_STATIC_SCRATCH_BYTES, &need);
     if (rc) return rc;
     NKV_REQUIRE(need <= (size_t)NKV_STATIC_SCRATCH_BYTES, NKV_ERR_WORKSPACE,
                 "the call needs " + std::to_string(need) + " bytes of scratch; "
@@ -1303,7 +1295,7 @@ extern "C" int nkv_attend_static(void* stream, const nkv_attend_args* a) {
     void* ptr = nullptr;
     rc = scratch_address(dev, &ptr);
     if (rc) return rc;
-    return attend_any((hipStream_t)stream, a, need ? ptr : nullptr, need, limit);
+    return nkv_attend(stream, a, ptr, NKV_STATIC_SCRATCH_BYTES);
 }
 
 extern "C" int nkv_lse_merge(void* stream, int64_t rows, int D, const uint16_t* a,

@@ -2310,8 +2310,9 @@ void plan_layout(const ChunkLaunchDesc* d, int n, MultiPlan& P) {
 // 26 tiles 25.2 and 23.3).  Over 34 calls of at most 24 heads x 2,000 x 500
 // keys and queries, 1.08x as a geometric mean, none more than 2% slower;
 // without the combine's chain in the model 1.07x, one 5% slower.  With a
-// workspace limit, split counts whose plan exceeds it are left out.
-void plan_flash(const ChunkLaunchDesc* d, int n, MultiPlan& P) {
+// workspace limit (not 0), split counts whose plan exceeds it are left out; if
+// all do, one split each remains, and the caller finds that plan too large.
+void plan_flash(const ChunkLaunchDesc* d, int n, size_t limit, MultiPlan& P) {
     std::vector<double> cand;
     double work[NKV_MAX_PARTS];
     int smax[NKV_MAX_PARTS];
@@ -2325,10 +2326,11 @@ void plan_flash(const ChunkLaunchDesc* d, int n, MultiPlan& P) {
     double best = 1e300;
     int64_t best_blocks = 0;
     int best_sp[NKV_MAX_PARTS] = {};
+    for (int i = 0; i < n; ++i) best_sp[i] = P.f[i].ntiles > 0 ? 1 : 0;
     auto fits = [&](const int (&sp)[NKV_MAX_PARTS]) {
         for (int i = 0; i < n; ++i) P.f[i].splits = sp[i];
         plan_layout(d, n, P);
-        return P.total <= d[0].ws_limit;
+        return P.total <= limit;
     };
     for (const double c : cand) {
         std::vector<std::pair<double, int64_t>> groups;
@@ -2347,9 +2349,7 @@ void plan_flash(const ChunkLaunchDesc* d, int n, MultiPlan& P) {
             blocks += nb;
             bytes += 2.0 * (double)d[i].B * d[i].H * sp[i] * cdiv(d[i].Q, 32) * 32 * PARTIAL_ROW_BYTES;
         }
-        // (none within the limit: the first candidate, one split each, stays,
-        // and the caller finds the plan too large)
-        if (d[0].ws_limit && best < 1e300 && !fits(sp)) continue;
+        if (limit && !fits(sp)) continue;
         // a head's merge folds in partition 0's splits and one other's
         int folds = sp[0], others = 0;
         for (int i = 1; i < n; ++i) others = std::max(others, sp[i]);
@@ -2517,25 +2517,38 @@ bool plan_extents_ok(const MultiPlan& P, const ChunkLaunchDesc* d, int n, int v_
 }
 
 // The plan depends on the partitions' shapes and codec ranks alone; the last
-// one is kept (a layer loop repeats the same shapes).
+// one is kept (a layer loop repeats the same shapes), and beside it the last
+// one that had to fit a smaller workspace.
 MultiPlan multi_plan(const ChunkLaunchDesc* d, int n) {
     std::vector<int64_t> key{n};
     for (int i = 0; i < n; ++i)
         for (int64_t v : {(int64_t)d[i].B, (int64_t)d[i].H, (int64_t)d[i].dk, d[i].Q, d[i].n_rows,
                           d[i].Nc, (int64_t)staged_gemm(d[i]), cam_table_bytes(d[i]),
-                          (int64_t)d[i].key.r, (int64_t)d[i].value.r, (int64_t)d[i].ws_limit})
+                          (int64_t)d[i].key.r, (int64_t)d[i].value.r})
             key.push_back(v);
     thread_local std::vector<int64_t> last_key;
-    thread_local MultiPlan last;
-    if (key == last_key) return last;
-    MultiPlan P{};
-    P.n = n;
-    plan_flash(d, n, P);
-    plan_decode(d, n, P);
-    plan_layout(d, n, P);
-    last_key = key;
-    last = P;
-    return P;
+    thread_local MultiPlan last, small;
+    thread_local size_t small_limit = 0;
+    auto plan = [&](size_t limit) {
+        MultiPlan P{};
+        P.n = n;
+        plan_flash(d, n, limit, P);
+        plan_decode(d, n, P);
+        plan_layout(d, n, P);
+        return P;
+    };
+    if (key != last_key) {
+        last = plan(0);
+        last_key = key;
+        small_limit = 0;
+    }
+    const size_t limit = d[0].ws_limit;
+    if (limit == 0 || last.total <= limit) return last;
+    if (small_limit != limit) {
+        small = plan(limit);
+        small_limit = limit;
+    }
+    return small;
 }
 
 template <int KQ>
@@ -2985,14 +2998,14 @@ int chunk_check(const nkv_attend_args* a) {
 }
 
 int chunk_attend_launch(hipStream_t s, const nkv_attend_args* a, void* workspace,
-                        size_t workspace_bytes, int out_cols, size_t ws_limit) {
+                        size_t workspace_bytes, int out_cols) {
     int rc = chunk_check(a);
     if (rc) return rc;
     ChunkLaunchDesc d;
     rc = full_desc(a, &d);
     if (rc) return rc;
     d.o_cols = out_cols;
-    d.ws_limit = ws_limit;
+    d.ws_limit = workspace_bytes;
     return chunk_launch(s, d, workspace, workspace_bytes);
 }
 
@@ -3004,7 +3017,8 @@ int chunk_attend_launch(hipStream_t s, const nkv_attend_args* a, void* workspace
 // write against the plan (v_dk != 0 addresses the V^T images at that width,
 // to show that a layout mismatch is caught).  Host arithmetic only: it runs
 // without a GPU.  Returns NKV_OK, or NKV_ERR_INVALID with the violation in
-// nkv_last_error; *total receives the plan's workspace bytes.
+// nkv_last_error; *total receives the plan's workspace bytes (on entry the
+// workspace it shall fit, or 0).
 extern "C" int nkv_plan_check(const int64_t* shapes, int n, int v_dk, size_t* total) {
     using namespace nkv;
     clear_error();
@@ -3031,6 +3045,7 @@ extern "C" int nkv_plan_check(const int64_t* shapes, int n, int v_dk, size_t* to
         NKV_REQUIRE(use_staged(d[i]), NKV_ERR_INVALID,
                     "partition " + std::to_string(i) + " is not staged");
     }
+    d[0].ws_limit = total ? *total : 0;
     const MultiPlan P = multi_plan(d, n);
     if (total) *total = P.total;
     std::string why;

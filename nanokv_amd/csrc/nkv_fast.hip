@@ -310,6 +310,7 @@ struct FastLayout {
     size_t lse_n;                  // [B, H, Q] f32
     std::vector<size_t> q_low, kc, vc, kb, vb, out_l, lse_l;  // per group
     size_t partials;
+    size_t limit;                  // ChunkLaunchDesc::ws_limit of every launch
     size_t total;
 };
 
@@ -618,6 +619,7 @@ int multi_descs(const nkv_fast_args* f, unsigned char* ws, const FastLayout& L,
                 ChunkLaunchDesc* d, const int32_t** heads) {
     d[0] = native_desc(f, f->attend.lse);
     add_transforms(f, nullptr, d[0]);
+    d[0].ws_limit = L.limit;
     heads[0] = nullptr;
     for (int g = 0; g < f->num_groups; ++g) {
         d[1 + g] = low_desc(f, g, ws, L, true);
@@ -643,7 +645,9 @@ bool use_multi(const nkv_fast_args* f) {
     return staged_multi_supported(d, n);
 }
 
-FastLayout layout(const nkv_fast_args* f) {
+// ws_bytes: the caller's workspace, which the launches' key splits are chosen to
+// fit where they can (0: no limit).
+FastLayout layout(const nkv_fast_args* f, size_t ws_bytes) {
     const nkv_attend_args& a = f->attend;
     FastLayout L;
     L.multi = use_multi(f);
@@ -668,6 +672,10 @@ FastLayout layout(const nkv_fast_args* f) {
         L.out_l.push_back(take(L.multi ? 0 : (size_t)a.B * a.Q * nh * D * 2));
         L.lse_l.push_back(take(L.multi ? 0 : (size_t)a.B * nh * a.Q * sizeof(float)));
     }
+    // what the workspace leaves for the partials (nothing: one byte, which no
+    // plan fits)
+    L.limit = 0;
+    if (ws_bytes) L.limit = std::max<size_t>(1, (ws_bytes - std::min(ws_bytes, off)) & ~(size_t)255);
     size_t part;
     if (L.multi) {
         ChunkLaunchDesc d[NKV_MAX_PARTS];
@@ -677,10 +685,12 @@ FastLayout layout(const nkv_fast_args* f) {
     } else {
         ChunkLaunchDesc nd = native_desc(f, nullptr);
         add_transforms(f, nullptr, nd);
+        nd.ws_limit = L.limit;
         part = chunk_launch_workspace(nd);
         for (int g = 0; g < f->num_groups; ++g) {
             ChunkLaunchDesc ld = low_desc(f, g, nullptr, L);
             add_transforms(f, &f->groups[g], ld);
+            ld.ws_limit = L.limit;
             part = std::max(part, chunk_launch_workspace(ld));
         }
     }
@@ -821,7 +831,7 @@ using namespace nkv;
 extern "C" size_t nkv_fast_attend_workspace_size(const nkv_fast_args* f) {
     clear_error();
     if (validate(f)) return 0;
-    return layout(f).total;
+    return layout(f, 0).total;
 }
 
 extern "C" int nkv_fast_attend(void* stream, const nkv_fast_args* f, void* workspace,
@@ -832,7 +842,7 @@ extern "C" int nkv_fast_attend(void* stream, const nkv_fast_args* f, void* works
     const nkv_attend_args& a = f->attend;
     if (a.Q == 0) return NKV_OK;
     hipStream_t s = (hipStream_t)stream;
-    const FastLayout L = layout(f);
+    const FastLayout L = layout(f, workspace_bytes);
     NKV_REQUIRE(workspace && workspace_bytes >= L.total, NKV_ERR_WORKSPACE,
                 "workspace missing or smaller than nkv_fast_attend_workspace_size()");
     unsigned char* ws = reinterpret_cast<unsigned char*>(workspace);
@@ -877,6 +887,7 @@ extern "C" int nkv_fast_attend(void* stream, const nkv_fast_args* f, void* works
     // 1. native partition -> out, lse_n
     ChunkLaunchDesc nd = native_desc(f, lse_n);
     add_transforms(f, nullptr, nd);
+    nd.ws_limit = L.limit;
     rc = chunk_launch(s, nd, ws + L.partials, part_bytes);
     if (rc) return rc;
     // no low rows: the native partition is the whole attention
@@ -895,6 +906,7 @@ extern "C" int nkv_fast_attend(void* stream, const nkv_fast_args* f, void* works
         const int nh = G.num_heads, D = a.D;
         ChunkLaunchDesc ld = low_desc(f, g, ws, L);
         add_transforms(f, &G, ld);
+        ld.ws_limit = L.limit;
         rc = chunk_launch(s, ld, ws + L.partials, part_bytes);
         if (rc) return rc;
         const int64_t threads = (int64_t)a.B * a.Q * nh * (D / 8);

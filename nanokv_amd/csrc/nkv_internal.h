@@ -133,8 +133,8 @@ struct ChunkLaunchDesc {
     const uint32_t* cur_mask;
     const int32_t* q_group;
     int n_groups, mask_words;
-    // the staged plan stays within this many workspace bytes if any of its
-    // key splits does (0: no limit)
+    // workspace bytes: the staged plan stays within them if any choice of key
+    // splits does (0: no limit; the first partition's counts)
     size_t ws_limit;
 };
 
@@ -154,11 +154,11 @@ int check_segments(const nkv_codec& c, int64_t N);
 
 // Key-chunk schedule (nkv_chunk.hip).
 int chunk_check(const nkv_attend_args* a);
-// ws_limit: ChunkLaunchDesc's; out_cols: columns of each output row to write
-// (0: all 128).
+// ws_limit: ChunkLaunchDesc's (the launch takes workspace_bytes for it);
+// out_cols: columns of each output row to write (0: all 128).
 size_t chunk_workspace_bytes(const nkv_attend_args* a, size_t ws_limit);
 int chunk_attend_launch(hipStream_t s, const nkv_attend_args* a, void* workspace,
-                        size_t workspace_bytes, int out_cols, size_t ws_limit);
+                        size_t workspace_bytes, int out_cols);
 size_t chunk_launch_workspace(const ChunkLaunchDesc& d);
 int chunk_launch(hipStream_t s, const ChunkLaunchDesc& d, void* workspace, size_t workspace_bytes);
 

@@ -20,7 +20,7 @@ import pytest
 from nanokv_amd import _lib
 
 
-def _check(parts, v_dk=0):
+def _check(parts, v_dk=0, limit=0):
     lib = _lib.lib()
     fn = lib.nkv_plan_check
     fn.argtypes = [ctypes.POINTER(ctypes.c_int64), ctypes.c_int, ctypes.c_int,
@@ -28,7 +28,7 @@ def _check(parts, v_dk=0):
     fn.restype = ctypes.c_int
     flat = [v for p in parts for v in p]
     arr = (ctypes.c_int64 * len(flat))(*flat)
-    total = ctypes.c_size_t(0)
+    total = ctypes.c_size_t(limit)
     rc = fn(arr, len(parts), v_dk, ctypes.byref(total))
     return rc, lib.nkv_last_error().decode(), total.value
 
@@ -103,3 +103,30 @@ def test_unstaged_partitions_are_refused():
 def test_decode_block_plan(B, H, n_rows, Nc, rK, rV):
     rc, err, _ = _check([(B, H, 128, 1024, n_rows, Nc, rK, rV, 0)])
     assert rc == _lib.NKV_OK, err
+
+
+@pytest.mark.parametrize("parts", [
+    [(1, 8, 128, 256, 2048, 256, 64, 64, 0)],         # many splits of few tiles
+    [CFG1],
+    # one short partition before a long one: the first candidate splits are
+    # neither the fewest nor always the ones that fit
+    [(1, 4, 128, 300, 200, 60, 384, 384, 0), (1, 4, 64, 300, 4000, 0, 384, 384, 0)],
+    [CFG3_NATIVE, (1, 6, 128, 1560, 9360, 0, 384, 384, 0),
+     (1, 6, 32, 1560, 9360, 0, 384, 384, 0), (1, 12, 64, 1560, 9360, 0, 384, 384, 0)],
+])
+def test_plan_fits_a_smaller_workspace(parts):
+    """Fewer splits down to one each; below that the least plan, which the
+    caller refuses."""
+    full = _check(parts)[2]
+    least = _check(parts, limit=1)[2]
+    areas = [p[0] * p[1] * -(-p[3] // 32) * 32 * (128 * 2 + 8) for p in parts]
+    assert least == sum(_tiles(p[1], p[2], p[4], p[5], p[0]) for p in parts) + \
+        sum(-(-a // 256) * 256 for a in areas)
+    assert full > least
+    for limit in (least, least + 1, (least + full) // 2, full - 1):
+        rc, err, total = _check(parts, limit=limit)
+        assert rc == _lib.NKV_OK, err
+        assert least <= total <= limit
+    for limit in (full, full + 1, 1 << 40, 0):
+        assert _check(parts, limit=limit)[2] == full
+    assert _check(parts, limit=least - 1)[2] == least
