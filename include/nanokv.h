@@ -353,6 +353,8 @@ int nkv_encode_batch(void* stream, const nkv_encode_args* args, int n);
  * keeps its value.  labels are the last round's (zero for 0 rounds).
  *   x [B, S, HD] fp32; centers out [B, C, HD] fp32; labels out [B, S] int32;
  *   1 <= C <= min(S, 256).
+ * A workspace of 4 B S bytes, rounded up to 256, is enough for fp32 rows; with
+ * less than nkv_c64_fit_workspace_size() the search is slower.
  */
 size_t nkv_c64_fit_workspace_size(int B, int64_t S, int C);
 int nkv_c64_fit(void* stream, const float* x, int B, int64_t S, int HD, int C, int iterations,

@@ -2471,6 +2471,9 @@ static size_t fit_part_bytes(int B, int64_t S, int C, size_t elem) {
     return fit_ws_align((size_t)cdiv(C, FS_CENT) * B * S * elem);
 }
 
+// What the search by whole rows needs.
+static size_t fit_label_bytes(int B, int64_t S) { return fit_ws_align((size_t)B * S * sizeof(int32_t)); }
+
 extern "C" size_t nkv_c64_fit_workspace_size(int B, int64_t S, int C) {
     if (B <= 0 || S <= 0 || C <= 0) return 0;
     return fit_part_bytes(B, S, C, sizeof(double)) + fit_part_bytes(B, S, C, sizeof(int32_t));
@@ -2508,23 +2511,25 @@ extern "C" int nkv_c64_fit_rows(void* stream, const nkv_c64_fit_args* a) {
     NKV_REQUIRE((a->x || a->x_bf16) && (a->init_rows || a->init_rows_host) && a->centers && a->labels,
                 NKV_ERR_INVALID, "null pointer");
     NKV_REQUIRE(!(a->x && a->x_bf16), NKV_ERR_INVALID, "give x or x_bf16, not both");
-    const size_t need = nkv_c64_fit_workspace_size(B, S, C);
-    NKV_REQUIRE(a->workspace && a->workspace_bytes >= need, NKV_ERR_WORKSPACE,
-                "workspace missing or smaller than nkv_c64_fit_workspace_size()");
     const bool xb = a->x_bf16 != nullptr;
     const void* x = xb ? (const void*)a->x_bf16 : (const void*)a->x;
-    // the fp64 MFMA search: whole 32-wide steps, 16-byte rows
-    const bool mfma = HD % 32 == 0 && reinterpret_cast<uintptr_t>(x) % 16 == 0 &&
-                      reinterpret_cast<uintptr_t>(a->centers) % 16 == 0 && B <= 65535 &&
-                      reinterpret_cast<uintptr_t>(a->workspace) % 8 == 0;
-    const bool rounds = a->iterations > 0;
-    NKV_REQUIRE(!xb || (mfma && rounds), NKV_ERR_UNSUPPORTED,
+    // the fp64 MFMA search: whole 32-wide steps, 16-byte rows; a workspace too
+    // small for its partial results takes the search by whole rows, which keeps
+    // their labels alone (fp32 rows)
+    const bool fits = a->workspace_bytes >= nkv_c64_fit_workspace_size(B, S, C);
+    const bool steps = HD % 32 == 0 && reinterpret_cast<uintptr_t>(x) % 16 == 0 &&
+                       reinterpret_cast<uintptr_t>(a->centers) % 16 == 0 && B <= 65535 &&
+                       reinterpret_cast<uintptr_t>(a->workspace) % 8 == 0;
+    const bool mfma = steps && fits, rounds = a->iterations > 0;
+    NKV_REQUIRE(a->workspace && (fits || (!xb && a->workspace_bytes >= fit_label_bytes(B, S))),
+                NKV_ERR_WORKSPACE, "workspace missing or smaller than nkv_c64_fit_workspace_size()");
+    NKV_REQUIRE(!xb || (steps && rounds), NKV_ERR_UNSUPPORTED,
                 "a bf16 fit needs HD % 32 == 0, 16-byte aligned rows and at least one round");
     NKV_REQUIRE(rounds || !(a->centers_bf16 || a->ids_u8), NKV_ERR_UNSUPPORTED,
                 "bf16 centers and uint8 ids need at least one round");
     unsigned char* ws = reinterpret_cast<unsigned char*>(a->workspace);
     double* part_d = reinterpret_cast<double*>(ws);
-    int32_t* part_c = reinterpret_cast<int32_t*>(ws + fit_part_bytes(B, S, C, sizeof(double)));
+    int32_t* part_c = reinterpret_cast<int32_t*>(ws + (mfma ? fit_part_bytes(B, S, C, sizeof(double)) : 0));
     FitInit init{};
     init.dev = a->init_rows;
     if (!init.dev) std::copy(a->init_rows_host, a->init_rows_host + C, init.v);

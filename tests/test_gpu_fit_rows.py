@@ -7,7 +7,7 @@ import pytest
 import torch
 
 import oracle.oracle as orc
-from nanokv_amd import ops
+from nanokv_amd import _lib, ops
 from tests._helpers import u16
 
 pytestmark = pytest.mark.gpu
@@ -29,6 +29,29 @@ def test_fit_rows_match_oracle(dev, B, S, HD, C, iters):
             assert np.array_equal(labels.cpu().numpy().astype(np.int64), rl)
             assert np.array_equal(ids.cpu().numpy().astype(np.int64), rl)
             assert np.array_equal(u16(centers), orc.f32_to_bf16(rc))
+
+
+@pytest.mark.parametrize("B,S,HD,C", [(1, 40, 64, 33), (2, 130, 96, 64), (1, 300, 3072, 256)])
+def test_fit_in_a_label_sized_workspace(dev, B, S, HD, C):
+    """A workspace for the rows' labels alone serves fp32 rows; one byte less
+    is refused."""
+    g = torch.Generator().manual_seed(S)
+    x = torch.randn(B, S, HD, generator=g)
+    init = torch.randperm(S, generator=g)[:C].to(torch.int32)
+    rc, rl = orc.c64_fit(x.numpy(), init.numpy(), 2)
+    xd, rows = x.to(dev), init.to(dev)
+    centers = torch.empty(B, C, HD, device=dev)
+    labels = torch.empty(B, S, device=dev, dtype=torch.int32)
+    need = -(-4 * B * S // 256) * 256
+    assert need < _lib.lib().nkv_c64_fit_workspace_size(B, S, C)
+    buf = torch.full((need + 4096,), 0x5a, device=dev, dtype=torch.uint8)
+    for nbytes, want in ((need, _lib.NKV_OK), (need - 1, _lib.NKV_ERR_WORKSPACE)):
+        assert _lib.lib().nkv_c64_fit(torch.cuda.current_stream().cuda_stream, xd.data_ptr(), B, S, HD,
+                                      C, 2, rows.data_ptr(), centers.data_ptr(), labels.data_ptr(),
+                                      buf.data_ptr(), nbytes) == want
+    assert (buf[need:] == 0x5a).all()
+    assert np.array_equal(labels.cpu().numpy().astype(np.int64), rl)
+    assert np.array_equal(centers.cpu().numpy(), rc)
 
 
 @pytest.mark.parametrize("rows,r,G", [(1, 8, 8), (5, 24, 24), (33, 64, 16), (7, 120, 40),
