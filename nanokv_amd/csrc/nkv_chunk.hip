@@ -2151,17 +2151,6 @@ void launch_dk(const ChunkParams& p, int64_t blocks, hipStream_t s, int* rc) {
     }
 }
 
-template <typename K>
-int set_smem(K* kernel, size_t smem) {
-    const hipError_t e = hipFuncSetAttribute((const void*)kernel,
-                                             hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem);
-    if (e != hipSuccess) {
-        set_error(std::string("chunk_launch: hipFuncSetAttribute failed: ") + hipGetErrorString(e));
-        return NKV_ERR_HIP;
-    }
-    return NKV_OK;
-}
-
 // ---------------------------------------------------------- staged (host)
 constexpr int FT_CUS = 256;          // compute units of an MI355X
 // The staged schedule from one query block up.  Measured on MI355X against

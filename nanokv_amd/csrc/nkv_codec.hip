@@ -1629,19 +1629,6 @@ __global__ void __launch_bounds__(64 * EP_WAVES) encode_proj_kernel(EncBatch B) 
     }
 }
 
-// Dynamic LDS of the projection kernels (above 64 KB), set once per process.
-static int encode_proj_smem() {
-    static const int rc = [] {
-        const hipError_t e0 = hipFuncSetAttribute((const void*)encode_proj_kernel<true>,
-                                                  hipFuncAttributeMaxDynamicSharedMemorySize,
-                                                  EncProjFmt<true>::SMEM);
-        const hipError_t e1 = hipFuncSetAttribute((const void*)encode_proj_kernel<false>,
-                                                  hipFuncAttributeMaxDynamicSharedMemorySize,
-                                                  EncProjFmt<false>::SMEM);
-        return e0 == hipSuccess && e1 == hipSuccess ? (int)NKV_OK : (int)NKV_ERR_HIP;
-    }();
-    return rc;
-}
 static_assert(EncProjFmt<false>::SMEM <= 160 * 1024, "LDS budget");
 
 struct DecodeEpi {
@@ -2390,19 +2377,11 @@ static int launch_assign_batch(hipStream_t s, EncBatch B, bool xb) {
     const dim3 grid((unsigned)cdiv(rows, AB_ROWS), (unsigned)B.n);
     const unsigned threads = 64 * AB_WAVES;
     if (xb) {
-        static const hipError_t attr = [] {
-            hipError_t e = hipSuccess;
-            for (const void* f : {(const void*)assign_dma_kernel<1>, (const void*)assign_dma_kernel<2>,
-                                  (const void*)assign_dma_kernel<4>})
-                if (e == hipSuccess)
-                    e = hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, AD_SMEM);
-            return e;
-        }();
-        NKV_REQUIRE(attr == hipSuccess, NKV_ERR_HIP, "hipFuncSetAttribute failed for the search kernels");
-        const unsigned g1 = xcd_grid(B.n * B.row_blocks);
-        if (B.id_bytes == 1) assign_dma_kernel<1><<<g1, threads, AD_SMEM, s>>>(B);
-        else if (B.id_bytes == 2) assign_dma_kernel<2><<<g1, threads, AD_SMEM, s>>>(B);
-        else assign_dma_kernel<4><<<g1, threads, AD_SMEM, s>>>(B);
+        const auto kernel = B.id_bytes == 1 ? assign_dma_kernel<1>
+                            : B.id_bytes == 2 ? assign_dma_kernel<2> : assign_dma_kernel<4>;
+        const int rc = set_smem(kernel, AD_SMEM);
+        if (rc) return rc;
+        kernel<<<xcd_grid(B.n * B.row_blocks), threads, AD_SMEM, s>>>(B);
     } else {
         if (B.id_bytes == 1) assign_bf16_kernel<1, false><<<grid, threads, 0, s>>>(B);
         else if (B.id_bytes == 2) assign_bf16_kernel<2, false><<<grid, threads, 0, s>>>(B);
@@ -2689,18 +2668,6 @@ EncPlan enc_plan(const nkv_encode_args* a, int n) {
 
 int encode_staged(hipStream_t s, const EncBatch& B, bool xb, bool search, const nkv_encode_args* a,
                   const EncPlan& pl) {
-    static const hipError_t attr = [] {
-        const std::pair<const void*, int> k[] = {{(const void*)search_dots_kernel, DotsTile::SMEM},
-                                                 {(const void*)project_kernel<Proj64>, Proj64::SMEM},
-                                                 {(const void*)project_kernel<Proj96>, Proj96::SMEM},
-                                                 {(const void*)project_kernel<Proj128>, Proj128::SMEM}};
-        hipError_t e = hipSuccess;
-        for (const auto& f : k)
-            if (e == hipSuccess)
-                e = hipFuncSetAttribute(f.first, hipFuncAttributeMaxDynamicSharedMemorySize, f.second);
-        return e;
-    }();
-    NKV_REQUIRE(attr == hipSuccess, NKV_ERR_HIP, "hipFuncSetAttribute failed for the encode kernels");
     EncWsBatch W{};
     W.e = B;
     W.splits = pl.splits;
@@ -2733,6 +2700,8 @@ int encode_staged(hipStream_t s, const EncBatch& B, bool xb, bool search, const 
                 NKV_LAUNCH_CHECK();
             }
             const unsigned tiles = (unsigned)(cdiv(W.rows, DotsTile::TM) * cdiv(B.num_centers, DotsTile::TN));
+            const int rc = set_smem(search_dots_kernel, DotsTile::SMEM);
+            if (rc) return rc;
             search_dots_kernel<<<dim3(tiles, pl.splits, n), DotsTile::THREADS, DotsTile::SMEM, s>>>(W);
             NKV_LAUNCH_CHECK();
         }
@@ -2748,15 +2717,19 @@ int encode_staged(hipStream_t s, const EncBatch& B, bool xb, bool search, const 
             xb ? decide(decide_kernel<4, true, true>) : decide(decide_kernel<4, false, true>);
         }
         NKV_LAUNCH_CHECK();
-        auto project = [&](auto tile, auto kernel) {
+        auto project = [&](auto tile, auto kernel) -> int {
             using T = decltype(tile);
             W.e.qgroup = T::TN % a->group == 0 ? a->group : 0;
+            const int rc = set_smem(kernel, T::SMEM);
+            if (rc) return rc;
             kernel<<<xcd_grid(n * cdiv(W.rows, T::TM) * cdiv(B.r, T::TN)), T::THREADS, T::SMEM, s>>>(W);
+            NKV_LAUNCH_CHECK();
+            return NKV_OK;
         };
-        if (pl.cols == 64) project(Proj64{}, project_kernel<Proj64>);
-        else if (pl.cols == 96) project(Proj96{}, project_kernel<Proj96>);
-        else project(Proj128{}, project_kernel<Proj128>);
-        NKV_LAUNCH_CHECK();
+        const int rc = pl.cols == 64   ? project(Proj64{}, project_kernel<Proj64>)
+                       : pl.cols == 96 ? project(Proj96{}, project_kernel<Proj96>)
+                                       : project(Proj128{}, project_kernel<Proj128>);
+        if (rc) return rc;
     }
     if (W.e.qgroup) return NKV_OK;
     const dim3 qgrid((unsigned)cdiv(rows * (B.r / a->group) * quant_lanes(a->group), 256), (unsigned)n);
@@ -2840,16 +2813,17 @@ int encode_batch(hipStream_t s, const nkv_encode_args* a, int n) {
         if (rc) return rc;
     }
     if (fast_proj && aligned) {
-        NKV_REQUIRE(encode_proj_smem() == NKV_OK, NKV_ERR_HIP,
-                    "hipFuncSetAttribute failed for the projection kernels");
         B.row_blocks = cdiv(rows, EP_ROWS);
         // groups that do not straddle column blocks are quantised in the same launch
         B.qgroup = EP_COLS % a->group == 0 ? a->group : 0;
         B.scale_dtype = a->scale_dtype;
         B.quant_mode = a->quant_mode;
         const unsigned grid = xcd_grid(n * cdiv(r, EP_COLS) * B.row_blocks);
-        if (xb) encode_proj_kernel<true><<<grid, 64 * EP_WAVES, EncProjFmt<true>::SMEM, s>>>(B);
-        else encode_proj_kernel<false><<<grid, 64 * EP_WAVES, EncProjFmt<false>::SMEM, s>>>(B);
+        const auto kernel = xb ? encode_proj_kernel<true> : encode_proj_kernel<false>;
+        const int smem = xb ? EncProjFmt<true>::SMEM : EncProjFmt<false>::SMEM;
+        rc = set_smem(kernel, smem);
+        if (rc) return rc;
+        kernel<<<grid, 64 * EP_WAVES, smem, s>>>(B);
         NKV_LAUNCH_CHECK();
         if (B.qgroup) return NKV_OK;
     } else {
@@ -2949,9 +2923,8 @@ bool dec_aligned(const DecProb& p, const uint16_t* w) {
 template <int MI, int WR, int WC>
 int launch_decode_tiles(hipStream_t s, DecBatch& B, int64_t rows) {
     using F = DecFmt<MI, WR, WC>;
-    static const hipError_t attr = hipFuncSetAttribute(
-        (const void*)decode_tile_kernel<MI, WR, WC>, hipFuncAttributeMaxDynamicSharedMemorySize, F::SMEM);
-    NKV_REQUIRE(attr == hipSuccess, NKV_ERR_HIP, "hipFuncSetAttribute failed for the decode kernels");
+    const int rc = set_smem(decode_tile_kernel<MI, WR, WC>, F::SMEM);
+    if (rc) return rc;
     const int64_t items = B.n * cdiv(rows, F::ROWS) * cdiv(B.HD, F::COLS);
     NKV_REQUIRE(items < INT32_MAX - 8, NKV_ERR_UNSUPPORTED, "decode grid too large");
     B.row_blocks = (uint32_t)cdiv(rows, F::ROWS);

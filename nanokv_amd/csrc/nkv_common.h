@@ -50,6 +50,16 @@ void clear_error();
 // synchronising the stream.
 #define NKV_LAUNCH_CHECK() NKV_HIP_CHECK(hipGetLastError())
 
+// The dynamic LDS of a kernel that takes more than 64 KB, set before each
+// launch: the attribute belongs to the current device, and a process may use
+// several.
+template <typename K>
+int set_smem(K* kernel, size_t smem) {
+    NKV_HIP_CHECK(hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                      (int)smem));
+    return NKV_OK;
+}
+
 // ---------------------------------------------------------------- numbers
 __device__ __forceinline__ float bf16_bits_to_f32(uint16_t b) {
     return __uint_as_float(((uint32_t)b) << 16);
