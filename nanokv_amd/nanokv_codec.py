@@ -243,8 +243,10 @@ def preload_operator_weights(device: torch.device, path: Optional[str] = None) -
                           decoder=move(entry["decoder"]), mean=entry["mean"].float().to(device))
 
 
-def _indexed(device: torch.device) -> torch.device:
-    """device with its index: that of the current device for a bare "cuda"."""
+def _indexed(device) -> torch.device:
+    """device (or its name) with its index: that of the current device for a
+    bare "cuda"."""
+    device = torch.device(device)
     if device.type == "cuda" and device.index is None:
         return torch.device("cuda", torch.cuda.current_device())
     return device
@@ -442,7 +444,7 @@ def codec_view(part: dict, device: torch.device) -> ops.Codec:
     """Device tensors of one encoded segment as an ops.Codec."""
     if part.get("codec") != CODEC:
         raise RuntimeError(f"unsupported WorldPlay payload {part.get('codec')}")
-    batch, seq, _ = part["shape"]
+    batch, seq = int(part["shape"][0]), int(part["shape"][1])
     r = int(part["latent_shape"][-1])
     device = _indexed(device)
     op = _operator(str(part["kind"]), int(part["layer"]), device)
@@ -495,7 +497,7 @@ def decode_value(value: Any, *, dtype: torch.dtype, device: torch.device) -> tor
     if value.get("codec") == SEGMENTS:
         segments = value["segments"]
         if len(segments) > 1 and all(is_payload(p) and p["codec"] == CODEC for p in segments):
-            dev = _indexed(torch.device(device))
+            dev = _indexed(device)
             views = [codec_view(p, dev) for p in segments]
             first = views[0]
             if all(v.batch == 1 and v.w_dec is first.w_dec and v.mean is first.mean

@@ -145,3 +145,22 @@ def test_history_codecs_cache_releases_dropped_payloads():
     nc.history_codecs(k2, v2, torch.device("cpu"))
     assert len(nc._HISTORY_TABLES) == 1
     del storage
+
+
+@pytest.fixture
+def operators():
+    for kind in ("k", "v"):
+        nc.register_operator(kind, 0, encoder=torch.zeros(64, 128, dtype=torch.bfloat16),
+                             decoder=torch.zeros(128, 64, dtype=torch.bfloat16))
+    yield
+    for kind in ("k", "v"):
+        nc._OPERATORS.pop((kind, 0), None)
+
+
+@pytest.mark.parametrize("device", ["cpu", torch.device("cpu")])
+def test_codec_view_takes_device_names_and_whole_number_shapes(operators, device):
+    """Shapes as a file may hold them, and devices by name."""
+    p = _fake_payload("k", 10)
+    for shape in ((1, 10, 128), [1.0, 10.0, 128.0], np.array([1, 10, 128]), torch.tensor([1, 10, 128])):
+        view = nc.codec_view(dict(p, shape=shape), device)
+        assert tuple(view.packed.shape) == (1, 10, 32) and tuple(view.ids.shape) == (1, 10)
