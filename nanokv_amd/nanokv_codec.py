@@ -499,12 +499,12 @@ def decode_value(value: Any, *, dtype: torch.dtype, device: torch.device) -> tor
         if len(segments) > 1 and all(is_payload(p) and p["codec"] == CODEC for p in segments):
             dev = _indexed(device)
             views = [codec_view(p, dev) for p in segments]
-            first = views[0]
+            first, width = views[0], int(segments[0]["shape"][2])
             if all(v.batch == 1 and v.w_dec is first.w_dec and v.mean is first.mean
                    and (v.group, v.scales.dtype) == (first.group, first.scales.dtype)
-                   for v in views):
+                   and int(p["shape"][2]) == width for v, p in zip(views, segments)):
                 # one operator: every segment straight into its rows of the result
-                return ops.decode_batch(views, int(segments[0]["shape"][2])).to(dtype)
+                return ops.decode_batch(views, width).to(dtype)
         parts = [decode_value(item, dtype=dtype, device=device) for item in segments]
         return torch.cat(parts, dim=1) if parts else None
     return decode_tensor(value, dtype=dtype, device=device)

@@ -164,3 +164,24 @@ def test_codec_view_takes_device_names_and_whole_number_shapes(operators, device
     for shape in ((1, 10, 128), [1.0, 10.0, 128.0], np.array([1, 10, 128]), torch.tensor([1, 10, 128])):
         view = nc.codec_view(dict(p, shape=shape), device)
         assert tuple(view.packed.shape) == (1, 10, 32) and tuple(view.ids.shape) == (1, 10)
+
+
+def test_decode_value_checks_every_segment_width(operators, monkeypatch):
+    """Segments go to one decode only where all state one width; a segment
+    that states another is decoded by itself, which refuses it."""
+    batched = []
+    monkeypatch.setattr(nc.ops, "decode_batch",
+                        lambda views, hd: batched.append(hd) or torch.zeros(1, 17, hd))
+
+    def decode(view, hd, row_index=None):
+        view.validate(hd)
+        return torch.zeros(1, view.tokens, hd)
+
+    monkeypatch.setattr(nc.ops, "decode", decode)
+    good, bad = _fake_payload("k", 10), dict(_fake_payload("k", 7), shape=(1, 7, 256))
+    seg = nc.concat_values(good, _fake_payload("k", 7))
+    assert nc.decode_value(seg, dtype=torch.float32, device="cpu").shape == (1, 17, 128)
+    assert batched == [128]
+    with pytest.raises(ValueError):
+        nc.decode_value(nc.concat_values(good, bad), dtype=torch.float32, device="cpu")
+    assert batched == [128]
