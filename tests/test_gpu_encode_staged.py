@@ -12,15 +12,29 @@ from nanokv_amd import _lib, ops
 pytestmark = pytest.mark.gpu
 
 
-def _plain(problems, **kw):
-    """encode_batch of problems without a workspace."""
+def _call(problems, scratch, **kw):
+    """encode_batch of problems without a workspace, or (scratch) in one that
+    the call has to use."""
     built = [ops._encode_args(p["x"], p["w_enc"], p.get("centers"), p.get("mean"), kw["group"],
                               kw["scale_dtype"], kw["quant_mode"], p.get("id_dtype"), None,
                               p.get("ids")) for p in problems]
     arr = (_lib.NkvEncodeArgs * len(built))(*(b[0] for b in built))
+    buf = None
+    if scratch:
+        need = _lib.lib().nkv_encode_workspace_size(arr, len(built))
+        assert need > 0
+        buf = torch.full((need + 4096,), 0x5a, device=problems[0]["x"].device, dtype=torch.uint8)
+        arr[0].workspace, arr[0].workspace_bytes = buf.data_ptr(), need
     _lib.check("nkv_encode_batch", _lib.lib().nkv_encode_batch(
         torch.cuda.current_stream().cuda_stream, arr, len(built)))
+    if scratch:
+        # the residual of the first row, at the front of it, was written, and nothing past it
+        assert (buf[:problems[0]["x"].shape[1]] != 0x5a).any() and (buf[need:] == 0x5a).all()
     return [b[1] for b in built]
+
+
+def _plain(problems, **kw):
+    return _call(problems, False, **kw)
 
 
 # rows around the 64- and 128-row tiles and past one pass of 4,096; widths of one
@@ -61,8 +75,9 @@ def test_staged_encode_is_the_plain_one(dev, n, rows, HD, r, G, C, dtype, ids, m
         problems.append(p)
     for mode in ("fp32", "bf16"):
         kw = dict(group=G, scale_dtype=torch.float16, quant_mode=mode)
-        got, ref = ops.encode_batch(problems, **kw), _plain(problems, **kw)
-        for a, b in zip(got, ref):
+        ref = _plain(problems, **kw)
+        got = ops.encode_batch(problems, **kw) + _call(problems, True, **kw)
+        for a, b in zip(got, ref + ref):
             for name in ("ids", "coeff", "packed", "scales"):
                 if b[name] is None:
                     continue
