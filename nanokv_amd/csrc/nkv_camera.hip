@@ -7,6 +7,8 @@
 
 #include "nkv_internal.h"
 
+#include <type_traits>
+
 namespace nkv {
 
 int camera_from_abi(const nkv_camera* c, int D, int B, CameraDev* dev) {
@@ -79,15 +81,20 @@ __global__ void __launch_bounds__(256) camera_apply_kernel(CameraApplyParams p) 
 }
 
 // 16-byte pieces: one thread transforms piece `part` (8 dims, two 4-vectors)
-// of one (b, s) in CA_HEADS heads: the frame's matrices are fetched and rounded
+// of one (b, s) in HEADS heads: the frame's matrices are fetched and rounded
 // once for them, their loads are in flight together.
 // INTER: the vectors are the even and the odd dims, one sub-frame (FULL at
 // D = 128); else dims 0..3 and 4..7, each with its own sub-frame or (< 0) left
-// alone (FULL at D = 64, SF13).  1,560 x 24 x 128 (19 MB moved): 7.7 us; one
-// 4-vector per thread, four 2-byte accesses each way, 14 us.
-constexpr int CA_HEADS = 8;
+// alone (FULL at D = 64, SF13).  Per call in a graph with 1, 2, 4, 8 and 16
+// heads, FULL, us: 37 x 8 x 128 2.57, 2.82, 3.31, 4.34, 7.2 (a thread's chain over
+// its heads); 780 x 24 4.48, 4.27, 4.34, 4.96, 13.1; 1,560 x 24 (19 MB moved)
+// 6.74, 5.85, 5.72, 6.50, 15.5; 3,120 x 24 10.6, 9.3, 8.6, 9.4; 12,480 x 24 31.0,
+// 30.6, 29.7, 30.6 (SF13 38.6, 32.2, 28.1, 26.1); one 4-vector per thread, four
+// 2-byte accesses each way: 2.82, 7.60, 12.2, 21.0, 72.  Two up to PIECES_FEW
+// pieces, eight above.
+constexpr int64_t PIECES_FEW = 512 << 10;
 
-template <bool INTER>
+template <bool INTER, int CA_HEADS>
 __global__ void __launch_bounds__(256) camera_pieces_kernel(CameraApplyParams p, uint32_t items) {
     const uint32_t per_row = (uint32_t)p.D / 8, S = (uint32_t)p.S;
     const uint32_t i = blockIdx.x * 256 + threadIdx.x;
@@ -155,13 +162,18 @@ int camera_launch(hipStream_t s, const CameraApplyParams& p) {
     const int D = p.D, layout = p.cam.layout;
     const int64_t pieces = (int64_t)p.B * p.S * (D / 8);
     const bool fits = layout == NKV_CAMERA_SF13 || D == 64 || D == 128;
-    if (D % 8 == 0 && fits && pieces <= INT32_MAX && cdiv(p.H, CA_HEADS) <= 65535 &&
+    if (D % 8 == 0 && fits && pieces <= INT32_MAX && cdiv(p.H, 8) <= 65535 &&
         rows16(p.x, p.x_sb, p.x_st, p.x_sh) && rows16(p.out, p.o_sb, p.o_st, p.o_sh)) {
-        const dim3 grid((unsigned)cdiv(pieces, 256), (unsigned)cdiv(p.H, CA_HEADS));
-        if (layout == NKV_CAMERA_FULL && D == 128)
-            camera_pieces_kernel<true><<<grid, 256, 0, s>>>(p, (uint32_t)pieces);
-        else
-            camera_pieces_kernel<false><<<grid, 256, 0, s>>>(p, (uint32_t)pieces);
+        auto run = [&](auto inter, auto heads) {
+            const dim3 grid((unsigned)cdiv(pieces, 256), (unsigned)cdiv(p.H, heads()));
+            camera_pieces_kernel<inter(), heads()><<<grid, 256, 0, s>>>(p, (uint32_t)pieces);
+        };
+        auto split = [&](auto heads) {
+            if (layout == NKV_CAMERA_FULL && D == 128) run(std::true_type{}, heads);
+            else run(std::false_type{}, heads);
+        };
+        if (pieces * p.H <= PIECES_FEW && cdiv(p.H, 2) <= 65535) split(std::integral_constant<int, 2>{});
+        else split(std::integral_constant<int, 8>{});
     } else {
         const int64_t items = (int64_t)p.B * p.S * p.H * camera_vectors(layout, D);
         const unsigned grid = (unsigned)std::min<int64_t>(cdiv(items, 256), 65536);

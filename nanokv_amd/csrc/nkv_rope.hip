@@ -60,12 +60,18 @@ struct RopeApplyParams {
 };
 
 // 16-byte pieces (D % 8 == 0): one thread rotates the four pairs of piece
-// `part` of one (b, s) in RA_HEADS heads, so that the position's index arithmetic
+// `part` of one (b, s) in HEADS heads, so that the position's index arithmetic
 // and its four (cos, sin) entries are fetched once for them and their loads are
-// in flight together.  1,560 x 24 x 128 (19 MB moved): 7.0 us; one head per
-// thread, 11 us (four 64-bit divisions and 64 bytes of table per 16 of x).
-constexpr int RA_HEADS = 8;
+// in flight together (one head per thread took four 64-bit divisions and 64
+// bytes of table per 16 of x).  Per call in a graph with 1, 2, 4, 8 and 16 heads,
+// a table per row, us: 37 x 8 x 128 2.25, 2.35, 2.61, 3.14, 5.6 (a thread's chain
+// over its heads); 780 x 24 4.05, 3.59, 3.60, 3.80, 10.3; 1,560 x 24 (19 MB
+// moved) 6.05, 4.99, 4.99, 5.29, 13.8; 2,340 x 24 10.0, 8.25, 7.55, 6.58; 12,480
+// x 24 47.9, 42.0, 34.0, 28.9 (the table's traffic).  Two up to PIECES_FEW
+// pieces, eight above.
+constexpr int64_t PIECES_FEW = 512 << 10;
 
+template <int RA_HEADS>
 __global__ void __launch_bounds__(256) rope_pieces_kernel(RopeApplyParams p, uint32_t items) {
     const uint32_t per_row = (uint32_t)p.D / 8, S = (uint32_t)p.S;
     const uint32_t i = blockIdx.x * 256 + threadIdx.x;
@@ -154,9 +160,14 @@ extern "C" int nkv_rope_apply(void* stream, const nkv_rope* rope, int B, int64_t
     p.o_sh = o_sh;
     hipStream_t s = reinterpret_cast<hipStream_t>(stream);
     const int64_t pieces = (int64_t)B * S * (D / 8);
-    if (vec && pieces <= INT32_MAX && (H + RA_HEADS - 1) / RA_HEADS <= 65535) {
-        const dim3 grid((unsigned)cdiv(pieces, 256), (unsigned)cdiv(H, RA_HEADS));
-        rope_pieces_kernel<<<grid, 256, 0, s>>>(p, (uint32_t)pieces);
+    if (vec && pieces <= INT32_MAX && cdiv(H, 8) <= 65535) {
+        auto grid = [&](int heads) {
+            return dim3((unsigned)cdiv(pieces, 256), (unsigned)cdiv(H, heads));
+        };
+        if (pieces * H <= PIECES_FEW && cdiv(H, 2) <= 65535)
+            rope_pieces_kernel<2><<<grid(2), 256, 0, s>>>(p, (uint32_t)pieces);
+        else
+            rope_pieces_kernel<8><<<grid(8), 256, 0, s>>>(p, (uint32_t)pieces);
     } else {
         const int64_t items = (int64_t)B * S * H * (D / 2);
         rope_apply_kernel<<<(unsigned)std::min<int64_t>(cdiv(items, 256), 65536), 256, 0, s>>>(p);

@@ -33,8 +33,10 @@ def _same(a, b):
     assert (u16(a.nan_to_num()) == u16(b.nan_to_num())).all()
 
 
-# one head, a full group of eight, ragged ones; pieces that end inside a block
-@pytest.mark.parametrize("B,S,H,D", [(1, 1, 1, 8), (2, 17, 8, 128), (1, 33, 9, 96), (1, 130, 24, 64)])
+# one head, a full group of two and eight heads, ragged ones; pieces that end
+# inside a block; past the few pieces that two heads a thread serve
+@pytest.mark.parametrize("B,S,H,D", [(1, 1, 1, 8), (2, 17, 8, 128), (1, 33, 9, 96), (1, 130, 24, 64),
+                                     (2, 2501, 9, 128), (1, 1366, 24, 128), (1, 1365, 24, 128)])
 def test_rope_pieces(dev, B, S, H, D):
     x = _x(dev, B, S, H, D, S + H)
     g = torch.Generator().manual_seed(S)
@@ -45,7 +47,7 @@ def test_rope_pieces(dev, B, S, H, D):
 
 
 @pytest.mark.parametrize("layout,D", [("full", 128), ("full", 64), ("sf13", 128), ("sf13", 40)])
-@pytest.mark.parametrize("B,S,H", [(1, 1, 1), (2, 37, 8), (1, 70, 17)])
+@pytest.mark.parametrize("B,S,H", [(1, 1, 1), (2, 37, 8), (1, 70, 17), (2, 4903, 17)])
 def test_camera_pieces(dev, layout, D, B, S, H):
     x = _x(dev, B, S, H, D, S + D)
     P = synth.camera_matrices(3, seed=S)[2].to(dev)
