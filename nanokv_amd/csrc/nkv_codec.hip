@@ -2633,6 +2633,25 @@ struct EncPlan {
 // 64 x 6 tiles of the projection at r = 384: more fill the chip no better.
 constexpr int64_t ENC_PASS = 4096;
 
+// Whether the GEMMs over the workspace beat the batched kernels without one
+// (HD % 256 == 0, to search at most 256 centers), which read every row once and
+// whose time is flat until their blocks of 32 rows x 192 columns fill the chip.
+// us without / with a workspace, in a graph:
+//   one pass, no search, r = 64, 780 rows: HD 512 12 / 11, 1,024 16 / 13, 3,072
+//   33 / 24; a call from the host costs 4 us more with one (the scratch, a launch
+//   more): 13 / 17 and 17 / 17 at 512 and 1,024.
+//   one pass, a search of 16 centers, r = 64, 1,560 rows: HD 256 bf16 22 / 20, fp32
+//   24 / 26 (300 rows 24 / 24); 512 bf16 28 / 25, fp32 29 / 28; two problems of 512
+//   and 64 centers 28 / 27, from the host 31.6 / 33.5.
+//   6,000 rows, two passes, 64 centers: HD 512 r = 384 43 / 57, 3,072 r = 64 79 / 93,
+//   r = 384 120 / 103 (two column blocks of the projection); fp32 rows, which
+//   a search splits in two planes, 135 / 142.
+bool enc_gemm_pays(const nkv_encode_args* a, int n, bool search, int64_t rows, int64_t pass) {
+    if (rows > pass) return a->HD >= 2048 && a->r > EP_COLS && (!search || a->x_bf16);
+    if (!search || n > 1) return a->HD >= 1024;
+    return a->x_bf16 || a->HD >= 512 || rows <= 512;
+}
+
 EncPlan enc_plan(const nkv_encode_args* a, int n) {
     EncPlan p{};
     const bool search = a->centers && !a->ids_in;
@@ -2644,7 +2663,11 @@ EncPlan enc_plan(const nkv_encode_args* a, int n) {
     if ((int64_t)std::max(a->r, search ? a->num_centers : 0) * a->HD * 2 > UINT32_MAX) return p;
     for (int i = 0; i < n; ++i)
         if (a[i].x_stride > (1 << 20)) return p;
-    p.pass = std::min(rows, std::max<int64_t>(ENC_PASS / n / DotsTile::TM, 1) * DotsTile::TM);
+    const int64_t pass = std::max<int64_t>(ENC_PASS / n / DotsTile::TM, 1) * DotsTile::TM;
+    if (a->HD % 256 == 0 && !(search && a->num_centers > AB_MAXC) &&
+        !enc_gemm_pays(a, n, search, rows, pass))
+        return p;
+    p.pass = std::min(rows, pass);
     auto up = [](size_t b) { return (b + 255) / 256 * 256; };
     p.resid = up((size_t)p.pass * a->HD * 2);
     // the narrowest tile whose blocks run in one round of the 256 CUs (one

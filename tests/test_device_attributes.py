@@ -92,7 +92,7 @@ def attend():
 
 # (call, whether some of its launches take more than 64 KB)
 calls = [(lambda: decode(8192, 3072), True), (lambda: decode(40, 256), False), (attend, True)]
-calls += [(lambda r=r, b=b, s=s: encode(rows, r, b, s), True) for rows, r in ((64, 64), (6000, 96), (6000, 384))
+calls += [(lambda r=r, b=b, s=s: encode(rows, r, b, s), True) for rows, r in ((64, 64), (3000, 384), (4096, 480))
           for b in (False, True) for s in (False, True)]
 for i, (call, large) in enumerate(calls):
     for dev in (0, 1, 0):

@@ -130,3 +130,28 @@ def test_plan_fits_a_smaller_workspace(parts):
     for limit in (full, full + 1, 1 << 40, 0):
         assert _check(parts, limit=limit)[2] == full
     assert _check(parts, limit=least - 1)[2] == least
+
+
+@pytest.mark.parametrize("n,rows,HD,r,C,bf16,used", [
+    # 256 centers and more, or widths that only the general kernels take: always
+    (1, 5000, 256, 64, 257, False, True), (2, 5000, 384, 64, 64, False, True), (2, 50, 384, 64, 0, False, True),
+    # one pass (4,096 rows of all problems)
+    (1, 4096, 1024, 64, 0, True, True), (1, 4096, 768, 384, 0, True, False), (2, 2048, 1024, 64, 64, True, True),
+    (2, 64, 768, 64, 64, True, False), (1, 4096, 256, 64, 64, True, True), (1, 4096, 512, 64, 64, False, True),
+    (1, 512, 256, 64, 64, False, True), (1, 513, 256, 64, 64, False, False),
+    # more: wide rows and more than one column block of the projection
+    (1, 4097, 2048, 224, 0, True, True), (1, 4097, 2048, 192, 0, True, False), (1, 4097, 1792, 384, 0, True, False),
+    (1, 4097, 3072, 384, 256, True, True), (1, 4097, 3072, 384, 256, False, False),
+    (2, 2049, 3072, 384, 0, False, True), (2, 2049, 3072, 96, 64, True, False)])
+def test_encode_workspace_is_asked_for_where_it_pays(n, rows, HD, r, C, bf16, used):
+    args = (_lib.NkvEncodeArgs * n)()
+    for a in args:
+        a.rows, a.HD, a.r, a.group, a.scale_dtype = rows, HD, r, 32, _lib.NKV_DTYPE_FP16
+        a.num_centers, a.id_bytes = C, 2
+        setattr(a, "x_bf16" if bf16 else "x", 256)     # only looked at
+        a.w_enc = a.coeff = a.packed = a.scales = 256
+        if C:
+            a.centers = a.ids = 256
+    lib = _lib.lib()
+    need = lib.nkv_encode_workspace_size(args, n)
+    assert lib.nkv_last_error() == b"" and (need > 0) == used
