@@ -2983,12 +2983,26 @@ int launch_decode(hipStream_t s, const nkv_decode_args* first, const DecProb* p,
     return NKV_OK;
 }
 
+// Few rows of a low rank: decode_gemm_kernel's one tile per block starts sooner
+// than the staged tiles' first slice.  us in a graph, that kernel / the staged
+// ones: no centers, 1 x 256 2.80 / 3.61 (r = 32), 3.70 / 4.24 (96), 5.85 / 5.97
+// (256), 7.64 / 7.55 (384); 300 x 3,072 4.17 / 4.28 (r = 64), 5.10 / 5.05 (128); 600 x
+// 3,072 at r = 64 4.73 / 4.60; 24 x 256 at r = 256 6.26 / 6.14.  With centers, which
+// it adds two bytes at a time: 2 x 3,072 3.39 / 4.06 (r = 32), 6.47 / 6.48 (256);
+// 4 x 3,072 at r = 64 4.27 / 4.18.
+bool plain_decode_pays(const nkv_decode_args* a) {
+    const nkv_codec& c = a->codec;
+    if (a->B != 1 || c.r > 256) return false;
+    if (c.centers) return a->rows <= 2;
+    return a->rows <= 16 || (c.r <= 96 && a->rows * a->HD <= (1 << 20));
+}
+
 int decode_one(hipStream_t s, const nkv_decode_args* a) {
     const nkv_codec& c = a->codec;
     if (a->rows == 0) return NKV_OK;
-    bool aligned = true;
-    for (int b = 0; b < a->B; ++b) aligned = aligned && dec_aligned(dec_problem(a, b), c.w_dec);
-    if (aligned) {
+    bool staged = !plain_decode_pays(a);
+    for (int b = 0; b < a->B; ++b) staged = staged && dec_aligned(dec_problem(a, b), c.w_dec);
+    if (staged) {
         DecProb p[DEC_MAXB];
         for (int b0 = 0; b0 < a->B; b0 += DEC_MAXB) {
             const int nb = std::min(a->B - b0, DEC_MAXB);

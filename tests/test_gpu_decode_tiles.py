@@ -1,6 +1,6 @@
 """The staged decode kernels (nkv_decode, nkv_decode_batch) against
-decode_gemm_kernel, which a misaligned decoder still takes: the same
-accumulation order, so the same bits."""
+decode_gemm_kernel, which a misaligned decoder and few rows of a low rank
+still take: the same accumulation order, so the same bits."""
 import pytest
 import torch
 
@@ -39,6 +39,7 @@ def _misaligned(c):
 # ones, whole and half rank slices, groups of one chunk, a slice, the row
 @pytest.mark.parametrize("N,HD,r,G,C,mean", [
     (1, 32, 32, 8, 3, True), (63, 160, 96, 24, 0, True), (65, 288, 64, 64, 5, False),
+    (3, 32, 32, 8, 3, True), (17, 32, 160, 40, 0, True), (67, 16384, 96, 24, 0, True),
     (129, 544, 224, 224, 0, False), (8321, 1056, 160, 32, 7, True), (2000, 4128, 384, 48, 9, True)])
 def test_decode_tiles_match_the_plain_kernel(dev, N, HD, r, G, C, mean):
     c = _codec(dev, N, HD, r, G, C, mean, seed=N + HD)
