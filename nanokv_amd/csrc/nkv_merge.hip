@@ -233,8 +233,11 @@ extern "C" int nkv_lift_lse_combine(void* stream, const nkv_lift_combine_args* a
     const int64_t heads = 2 * (int64_t)a->B * a->H;
     NKV_REQUIRE(heads <= 65535, NKV_ERR_UNSUPPORTED, "at most 65535 batch x head pairs");
     // MFMA for rows of unit stride in 16-byte pieces; any other stride one
-    // element at a time
-    if (a->n_sd == 1 && a->l_sd == 1 && rows16(a->native, a->n_sb, a->n_sh, a->n_sq) &&
+    // element at a time, as are up to four queries of low_dim 32, whose few
+    // products take less than staging the lift transposed (24 heads, us in a
+    // graph: 1 query 4.9, by MFMA 6.4; 4 queries 5.75, 6.4; 8 queries 7.2, 6.3;
+    // low_dim 64, 1 query 7.3, 7.0)
+    if ((a->low_dim > 32 || a->Q > 4) && a->n_sd == 1 && a->l_sd == 1 && rows16(a->native, a->n_sb, a->n_sh, a->n_sq) &&
         rows16(a->low, a->l_sb, a->l_sh, a->l_sq) && reinterpret_cast<uintptr_t>(a->out) % 16 == 0) {
         const dim3 grid((unsigned)cdiv(a->Q, 32 * LM_WAVES), (unsigned)heads);
         auto run = [&](auto kernel) { kernel<<<grid, 64 * LM_WAVES, 0, (hipStream_t)stream>>>(*a); };

@@ -88,7 +88,7 @@ def test_camera_pieces_at_the_limits(dev, layout, D):
 
 
 @pytest.mark.parametrize("low", [32, 64, 96])
-@pytest.mark.parametrize("B,H,Q", [(1, 1, 1), (1, 2, 127), (2, 3, 161)])
+@pytest.mark.parametrize("B,H,Q", [(1, 1, 1), (1, 2, 4), (1, 2, 5), (1, 2, 127), (2, 3, 161)])
 def test_lift_pieces(dev, low, B, H, Q):
     g = torch.Generator().manual_seed(low + Q)
     native = torch.randn(2 * B, H, Q, 128, generator=g).to(torch.bfloat16).to(dev)
