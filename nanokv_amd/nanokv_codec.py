@@ -444,9 +444,11 @@ def codec_view(part: dict, device: torch.device) -> ops.Codec:
     """Device tensors of one encoded segment as an ops.Codec."""
     if part.get("codec") != CODEC:
         raise RuntimeError(f"unsupported WorldPlay payload {part.get('codec')}")
-    batch, seq = int(part["shape"][0]), int(part["shape"][1])
+    shape = part["shape"]
+    batch, seq = int(shape[0]), int(shape[1])
     r = int(part["latent_shape"][-1])
-    device = _indexed(device)
+    if not isinstance(device, torch.device) or device.index is None:
+        device = _indexed(device)
     op = _operator(str(part["kind"]), int(part["layer"]), device)
     group = int(part.get("scale_group", r))
 
@@ -496,15 +498,17 @@ def decode_value(value: Any, *, dtype: torch.dtype, device: torch.device) -> tor
         return value.to(device=device, dtype=dtype)
     if value.get("codec") == SEGMENTS:
         segments = value["segments"]
-        if len(segments) > 1 and all(is_payload(p) and p["codec"] == CODEC for p in segments):
+        if len(segments) > 1 and all(isinstance(p, dict) and p.get("codec") == CODEC
+                                     for p in segments):
             dev = _indexed(device)
             views = [codec_view(p, dev) for p in segments]
-            first, width = views[0], int(segments[0]["shape"][2])
-            if all(v.batch == 1 and v.w_dec is first.w_dec and v.mean is first.mean
-                   and (v.group, v.scales.dtype) == (first.group, first.scales.dtype)
-                   and int(p["shape"][2]) == width for v, p in zip(views, segments)):
+            first, widths = views[0], {int(p["shape"][2]) for p in segments}
+            if len(widths) == 1 and all(
+                    v.batch == 1 and v.w_dec is first.w_dec and v.mean is first.mean
+                    and v.group == first.group and v.scales.dtype == first.scales.dtype
+                    for v in views):
                 # one operator: every segment straight into its rows of the result
-                return ops.decode_batch(views, width).to(dtype)
+                return ops.decode_batch(views, widths.pop()).to(dtype)
         parts = [decode_value(item, dtype=dtype, device=device) for item in segments]
         return torch.cat(parts, dim=1) if parts else None
     return decode_tensor(value, dtype=dtype, device=device)
