@@ -804,7 +804,7 @@ namespace {
 // kernels (D = 128, ranks multiples of 64, scale groups multiples of 32),
 // query tiles otherwise.  Measured on MI355X at every query count tried,
 // 1 .. 320 queries with 2 .. 24 heads and 700 .. 49,920 history keys, the
-// key-chunk decomposition (the staged schedule from 8 query blocks) was
+// key-chunk decomposition (the staged schedule from one query block) was
 // faster: e.g. 0.17 vs 0.24 ms for one query over 12,480 keys at 24 heads,
 // 0.60 vs 0.86 ms for 256 queries over 49,920 keys.  Read-time RoPE and the
 // other read-time features are built into the key-chunk kernels only.

@@ -1806,8 +1806,10 @@ constexpr int CB_LOADS = 16;  // payload rows a wave has in flight
 // two rows a wave, since every wave loads the (m, l) again.  Measured with 1,
 // 2 and 4 rows: 64 blocks of 9 splits 5.2, 6.4, 7.2 us; 224 of 7 (16 heads,
 // 417 queries) 6.4, 6.3, 7.3; 600 of 4 (24 heads, 780 queries) 15.9, 13.4,
-// 16.2; 1,176 of 3 14.5, 12.0, 12.8.  With the output camera every wave loads
-// its queries' matrices too: four rows (1,176 blocks 24.9, 18.8, 16.4 us).
+// 16.2; 1,176 of 3 14.5, 12.0, 12.8.  The key-chunk kernel's merge takes two rows:
+// 1,078 blocks of 20 chunks 49.1, 41.2, 41.3 us, 49 of 5 4.9, 4.8, 6.6.  With the
+// output camera every wave loads its queries' matrices too: four rows (1,176
+// blocks 24.9, 18.8, 16.4 us; 600 14.4, 11.4, 12.1; 224 9.0, 9.4, 12.0).
 constexpr int64_t CB_FEW = 128;
 
 // The running merge of one wave: M the largest chunk max so far, L the
@@ -1904,32 +1906,31 @@ __device__ __forceinline__ void combine_partials(CombineAcc<ROWS>& A, const uint
 
 // Normalise and store this wave's share of query qi of (b, h): out = (acc +
 // shift * Lx) / L in bf16 (shift: the row of 128 values added to the
-// tracked source's output, or null), then, with ocam, bf16(P . out) for P
-// of query row qi in the FULL layout (nkv_camera_apply's arithmetic); half
-// 0 also writes lse = ln(sum) when lse is given.  With ocam both lanes of a
-// query (lane and lane ^ 32, which hold the two halves of every 8-dim
-// block) must reach this call.
-template <int ROWS>
+// tracked source's output, or null), then, with CAM, bf16(P . out) for P
+// of query row qi in the FULL layout (nkv_camera_apply's arithmetic).  The
+// first o_cols columns are written (o_cols >= 8: waves whose share lies past
+// them end early, share 0 never does); share 0 also writes lse = ln(sum) when
+// lse is given.  With CAM both lanes of a query (lane and lane ^ 32, which
+// hold the two halves of every 8-dim block) must reach this call.
+template <bool CAM, int ROWS>
 __device__ __forceinline__ void combine_store(const CombineAcc<ROWS>& A, uint16_t* out, int64_t o_sb,
                                               int64_t o_st, int64_t o_sh, int o_cols, float* lse,
                                               int64_t Q, int H, int b, int h, int64_t qi, int share, int lane,
-                                              const float* shift, const CameraDev* ocam = nullptr) {
+                                              const float* shift, const CameraDev& ocam) {
     const int hf = lane >> 5;
     const float inv = A.L > 0.0f ? 1.0f / A.L : 0.0f;
     uint16_t* orow = out + b * o_sb + qi * o_st + h * o_sh + 4 * hf;
-    // with ocam: rows 2 hf and 2 hf + 1 of P's sub-frames of this share's
-    // 8-column blocks (block k: sub-frame k % 4) for query qi, rounded to
-    // bf16 once
-    constexpr int NSUB = 2 * ROWS < 4 ? 2 * ROWS : 4;
-    const int sub0 = (2 * ROWS * share) & 3;
-    float pm[NSUB][2][4];
-    if (ocam) {
-        const float* M = camera_mats(*ocam, b, qi);
+    // with CAM: rows 2 hf and 2 hf + 1 of P's four sub-frames (of the 8-column
+    // blocks k with k % 4 the sub-frame) for query qi, rounded to bf16 once
+    static_assert(!CAM || ROWS % 2 == 0, "a share holds whole rounds of the four sub-frames");
+    float pm[4][2][4];
+    if constexpr (CAM) {
+        const float* M = camera_mats(ocam, b, qi);
 #pragma unroll
-        for (int c = 0; c < NSUB; ++c)
+        for (int c = 0; c < 4; ++c)
 #pragma unroll
             for (int r = 0; r < 2; ++r) {
-                const f32x4 m = ldg(reinterpret_cast<const f32x4*>(M + 16 * (sub0 + c) + 4 * (2 * hf + r)));
+                const f32x4 m = ldg(reinterpret_cast<const f32x4*>(M + 16 * c + 4 * (2 * hf + r)));
 #pragma unroll
                 for (int e = 0; e < 4; ++e) pm[c][r][e] = bf16_round(m[e]);
             }
@@ -1951,7 +1952,7 @@ __device__ __forceinline__ void combine_store(const CombineAcc<ROWS>& A, uint16_
             for (int e = 0; e < 4; ++e) v[e] = fmaf(shift[d + 4 * hf + e], A.Lx, v[e]);
         }
         u32x2 pk = {pack_bf16x2(v[0] * inv, v[1] * inv), pack_bf16x2(v[2] * inv, v[3] * inv)};
-        if (ocam) {
+        if constexpr (CAM) {
             // block d / 8: this lane holds dims 4 hf .. 4 hf + 4, lane ^ 32 the
             // other four; its 4-vectors are the block's even and odd dims,
             // and this lane forms outputs 2 hf, 2 hf + 1 of each
@@ -1962,7 +1963,7 @@ __device__ __forceinline__ void combine_store(const CombineAcc<ROWS>& A, uint16_
                                  __uint_as_float(hi0 << 16), __uint_as_float(hi1 << 16)};
             const float x1[4] = {__uint_as_float(lo0 & 0xffff0000u), __uint_as_float(lo1 & 0xffff0000u),
                                  __uint_as_float(hi0 & 0xffff0000u), __uint_as_float(hi1 & 0xffff0000u)};
-            const int c = n % NSUB;
+            const int c = n & 3;
             float y[2][2];
 #pragma unroll
             for (int r = 0; r < 2; ++r)
@@ -2001,8 +2002,8 @@ __global__ void __launch_bounds__(64 * CB_WAVES) chunk_combine_kernel(ChunkParam
     combine_partials(A, p.part_o, p.part_ml, bh, p.nch_total, p.qblocks, qblk, share, lane, false);
     const int64_t qi = (int64_t)qblk * 32 + (lane & 31);
     if (qi >= p.Q) return;
-    combine_store(A, p.out, p.o_sb, p.o_st, p.o_sh, p.o_cols, p.lse, p.Q, p.H,
-                  (int)(bh / p.H), (int)(bh % p.H), qi, share, lane, nullptr);
+    combine_store<false>(A, p.out, p.o_sb, p.o_st, p.o_sh, p.o_cols, p.lse, p.Q, p.H, (int)(bh / p.H),
+                         (int)(bh % p.H), qi, share, lane, nullptr, CameraDev{});
 }
 
 // The staged schedule's merge over every partition (CN/core.py:33-42 for
@@ -2011,7 +2012,8 @@ __global__ void __launch_bounds__(64 * CB_WAVES) chunk_combine_kernel(ChunkParam
 // the first other partition that lists h among its heads, whose output is
 // shifted by shift[b*sh_sb + h*sh_sh + d] (null: none; the value-mean
 // correction) before the merge.
-template <int ROWS>
+// CAM: the outputs take the camera ocam.
+template <int ROWS, bool CAM>
 __global__ void __launch_bounds__(64 * CB_WAVES) staged_combine_kernel(MultiParams P,
                                                                        const float* shift,
                                                                        int64_t sh_sb, int64_t sh_sh,
@@ -2044,9 +2046,8 @@ __global__ void __launch_bounds__(64 * CB_WAVES) staged_combine_kernel(MultiPara
     }
     const int64_t qi = (int64_t)qblk * 32 + (lane & 31);
     if (qi >= n.Q) return;
-    combine_store(A, n.out, n.o_sb, n.o_st, n.o_sh, n.o_cols, n.lse, n.Q, n.H, b, h, qi, share, lane,
-                  lp && shift ? shift + (int64_t)b * sh_sb + (int64_t)h * sh_sh : nullptr,
-                  ocam.mats ? &ocam : nullptr);
+    combine_store<CAM>(A, n.out, n.o_sb, n.o_st, n.o_sh, n.o_cols, n.lse, n.Q, n.H, b, h, qi, share, lane,
+                       lp && shift ? shift + (int64_t)b * sh_sb + (int64_t)h * sh_sh : nullptr, ocam);
 }
 
 // ------------------------------------------------------------------ host
@@ -2728,15 +2729,15 @@ int staged_run(hipStream_t s, const ChunkLaunchDesc* d, const ChunkParams* ps, i
         if (d[0].ev_end) NKV_HIP_CHECK(hipEventRecord((hipEvent_t)d[0].ev_end, s));
     }
     const int64_t qb = (int64_t)d[0].B * d[0].H * M.part[0].qblocks;
-    auto combine = [&](auto rows) {
+    auto combine = [&](auto rows, auto cam) {
         constexpr int ROWS = decltype(rows)::value;
-        staged_combine_kernel<ROWS>
+        staged_combine_kernel<ROWS, decltype(cam)::value>
             <<<dim3((unsigned)cdiv(qb * (8 / ROWS), CB_WAVES)), 64 * CB_WAVES, 0, s>>>(
                 M, shift, sh_sb, sh_sh, ocam);
     };
-    if (ocam.mats) combine(std::integral_constant<int, 4>{});  // the matrices once per wave
-    else if (qb <= CB_FEW) combine(std::integral_constant<int, 1>{});
-    else combine(std::integral_constant<int, 2>{});
+    if (ocam.mats) combine(std::integral_constant<int, 4>{}, std::true_type{});
+    else if (qb <= CB_FEW) combine(std::integral_constant<int, 1>{}, std::false_type{});
+    else combine(std::integral_constant<int, 2>{}, std::false_type{});
     NKV_LAUNCH_CHECK();
     return NKV_OK;
 }

@@ -2131,8 +2131,9 @@ struct Row8 {
 // eight waves: one wave per 16 rows x 64 centers (the whole HD each, 98 waves
 // with work) took 132 us per round, this 22 us.  In a step lane l holds
 // row / center l % 16, k 8 (l / 16) .. +8: whole 128-byte lines per row, and
-// any order of k is valid for the products.  Bound by the fp64 matrix rate
-// (0.61 GFLOP per round of 64 centers, 32 flop per cycle and SIMD).
+// any order of k is valid for the products.  Bound by latency: each wave's chain
+// of loads and dependent products (0.61 GFLOP per round of 64 centers would be 8
+// us at the fp64 matrix rate, 32 flop per cycle and SIMD).
 // part_d / part_c [center blocks][B * S]: the best center of each block.
 // FIRST: the centers are the initial rows of x.  HD % 32 == 0, 16-byte rows.
 constexpr int FS_ROWS = 16, FS_CENT = 32, FS_WAVES = 8, FS_AHEAD = 2;
