@@ -326,7 +326,7 @@ typedef struct nkv_encode_args {
 } nkv_encode_args;
 
 /* Scratch bytes an encode of these n problems can use (bounded: at most a few
- * thousand rows at a time); 0 if it uses none. */
+ * thousand rows at a time); 0 if it uses none or gains nothing from it. */
 size_t nkv_encode_workspace_size(const nkv_encode_args* args, int n);
 
 int nkv_encode(void* stream, const nkv_encode_args* args);
