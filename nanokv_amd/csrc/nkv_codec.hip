@@ -2634,21 +2634,36 @@ struct EncPlan {
 // 64 x 6 tiles of the projection at r = 384: more fill the chip no better.
 constexpr int64_t ENC_PASS = 4096;
 
-// Whether the GEMMs over the workspace beat the batched kernels without one
-// (HD % 256 == 0, to search at most 256 centers), which read every row once and
-// whose time is flat until their blocks of 32 rows x 192 columns fill the chip.
-// us without / with a workspace, in a graph:
-//   one pass, no search, r = 64, 780 rows: HD 512 12 / 11, 1,024 16 / 13, 3,072
-//   33 / 24; a call from the host costs 4 us more with one (the scratch, a launch
-//   more): 13 / 17 and 17 / 17 at 512 and 1,024.
-//   one pass, a search of 16 centers, r = 64, 1,560 rows: HD 256 bf16 22 / 20, fp32
-//   24 / 26 (300 rows 24 / 24); 512 bf16 28 / 25, fp32 29 / 28; two problems of 512
-//   and 64 centers 28 / 27, from the host 31.6 / 33.5.
-//   6,000 rows, two passes, 64 centers: HD 512 r = 384 43 / 57, 3,072 r = 64 79 / 93,
-//   r = 384 120 / 103 (two column blocks of the projection); fp32 rows, which
-//   a search splits in two planes, 135 / 142.
+// Whether the GEMMs over the workspace beat the kernels without one.  us
+// without / with a workspace, in a graph, r = 64 unless stated.
+//
+// The batched kernels (HD % 256 == 0, to search at most 256 centers) read every
+// row once; their time is flat until blocks of 32 rows x 192 columns fill the chip:
+//   one pass, no search, 780 rows: HD 512 12 / 11, 1,024 16 / 13, 3,072 33 / 24; a
+//   call from the host costs 4 us more with one (the scratch, a launch more): 13 /
+//   17 and 17 / 17 at 512 and 1,024.
+//   one pass, a search of 16 centers, 1,560 rows: HD 256 bf16 22 / 20, fp32 24 / 26
+//   (300 rows 24 / 24); 512 bf16 28 / 25, fp32 29 / 28; two problems of 512 and 64
+//   centers 28 / 27, from the host 31.6 / 33.5.
+//   6,000 rows, two passes, 64 centers: HD 512 r = 384 43 / 57, 3,072 79 / 93, r = 384
+//   120 / 103 (two column blocks of the projection); fp32 rows, which a search
+//   splits in two planes, 135 / 142.
+//
+// The general kernels (other widths; more centers) search in fp64, 64 centers at
+// least, and project 64 x 64 tiles:
+//   no search: HD 128 9 / 9, 384 12 / 10 (1,560 rows); 12,480 rows 14 / 45 at 384, 35 /
+//   72 at 1,152 (r = 384 67 / 81); 6,000 rows of 3,200 77 / 60, r = 384 88 / 69.
+//   1,560 rows, centers x HD: 64 x 128 21 / 22, 64 x 384 37 / 30, 300 x 128 30 / 24.
+//   12,480 rows: 64 x 384 103 / 144, 300 x 128 83 / 115, 64 x 640 153 / 152, 1,024 x 128
+//   148 / 146, 300 x 384 178 / 152.
 bool enc_gemm_pays(const nkv_encode_args* a, int n, bool search, int64_t rows, int64_t pass) {
-    if (rows > pass) return a->HD >= 2048 && a->r > EP_COLS && (!search || a->x_bf16);
+    const bool one_pass = rows <= pass;
+    if (a->HD % 256 || (search && a->num_centers > AB_MAXC)) {
+        if (search)
+            return (int64_t)std::max(a->num_centers, 64) * a->HD >= (one_pass ? 24576 : 40960);
+        return one_pass ? a->HD >= 384 : a->HD >= 2048 && (a->r > EP_COLS || rows <= 2 * pass);
+    }
+    if (!one_pass) return a->HD >= 2048 && a->r > EP_COLS && (!search || a->x_bf16);
     if (!search || n > 1) return a->HD >= 1024;
     return a->x_bf16 || a->HD >= 512 || rows <= 512;
 }
@@ -2665,9 +2680,7 @@ EncPlan enc_plan(const nkv_encode_args* a, int n) {
     for (int i = 0; i < n; ++i)
         if (a[i].x_stride > (1 << 20)) return p;
     const int64_t pass = std::max<int64_t>(ENC_PASS / n / DotsTile::TM, 1) * DotsTile::TM;
-    if (a->HD % 256 == 0 && !(search && a->num_centers > AB_MAXC) &&
-        !enc_gemm_pays(a, n, search, rows, pass))
-        return p;
+    if (!enc_gemm_pays(a, n, search, rows, pass)) return p;
     p.pass = std::min(rows, pass);
     auto up = [](size_t b) { return (b + 255) / 256 * 256; };
     p.resid = up((size_t)p.pass * a->HD * 2);

@@ -133,13 +133,16 @@ def test_plan_fits_a_smaller_workspace(parts):
 
 
 @pytest.mark.parametrize("n,rows,HD,r,C,bf16,used", [
-    # 256 centers and more, or widths that only the general kernels take: always
-    (1, 5000, 256, 64, 257, False, True), (2, 5000, 384, 64, 64, False, True), (2, 50, 384, 64, 0, False, True),
-    # one pass (4,096 rows of all problems)
+    # against the general kernels (other widths, more centers): by centers x width
+    (1, 5000, 256, 64, 257, False, True), (2, 50, 384, 64, 1, False, True), (2, 50, 128, 64, 191, False, False),
+    (2, 50, 128, 64, 192, False, True), (2, 5000, 384, 64, 64, False, False), (1, 5000, 640, 64, 64, False, True),
+    (2, 50, 384, 64, 0, False, True), (2, 50, 128, 64, 0, False, False), (1, 5000, 1152, 384, 0, False, False),
+    (1, 8192, 3200, 64, 0, False, True), (1, 8193, 3200, 64, 0, False, False), (1, 8193, 3200, 224, 0, False, True),
+    # against the batched ones: one pass (4,096 rows of all problems)
     (1, 4096, 1024, 64, 0, True, True), (1, 4096, 768, 384, 0, True, False), (2, 2048, 1024, 64, 64, True, True),
     (2, 64, 768, 64, 64, True, False), (1, 4096, 256, 64, 64, True, True), (1, 4096, 512, 64, 64, False, True),
     (1, 512, 256, 64, 64, False, True), (1, 513, 256, 64, 64, False, False),
-    # more: wide rows and more than one column block of the projection
+    # more than a pass: wide rows and more than one column block of the projection
     (1, 4097, 2048, 224, 0, True, True), (1, 4097, 2048, 192, 0, True, False), (1, 4097, 1792, 384, 0, True, False),
     (1, 4097, 3072, 384, 256, True, True), (1, 4097, 3072, 384, 256, False, False),
     (2, 2049, 3072, 384, 0, False, True), (2, 2049, 3072, 96, 64, True, False)])
